@@ -5,13 +5,11 @@
 // YvDynamicMoELayer._compute_shared_expert_output model/moe/layer.py:812-865, the gate
 // projection model/moe/gate.py:1179 and the complexity predictor gate.py:1112-1117.
 //
-// Tiling. A work-group is 4 wavefronts. It owns one 64-row tile of one expert segment
-// (rows are expert-sorted slots; shared experts are extra segments of all N tokens) and
-// 4 * NCB * 16 output columns; each wavefront owns NCB 16-column blocks over the whole K
-// range and up to four 16-row MFMA blocks (only the row blocks that hold rows are
-// computed). The B operand (weights, [out][in] row-major as nn.Linear stores them) streams
-// from HBM with 16-byte loads per lane and is dequantized in registers to bf16; the A
-// operand (activations gathered through the permutation) comes through L1/L2.
+// Forms. Every expert GEMM runs over a table of tiles (up to 16, 64, 128 or 256 rows of one expert
+// segment: rows are expert-sorted slots, shared experts are extra segments of all N tokens) times
+// column groups: the weight-streaming form at decode, the mid-sized form for tens of rows per
+// expert, the LDS-tiled form at prefill (ffn_tile_rows draws the lines). The weights are
+// dequantized in registers to bf16; the activations are gathered through the permutation.
 //
 // Rounding points follow the reference's bf16 path, because the reference's own bf16
 // chain sits about 2e-2 (max-abs) from exact arithmetic at these shapes and a more exact
@@ -317,30 +315,20 @@ struct NMat {
     static constexpr int value = (EPI == EPI_SWIGLU) ? 2 : 1;
 };
 
-// ------------------------------------------------------------------ bf16 activations
-// RB: B-operand ring depth (weight loads run RB-1 k-steps ahead of the MFMAs); RA: A-operand
-// ring depth (RA divides RB).
-template <int WF, int EPI, int NCB, int MAXRB, int RB = 4, int RA = 2>
+// ------------------------------------------------------------------ bf16, dense fp32 output
+// out[r][n] (+ split z at z * split_stride) = A · Wᵀ for bf16 weights and row counts between the
+// streaming and the tiled forms: 64-row tiles, NCB 16-column blocks per wavefront. Weight loads
+// run RB - 1 k-steps ahead of the MFMAs, activation loads RA - 1 (RA divides RB).
+template <int NCB, int RB = 4, int RA = 2>
 __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
-    constexpr int NM = NMat<EPI>::value;
-    constexpr bool GROUPED = (WF == YVMOE_W_INT4 || WF == YVMOE_W_FP8);
     static_assert(RB % RA == 0, "A ring depth must divide the B ring depth");
-    constexpr int R = RB;
-    typedef BLoad<WF> BL;
+    constexpr int MAXRB = 4;
+    typedef BLoad<YVMOE_W_BF16> BL;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    int e = 0, row0, seg_end;
-    if (p.tile_seg != nullptr) {
-        const int tile = blockIdx.x;
-        if (tile >= *p.ntiles) return;
-        e = p.tile_seg[tile];
-        row0 = p.tile_row0[tile];
-        seg_end = p.seg_start[e + 1];
-    } else {
-        row0 = blockIdx.x * MAXRB * 16;
-        if (row0 >= p.nrows) return;
-        seg_end = p.nrows;
-    }
+    const int row0 = blockIdx.x * MAXRB * 16;
+    if (row0 >= p.nrows) return;
+    const int seg_end = p.nrows;
     const int col0 = (blockIdx.y * 4 + wave) * NCB * 16;
     if (col0 >= p.ncols) return;
     const int nrb = min(MAXRB, (seg_end - row0 + 15) / 16);
@@ -353,47 +341,26 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
     for (int rb = 0; rb < MAXRB; ++rb) {
         int r = row0 + rb * 16 + (lane & 15);
         if (r >= seg_end) r = row0;
-        arow[rb] = (const char*)p.A + ((long long)map_row(p, r) * p.lda + kbeg + kl) * 2;
+        arow[rb] = (const char*)p.A + ((long long)r * p.lda + kbeg + kl) * 2;
     }
-    const long long e_off = (long long)e * p.b_stride;
-    const long long s_off = (long long)e * p.s_stride;
-    const char* bptr[NM][NCB];
-    const void* sptr[2] = {p.S0, p.S1};
+    const char* bptr[NCB];
     int ncol[NCB];
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb) {
         ncol[cb] = col0 + cb * 16 + (lane & 15);
-        bptr[0][cb] = BL::bptr(p.B0, e_off, ncol[cb], p.K, kbeg, lane);
-        if constexpr (NM == 2) bptr[NM - 1][cb] = BL::bptr(p.B1, e_off, ncol[cb], p.K, kbeg, lane);
+        bptr[cb] = BL::bptr(p.B0, 0, ncol[cb], p.K, kbeg, lane);
     }
 
-    f32x4 acc[NM][NCB][MAXRB];
+    f32x4 acc[NCB][MAXRB];
 #pragma unroll
-    for (int m = 0; m < NM; ++m)
+    for (int cb = 0; cb < NCB; ++cb)
 #pragma unroll
-        for (int cb = 0; cb < NCB; ++cb)
-#pragma unroll
-            for (int rb = 0; rb < MAXRB; ++rb) acc[m][cb][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int rb = 0; rb < MAXRB; ++rb) acc[cb][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    typename BL::Raw braw[R][NM][NCB];
-    // per-k-step scales for group-scaled formats (ring), one scale per column otherwise
-    float sc[GROUPED ? R : 1][NM][NCB];
-    if constexpr (!GROUPED) {
+    Frag16 braw[RB][NCB];
+    auto load_b = [&](int ks, Frag16 (&dst)[NCB]) {
 #pragma unroll
-        for (int m = 0; m < NM; ++m)
-#pragma unroll
-            for (int cb = 0; cb < NCB; ++cb) sc[0][m][cb] = b_scale<WF>(sptr[m], s_off, ncol[cb], p.K, 0);
-    }
-    auto load_b = [&](int slot_ks, typename BL::Raw (&dst)[NM][NCB], float (&sdst)[NM][NCB]) {
-        const int k0 = slot_ks * 64;
-#pragma unroll
-        for (int m = 0; m < NM; ++m)
-#pragma unroll
-            for (int cb = 0; cb < NCB; ++cb) {
-                BL::load_blk(dst[m][cb], bptr[m][cb], slot_ks);
-                if constexpr (GROUPED)
-                    sdst[m][cb] = b_scale<WF>(sptr[m], s_off, ncol[cb], p.K, kbeg + k0);
-            }
+        for (int cb = 0; cb < NCB; ++cb) BL::load_blk(dst[cb], bptr[cb], ks);
     };
     // Loads are unconditional (k-step clamped to the last one, row blocks past nrb read the
     // tile's first row): with no branch around them the compiler can wait for exactly the
@@ -406,32 +373,25 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
             af[rb].u[1] = q[1];
         }
     };
-    auto mma = [&](const typename BL::Raw (&bw)[NM][NCB], const float (&bs)[NM][NCB],
-                   const Frag16 (&af)[MAXRB]) {
+    auto mma = [&](const Frag16 (&bf)[NCB], const Frag16 (&af)[MAXRB]) {
 #pragma unroll
-        for (int m = 0; m < NM; ++m) {
+        for (int cb = 0; cb < NCB; ++cb) {
 #pragma unroll
-            for (int cb = 0; cb < NCB; ++cb) {
-                Frag16 bf;
-                BL::cvt(bw[m][cb], bs[m][cb], bf);
-#pragma unroll
-                for (int rb = 0; rb < MAXRB; ++rb) {
-                    if (rb < nrb) {
-                        f32x4& dst = acc[m][cb][rb];
-                        dst = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[rb].v[0], bf.v[0], dst, 0, 0, 0);
-                        dst = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[rb].v[1], bf.v[1], dst, 0, 0, 0);
-                    }
+            for (int rb = 0; rb < MAXRB; ++rb) {
+                if (rb < nrb) {
+                    f32x4& dst = acc[cb][rb];
+                    dst = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[rb].v[0], bf[cb].v[0], dst, 0, 0, 0);
+                    dst = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[rb].v[1], bf[cb].v[1], dst, 0, 0, 0);
                 }
             }
         }
     };
     auto kc = [&](int ks) { return ks < nks ? ks : nks - 1; };
 
-    constexpr int SR = GROUPED ? R : 1;
     Frag16 abuf[RA][MAXRB];
     if (nks > 0) {
 #pragma unroll
-        for (int r = 0; r < RB - 1; ++r) load_b(kc(r), braw[r], sc[r % SR]);
+        for (int r = 0; r < RB - 1; ++r) load_b(kc(r), braw[r]);
 #pragma unroll
         for (int r = 0; r < RA - 1; ++r) load_a(kc(r), abuf[r]);
     }
@@ -440,9 +400,9 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
 #pragma unroll
         for (int r = 0; r < RB; ++r) {
             const int ks = ks0 + r;
-            load_b(kc(ks + RB - 1), braw[(r + RB - 1) % RB], sc[((r + RB - 1) % RB) % SR]);
+            load_b(kc(ks + RB - 1), braw[(r + RB - 1) % RB]);
             load_a(kc(ks + RA - 1), abuf[(r + RA - 1) % RA]);
-            mma(braw[r], sc[r % SR], abuf[r % RA]);
+            mma(braw[r], abuf[r % RA]);
         }
     }
     // tail (fewer than RB steps): their weights are already in ring slots 0..nks-ks0-1
@@ -450,11 +410,9 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
     for (int r = 0; r < RB - 1; ++r) {
         if (ks0 + r < nks) {
             load_a(kc(ks0 + r + RA - 1), abuf[(r + RA - 1) % RA]);
-            mma(braw[r], sc[r % SR], abuf[r % RA]);
+            mma(braw[r], abuf[r % RA]);
         }
     }
-
-    // epilogue (bf16 rounding points of YvSwiGLUExpert.forward)
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb) {
         const int n = ncol[cb];
@@ -464,20 +422,9 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int r = row0 + rb * 16 + (lane >> 4) * 4 + i;
-                    if (r < seg_end) {
-                        if constexpr (EPI == EPI_F32) {
-                            ((float*)p.out)[blockIdx.z * p.split_stride + (long long)r * p.ldo + n] =
-                                f32_out(p, acc[0][cb][rb][i], n, blockIdx.z);
-                        } else if constexpr (EPI == EPI_SWIGLU) {
-                            const float g = round_bf16(acc[0][cb][rb][i]);
-                            const float u = round_bf16(acc[NM - 1][cb][rb][i]);
-                            const float sg = round_bf16(silu(g));
-                            ((unsigned short*)p.out)[(long long)r * p.ldo + n] = f32_to_bf16_rne(sg * u);
-                        } else {
-                            ((unsigned short*)p.out)[(long long)r * p.ldo + n] =
-                                f32_to_bf16_rne(acc[0][cb][rb][i]);
-                        }
-                    }
+                    if (r < seg_end)
+                        ((float*)p.out)[blockIdx.z * p.split_stride + (long long)r * p.ldo + n] =
+                            f32_out(p, acc[cb][rb][i], n, blockIdx.z);
                 }
             }
         }
@@ -1716,6 +1663,243 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(GemmParams p, int ncb) {
     }
 }
 
+// ------------------------------------------------------------------ bf16, mid-sized form
+// Expert GEMM for batches whose experts hold about ten to a hundred rows: a tile is up to 128
+// (or 64) rows of one expert, a work-group of 4 wavefronts computes it against 64 h columns
+// (gate/up) or 128 output columns (down), each wavefront owning 32 weight rows (gate/up: the
+// gate and the up rows of the same 16 columns, so SwiGLU finishes in registers).
+//
+// What bounds it: HBM while the rows are few, then the conversion (2.3-2.5 VALU instructions per
+// weight) and the LDS reads of the activations beside the MFMAs. Every weight is read and
+// converted once per tile and needed by one wavefront only, so the weights go straight to
+// registers in their stored order (1 KB per load), kMidRing - 1 k-steps ahead of their use; the
+// activation rows, which all four wavefronts need, travel by direct-to-LDS loads through a
+// 3-stage ring two k-steps ahead (the swizzle of the 256-row tile). 48 KB of LDS and under 170
+// VGPRs put three work-groups on a CU, so one's conversion and LDS reads run beside another's
+// MFMAs and loads. A tile runs the copy of the loop for its row blocks rounded up to an even
+// count, so rows past its end are neither loaded nor multiplied. The scheduling barriers keep
+// the conversions of later steps from moving ahead of a work-group barrier, where they would
+// wait for their weights early (FFN at 64 experts of 47 rows: 288 us without, 271 us with).
+// A fifth wavefront that issued the activation loads (so the compiler's counts would cover the
+// weight loads alone) measured slower: two work-groups per CU instead of three (315 us).
+//
+// Measured (H 4096, 64 experts of 1408, 6 + 2 per token; FFN, against the form it replaced):
+// int8 200 tokens 345 -> 213 us, 500 516 -> 271 us, 700 486 -> 321 us (16-, 64- and 256-row
+// forms); bf16 341 tokens 859 -> 420 us; int4 341 tokens 462 -> 228 us.
+// Accumulation per output is in the order of the other forms (k-step by k-step, k = 16 g + 0..7
+// before 16 g + 8..15), so the results are bit-identical to them.
+constexpr int kMidGroups = 64;  // scale groups (128 of K) per LDS table
+
+template <int WF>
+struct MidCfg {
+    static constexpr int RING = WF == YVMOE_W_BF16 ? 3 : 4;  // weight ring, k-steps (deeper: no gain)
+    static constexpr int WD = WF == YVMOE_W_BF16 ? 4 : 2;    // weight loads per k-step
+    static constexpr bool GROUPED = WF == YVMOE_W_INT4 || WF == YVMOE_W_FP8;
+    // group scales of a range of K in LDS: int4 bf16, kMidGroups (+ 2 against bank conflicts) per
+    // weight row; fp8 fp32, kMidGroups per matrix
+    static constexpr int S_BYTES = WF == YVMOE_W_INT4 ? 128 * (kMidGroups + 2) * 2
+                                 : WF == YVMOE_W_FP8  ? 2 * kMidGroups * 4 : 16;
+};
+
+// One tile (rows row0 .. seg_end - 1, at most 16 * MRB) against column group cgroup.
+template <int WF, int EPI, int MRB, int MAXMRB>
+__device__ __forceinline__ void mid_item(const GemmParams& p, int e, int row0, int seg_end, int cgroup,
+                                         unsigned char (&lds_a)[3][MAXMRB * 2048], unsigned char* lds_s) {
+    typedef BLoad<WF> BL;
+    typedef MidCfg<WF> C;
+    constexpr bool SWIGLU = EPI == EPI_SWIGLU;
+    constexpr int RING = C::RING, AD = MRB / 2;  // AD: 1 KB activation loads (8 rows) per wavefront and k-step
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int g = lane >> 4, i16 = lane & 15;
+    const long long e_off = (long long)e * p.b_stride;
+    const long long s_off = (long long)e * p.s_stride;
+    // first column of this wavefront (columns past the last one: the last ones again, not stored)
+    const int nw = SWIGLU ? cgroup * 64 + wave * 16 : cgroup * 128 + wave * 32;
+    const int n0 = min(nw, p.ncols - (SWIGLU ? 16 : 32));
+    const char* bptr[2];
+    float cs[2];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+        const int n = SWIGLU ? n0 + i16 : n0 + nb * 16 + i16;
+        bptr[nb] = BL::bptr(SWIGLU && nb ? p.B1 : p.B0, e_off, n, p.K, 0, lane);
+        if constexpr (!C::GROUPED) cs[nb] = b_scale<WF>(SWIGLU && nb ? p.S1 : p.S0, s_off, n, p.K, 0);
+    }
+    // activation block j of this wavefront: tile rows 8 (AD w + j) .. + 7, lane L row + L / 8,
+    // logical chunk (L % 8) ^ (L / 8) ^ (block & 1); rows past the tile re-read its first row
+    const char* a_src[AD];
+#pragma unroll
+    for (int j = 0; j < AD; ++j) {
+        const int blk = wave * AD + j;
+        const int r = blk * 8 + lane / 8;
+        const int lc = (lane % 8) ^ (lane / 8) ^ (blk & 1);
+        const int gr = (row0 + r < seg_end) ? row0 + r : row0;
+        a_src[j] = (const char*)p.A + ((long long)map_row(p, gr) * p.lda + lc * 8) * 2;
+    }
+    const int a_rd0 = swz_a(i16, 2 * g), a_rd1 = swz_a(i16, 2 * g + 1);
+
+    f32x4 acc[MRB][2];
+#pragma unroll
+    for (int mb = 0; mb < MRB; ++mb) acc[mb][0] = acc[mb][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    const int nks = p.K / 64;
+    constexpr int SEG = C::GROUPED ? 2 * kMidGroups : 1 << 30;  // k-steps per scale table
+    for (int kb = 0; kb < nks; kb += SEG) {
+        const int n = min(SEG, nks - kb);
+        if constexpr (C::GROUPED) {
+            const int kg = p.K / 128, q0 = kb / 2, nq = (n + 1) / 2;
+            if constexpr (WF == YVMOE_W_INT4) {
+                unsigned short* tab = (unsigned short*)lds_s;
+                for (int i = t; i < 128 * nq; i += 256) {
+                    const int r = i / nq, q = i % nq;  // row r: wavefront r / 32, fragment (r / 16) % 2
+                    const int col = SWIGLU ? cgroup * 64 + (r >> 5) * 16 + (r & 15) : cgroup * 128 + r;
+                    const void* S = SWIGLU && (r & 16) ? p.S1 : p.S0;
+                    tab[r * (kMidGroups + 2) + q] =
+                        ((const unsigned short*)S)[s_off + (long long)min(col, p.ncols - 1) * kg + q0 + q];
+                }
+            } else {
+                // the work-group's columns lie in one 128-column scale block
+                float* tab = (float*)lds_s;
+                const int m = t / nq, q = t % nq;
+                if (m < (SWIGLU ? 2 : 1)) {
+                    const int col = cgroup * (SWIGLU ? 64 : 128);
+                    tab[m * kMidGroups + q] =
+                        ((const float*)(m ? p.S1 : p.S0))[s_off + (long long)(col / 128) * kg + q0 + q];
+                }
+            }
+            __syncthreads();  // the table, before any direct load is in flight
+        }
+        typename BL::Raw w[RING][2];
+        // loads past the end repeat the last k-step (into a free stage or ring slot, never used),
+        // so every wait below has a fixed count
+        auto load_w = [&](int c, typename BL::Raw (&dst)[2]) {
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) BL::load_blk_nt(dst[nb], bptr[nb], kb + min(c, n - 1));
+        };
+        auto issue_a = [&](int c, int st) {
+            const size_t off = (size_t)(kb + min(c, n - 1)) * 128;
+#pragma unroll
+            for (int j = 0; j < AD; ++j) dma16(a_src[j] + off, &lds_a[st][(wave * AD + j) * 1024]);
+        };
+#pragma unroll
+        for (int r = 0; r < RING - 3; ++r) load_w(r, w[r]);
+        issue_a(0, 0);
+        load_w(RING - 3, w[RING - 3]);
+        issue_a(1, 1);
+        load_w(RING - 2, w[RING - 2]);
+        int st = 0;
+        // k-step c from ring slot cur; AHEAD: the weights of step c + RING - 1 go to slot nxt
+        auto step = [&](int c, typename BL::Raw (&cur)[2], typename BL::Raw (&nxt)[2], auto ahead) {
+            constexpr bool AHEAD = decltype(ahead)::value;
+            // this wavefront's activation loads of step c have landed (younger: at least step
+            // c + 1's; with AHEAD also the weights of two steps); after the barrier every
+            // wavefront's have, and all reads of step c - 1 are done, so its stage takes step c + 2
+            __builtin_amdgcn_s_waitcnt(vmcnt_only(AHEAD ? 2 * C::WD + AD : AD));
+            __builtin_amdgcn_s_waitcnt(lgkm_only(0));
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            int s2 = st + 2;
+            if (s2 >= 3) s2 -= 3;
+            issue_a(c + 2, s2);
+            if constexpr (AHEAD) load_w(c + RING - 1, nxt);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            Frag16 bq[2];
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                float s;
+                if constexpr (WF == YVMOE_W_INT4)
+                    s = bf16_to_f32(((const unsigned short*)lds_s)[(wave * 32 + nb * 16 + i16) * (kMidGroups + 2) + (c >> 1)]);
+                else if constexpr (WF == YVMOE_W_FP8)
+                    s = ((const float*)lds_s)[(SWIGLU ? nb : 0) * kMidGroups + (c >> 1)];
+                else
+                    s = cs[nb];
+                BL::cvt(cur[nb], s, bq[nb]);
+            }
+            const unsigned char* As = lds_a[st];
+#pragma unroll
+            for (int mb = 0; mb < MRB; ++mb) {
+                const bf16x8 a0 = *(const bf16x8*)(As + a_rd0 + mb * 16 * 128);
+                const bf16x8 a1 = *(const bf16x8*)(As + a_rd1 + mb * 16 * 128);
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb) {
+                    acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bq[nb].v[0], a0, acc[mb][nb], 0, 0, 0);
+                    acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bq[nb].v[1], a1, acc[mb][nb], 0, 0, 0);
+                }
+            }
+            if (++st == 3) st = 0;
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        int c = 0;
+        for (; c + RING <= n; c += RING) {
+#pragma unroll
+            for (int r = 0; r < RING; ++r) step(c + r, w[r], w[(r + RING - 1) % RING], std::true_type{});
+        }
+        // fewer than RING steps left: their weights are in slots 0 .. (no weight loads here: the
+        // compiler would drop them as unused, and the counts above with them)
+#pragma unroll
+        for (int r = 0; r < RING - 1; ++r)
+            if (c + r < n) step(c + r, w[r], w[(r + RING - 1) % RING], std::false_type{});
+        // the repeated loads of the last steps have landed (and, before another range of K, every
+        // wavefront's reads are done)
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+        if (kb + SEG < nks) __syncthreads();
+    }
+    if (nw >= p.ncols) return;
+    // weights are the first operand: a lane holds row i16 of each row block and 4 consecutive
+    // columns of each fragment
+#pragma unroll
+    for (int mb = 0; mb < MRB; ++mb) {
+        const int r = row0 + mb * 16 + i16;
+        if (r >= seg_end) continue;
+        unsigned short* o = (unsigned short*)p.out + (long long)r * p.ldo + n0 + 4 * g;
+        if constexpr (SWIGLU) {
+            float hv[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float gt = round_bf16(acc[mb][0][i]);
+                const float up = round_bf16(acc[mb][1][i]);
+                hv[i] = round_bf16(silu(gt)) * up;
+            }
+            *(uint2*)o = make_uint2(pack_bf16(hv[0], hv[1]), pack_bf16(hv[2], hv[3]));
+        } else {
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb)
+                *(uint2*)(o + nb * 16) = make_uint2(pack_bf16(acc[mb][nb][0], acc[mb][nb][1]),
+                                                    pack_bf16(acc[mb][nb][2], acc[mb][nb][3]));
+        }
+    }
+}
+
+// Column groups per XCD and tile: consecutive work-group ids go to different XCDs, and XCD x
+// takes the groups x - e (mod 8) of every tile of expert e. Each XCD then sees every tile (an
+// even load, although the shared experts' tiles are the fullest and stand last in the table), the
+// tiles of one expert read a column group's weights on one XCD, and an XCD's groups of a tile
+// run together on the tile's rows. Tiles run last to first, so the full ones do not end the
+// launch. (FFN at 64 experts of 47 rows: contiguous ranges of the items per XCD 348 us tile by
+// tile, 309 us group by group; 288 us in this order.)
+template <int WF, int EPI, int MAXMRB>
+__global__ __launch_bounds__(256, (MAXMRB == 8 ? 3 : 4) - (WF == YVMOE_W_INT4 ? 1 : 0)) void gemm_mid_kernel(GemmParams p, int ngroups) {
+    __shared__ __attribute__((aligned(1024))) unsigned char lds_a[3][MAXMRB * 2048];
+    __shared__ __attribute__((aligned(16))) unsigned char lds_s[MidCfg<WF>::S_BYTES];
+    const int local = blockIdx.x / 8, x = blockIdx.x % 8;
+    const int per_tile = (ngroups + 7) / 8;
+    const int tile = *p.ntiles - 1 - local / per_tile;
+    if (tile < 0) return;
+    const int e = p.tile_seg[tile], row0 = p.tile_row0[tile];
+    const int cgroup = ((x + e) & 7) + 8 * (local % per_tile);
+    if (cgroup >= ngroups) return;
+    const int seg_end = min(p.seg_start[e + 1], row0 + MAXMRB * 16);
+    const int rows = seg_end - row0;
+    if constexpr (MAXMRB == 8) {
+        if (rows > 96) return mid_item<WF, EPI, 8, MAXMRB>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
+        if (rows > 64) return mid_item<WF, EPI, 6, MAXMRB>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
+    }
+    if (rows > 32) return mid_item<WF, EPI, 4, MAXMRB>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
+    mid_item<WF, EPI, 2, MAXMRB>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
+}
+
 // ------------------------------------------------------------------ fp32 activations
 // fp32 activations and fp32 weights (the reference's fp32 configuration).
 template <int EPI, int NCB>
@@ -2092,6 +2276,30 @@ int stream_dispatch(int wf, const GemmParams& p, int ntiles_max, hipStream_t st,
     return YVMOE_OK;
 }
 
+// Mid-sized form: tile_rows-row (64 or 128) tiles of the tile table; the grid covers 8 XCDs x
+// (the most tiles the batch can have) x column groups per XCD.
+template <int EPI>
+int mid_dispatch(int wf, const GemmParams& p, int ntiles_max, int tile_rows, hipStream_t st, const char* name) {
+    const int ngroups = ceil_div(p.ncols, EPI == EPI_SWIGLU ? 64 : 128);
+    const long long items = 8LL * ntiles_max * ceil_div(ngroups, 8);
+    if (items <= 0) return YVMOE_OK;
+#define YV_MID(WFV)                                                                                   \
+    do {                                                                                              \
+        if (tile_rows == 64) gemm_mid_kernel<WFV, EPI, 4><<<(unsigned)items, 256, 0, st>>>(p, ngroups); \
+        else gemm_mid_kernel<WFV, EPI, 8><<<(unsigned)items, 256, 0, st>>>(p, ngroups);               \
+    } while (0)
+    switch (wf) {
+        case YVMOE_W_BF16: YV_MID(YVMOE_W_BF16); break;
+        case YVMOE_W_INT8: YV_MID(YVMOE_W_INT8); break;
+        case YVMOE_W_INT4: YV_MID(YVMOE_W_INT4); break;
+        case YVMOE_W_FP8: YV_MID(YVMOE_W_FP8); break;
+        default: set_error("unsupported weight format %d for bf16 activations", wf); return YVMOE_ERR_DTYPE;
+    }
+#undef YV_MID
+    YV_LAUNCH_CHECK(name);
+    return YVMOE_OK;
+}
+
 // LDS-tiled (prefill) form: one work-group per (256-row tile, column block of 128 (gate/up)
 // or 256 (down)); grid = 8 x per-XCD range, sized for the most tiles the batch can have.
 // fold: the tile table folds remainders (tile_fold), so the form with folded rows runs.
@@ -2180,10 +2388,11 @@ int tile_launch(int wf, const GemmParams& p, int ntiles_max, hipStream_t st, con
     return YVMOE_OK;
 }
 
-// Launches one GEMM: grid (tiles, column groups, K splits); NCB 16-column blocks per wave.
+// Launches one GEMM: grid (tiles, column groups, K splits); NCB 16-column blocks per wave. bf16
+// activations: the dense fp32-output form only (the expert GEMMs have forms of their own).
 template <int EPI>
-int gemm_dispatch(int act, int wf, GemmParams p, int ntiles_max, int ncb, int ksplit,
-                  hipStream_t st, const char* name, int maxrb = 4) {
+int gemm_dispatch(int act, GemmParams p, int ntiles_max, int ncb, int ksplit, hipStream_t st,
+                  const char* name) {
     if (ntiles_max <= 0) return YVMOE_OK;
     if (p.ncols % (16 * ncb) != 0) {
         set_error("%s: %d columns are not a multiple of %d", name, p.ncols, 16 * ncb);
@@ -2194,25 +2403,12 @@ int gemm_dispatch(int act, int wf, GemmParams p, int ntiles_max, int ncb, int ks
     if (act == YVMOE_ACT_F32) {
         if (ncb == 2) gemm_f32_kernel<EPI, 2><<<grid, 256, 0, st>>>(p);
         else gemm_f32_kernel<EPI, 1><<<grid, 256, 0, st>>>(p);
+    } else if constexpr (EPI == EPI_F32) {
+        if (ncb == 2) gemm_bf16_kernel<2><<<grid, 256, 0, st>>>(p);
+        else gemm_bf16_kernel<1><<<grid, 256, 0, st>>>(p);
     } else {
-#define YV_GB(WFV)                                                                  \
-    do {                                                                            \
-        if (maxrb == 1) {                                                           \
-            if (ncb == 2) gemm_bf16_kernel<WFV, EPI, 2, 1><<<grid, 256, 0, st>>>(p); \
-            else gemm_bf16_kernel<WFV, EPI, 1, 1><<<grid, 256, 0, st>>>(p);         \
-        } else {                                                                    \
-            if (ncb == 2) gemm_bf16_kernel<WFV, EPI, 2, 4><<<grid, 256, 0, st>>>(p); \
-            else gemm_bf16_kernel<WFV, EPI, 1, 4><<<grid, 256, 0, st>>>(p);         \
-        }                                                                           \
-    } while (0)
-        switch (wf) {
-            case YVMOE_W_BF16: YV_GB(YVMOE_W_BF16); break;
-            case YVMOE_W_INT8: YV_GB(YVMOE_W_INT8); break;
-            case YVMOE_W_INT4: YV_GB(YVMOE_W_INT4); break;
-            case YVMOE_W_FP8: YV_GB(YVMOE_W_FP8); break;
-            default: set_error("unsupported weight format %d for bf16 activations", wf); return YVMOE_ERR_DTYPE;
-        }
-#undef YV_GB
+        set_error("%s: bf16 activations take another form", name);
+        return YVMOE_ERR_UNSUPPORTED;
     }
     YV_LAUNCH_CHECK(name);
     return YVMOE_OK;
@@ -2232,23 +2428,22 @@ int dense_gemm_launch(const void* x, int act, int N, int K, const void* w, int n
     p.ncols = ncols;
     p.ldo = ld;
     p.nrows = N;
-    const int wf = (act == YVMOE_ACT_F32) ? YVMOE_W_F32 : YVMOE_W_BF16;
     if (dense_tiled(act, N, ncols, K)) {
         p.kchunk = K;
         p.out = out;
-        return tile_dispatch<EPI_F32>(wf, p, ceil_div(N, TBM), st, name);
+        return tile_dispatch<EPI_F32>(YVMOE_W_BF16, p, ceil_div(N, TBM), st, name);
     }
     const int ks = dense_ksplit(N, ncols, K);
     const int ncb = (ncols % 32 == 0) ? 2 : 1;
     if (ks == 1 || partials == nullptr) {
         p.kchunk = K;
         p.out = out;
-        return gemm_dispatch<EPI_F32>(act, wf, p, ceil_div(N, kTileRows), ncb, 1, st, name);
+        return gemm_dispatch<EPI_F32>(act, p, ceil_div(N, kTileRows), ncb, 1, st, name);
     }
     p.kchunk = K / ks;
     p.out = partials;
     p.split_stride = (long long)N * ld;
-    int rc = gemm_dispatch<EPI_F32>(act, wf, p, ceil_div(N, kTileRows), ncb, ks, st, name);
+    int rc = gemm_dispatch<EPI_F32>(act, p, ceil_div(N, kTileRows), ncb, ks, st, name);
     if (rc) return rc;
     return reduce_splits_launch(partials, ks, (long long)N * ld, out, st, "dense_gemm_reduce");
 }
@@ -2281,8 +2476,7 @@ int dense_partials_launch(const void* x, int act, int N, int K, const void* w, i
         // or needing more partial sums)
         return stream_dispatch<EPI_F32, 1, 1, 4, YV_DPF>(YVMOE_W_BF16, p, 1, st, name, ks);
     }
-    const int wf = (act == YVMOE_ACT_F32) ? YVMOE_W_F32 : YVMOE_W_BF16;
-    return gemm_dispatch<EPI_F32>(act, wf, p, ceil_div(N, kTileRows), (ncols % 32 == 0) ? 2 : 1, ks,
+    return gemm_dispatch<EPI_F32>(act, p, ceil_div(N, kTileRows), (ncols % 32 == 0) ? 2 : 1, ks,
                                   st, name);
 }
 
@@ -2297,7 +2491,6 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
     p.ncols = router_ld(r->num_experts, act);
     p.ldo = ld;
     p.nrows = N;
-    const int wf = (act == YVMOE_ACT_F32) ? YVMOE_W_F32 : YVMOE_W_BF16;
     const int ks = router_ksplit(N, r->num_experts, act, r->hidden);
     if (router_tiled(act, N, p.ncols, r->hidden)) {
         // large batches: the LDS-tiled MFMA form over (tile, column block, K split) items, the
@@ -2319,7 +2512,7 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
         p.kchunk = r->hidden;
         p.out = out;
         const int ncb = (p.ncols % 32 == 0) ? 2 : 1;
-        return gemm_dispatch<EPI_F32>(act, wf, p, ceil_div(N, kTileRows), ncb, 1, st, "router_gemm");
+        return gemm_dispatch<EPI_F32>(act, p, ceil_div(N, kTileRows), ncb, 1, st, "router_gemm");
     }
     p.out = partials;
     p.split_stride = (long long)N * ld;
@@ -2330,20 +2523,37 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
     if (dense_streamed(act, N, p.ncols, r->hidden))
         rc = stream_dispatch<EPI_F32, 4, 1, 1>(YVMOE_W_BF16, p, ceil_div(N, 16), st, "router_gemm", ks);
     else
-        rc = gemm_dispatch<EPI_F32>(act, wf, p, ceil_div(N, kTileRows), 1, ks, st, "router_gemm");
+        rc = gemm_dispatch<EPI_F32>(act, p, ceil_div(N, kTileRows), 1, ks, st, "router_gemm");
     if (rc || !reduce) return rc;
     return reduce_splits_launch(partials, ks, (long long)N * ld, out, st, "router_reduce");
 }
 
+// Rows per tile of the expert GEMMs, which is also their form, by the mean rows per expert (slots
+// / E) and the weight format (bf16 activations; fp32 has its own kernel on 64-row tiles):
+// * 16: weight streaming, up to 8 rows (int4: 4). It reads a tile's weights once per 16 rows;
+//   int8 6 / 9 / 12 rows: 191 / 205 / 220 us against 197 / 200 / 204 on the mid form (H 4096, 64
+//   experts); int4 6 rows: 190 against 171 (its 8-byte weight loads want the mid form's ring).
+// * 64: the mid form with 64-row tiles, which take less LDS and give more work-groups: int4 up to
+//   48 rows (its scale table costs 128-row tiles a third work-group per CU: 32 rows 228 us
+//   against 246), and any format up to 48 rows when 128-row tiles would leave the down
+//   projection under two work-groups per CU (H 1024, 8 experts of 16 / 32 rows: 48.5 / 48.7 us
+//   against 48.2 / 58.3).
+// * 128: the mid form, up to 144 rows for int8 and int4 and 112 for bf16 and fp8, from where an
+//   expert's rows past 128 cost a second pass over its weights (H 4096, 64 experts, 96 / 131 /
+//   159 rows: int8 386 / 546 / 696 us against 576 / 601 / 669 on 256-row tiles, bf16 546 / 817 /
+//   1038 against 646 / 653 / 680; fp8 H 7168, 256 experts, 94 / 128 rows 2864 / 4203 against 3309 /
+//   3823), and any number of rows where the 256-row form does not take the shape.
+// * 256: the LDS-tiled form above that.
 int ffn_tile_rows(int act, int N, int k, int E, int H, int F, int wf) {
-    // 256-row LDS-tiled form when experts hold many rows (prefill-like batches)
-    const bool tiled = act == YVMOE_ACT_BF16 && N * k >= 64 * E && F % (TBN / 2) == 0 && H % TBN == 0 &&
-                       (wf == YVMOE_W_INT8 || wf == YVMOE_W_BF16 ||
-                        ((wf == YVMOE_W_FP8 || wf == YVMOE_W_INT4) && H <= 8192 && F <= 8192));
-    if (tiled) return TBM;
-    // 16-row tiles (one MFMA row block per wave) when experts hold few rows (decode-like
-    // batches), 64-row tiles otherwise
-    return (act == YVMOE_ACT_BF16 && N * k <= 32 * E) ? 16 : 64;
+    if (act != YVMOE_ACT_BF16) return kTileRows;
+    const long long slots = (long long)N * k;
+    if (slots < (wf == YVMOE_W_INT4 ? 4LL : 8LL) * E) return 16;
+    const bool tiles = F % (TBN / 2) == 0 && H % TBN == 0 &&
+                       (wf == YVMOE_W_INT8 || wf == YVMOE_W_BF16 || (H <= 8192 && F <= 8192));
+    const long long most = wf == YVMOE_W_INT8 || wf == YVMOE_W_INT4 ? 144 : 112;
+    if (tiles && slots >= most * E) return TBM;
+    if (slots <= 48LL * E && (wf == YVMOE_W_INT4 || (long long)E * ceil_div(H, 128) < 512)) return 64;
+    return 128;
 }
 
 TileTable ffn_tile_table(int N, int k, int E, int S, int F, int act, int tile_rows, char* ws) {
@@ -2373,8 +2583,8 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
     char* fws = ws + RL.bytes;
     void* hbuf = fws + FL.h;
     const int tile_rows = ffn_tile_rows(act, N, k, E, H, F, w->format);
-    const bool tiled = tile_rows == TBM;
-    const int maxrb = tile_rows == 16 ? 1 : 4;
+    const bool tiled = tile_rows == TBM, streaming = tile_rows == 16;
+    const bool mid = act == YVMOE_ACT_BF16 && !tiled && !streaming;
     const TileTable tt = ffn_tile_table(N, k, E, S, F, act, tile_rows, ws);
     int* seg = tt.seg;
     int* tile_seg = tt.tile_seg;
@@ -2430,13 +2640,12 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
     p.out = hbuf;
     p.ldo = F;
     p.kchunk = H;
-    const bool streaming = (maxrb == 1);
-    int rc = tiled ? tile_dispatch<EPI_SWIGLU>(wf, p, T, st, "expert_gemm1", tt.fold > 0)
+    int rc = mid ? mid_dispatch<EPI_SWIGLU>(wf, p, T, tile_rows, st, "expert_gemm1")
+           : tiled ? tile_dispatch<EPI_SWIGLU>(wf, p, T, st, "expert_gemm1", tt.fold > 0)
            : streaming ? (S > 0
                               ? stream_dispatch<EPI_SWIGLU, YV_U1, YV_NB1, 1, YV_PF1, YV_WV1, true>(wf, p, T, st, "expert_gemm1")
                               : stream_dispatch<EPI_SWIGLU, YV_U1, YV_NB1, 1, YV_PF1, YV_WV1>(wf, p, T, st, "expert_gemm1"))
-                       : gemm_dispatch<EPI_SWIGLU>(act, wf, p, T, (F % 32 == 0) ? 2 : 1, 1, st,
-                                                   "expert_gemm1", maxrb);
+                       : gemm_dispatch<EPI_SWIGLU>(act, p, T, (F % 32 == 0) ? 2 : 1, 1, st, "expert_gemm1");
     if (rc != YVMOE_OK) return rc;
     if (tt.light > 0) {
         rc = light_launch(p, std::integral_constant<int, EPI_SWIGLU>{}, "expert_gemm1_light");
@@ -2464,11 +2673,11 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
         if (rc != YVMOE_OK || tt.light == 0) return rc;
         return light_launch(p, std::integral_constant<int, EPI_DOWN>{}, "expert_gemm2_light");
     }
+    if (mid) return mid_dispatch<EPI_DOWN>(wf, p, T, tile_rows, st, "expert_gemm2");
     return streaming ? (S > 0
                             ? stream_dispatch<EPI_DOWN, YV_U2, YV_NB2, 1, YV_PF2, YV_WV2, true>(wf, p, T, st, "expert_gemm2")
                             : stream_dispatch<EPI_DOWN, YV_U2, YV_NB2, 1, YV_PF2, YV_WV2>(wf, p, T, st, "expert_gemm2"))
-                     : gemm_dispatch<EPI_DOWN>(act, wf, p, T, (H % 32 == 0) ? 2 : 1, 1, st,
-                                               "expert_gemm2", maxrb);
+                     : gemm_dispatch<EPI_DOWN>(act, p, T, (H % 32 == 0) ? 2 : 1, 1, st, "expert_gemm2");
 }
 
 int combine_launch(const void* y, int act, int N, int H, int k, int S, const yvmoe_routing* routing,

@@ -1,0 +1,59 @@
+"""The mid-sized expert GEMM form (64- and 128-row tiles, a few to about a hundred rows per
+expert) where it can go wrong: segment lengths at the edges of its row-block variants and
+tiles, K of fewer k-steps than its weight ring, partial last column groups, and scale tables
+refilled every 8192 of K."""
+import pytest
+import torch
+
+from test_gpu_layer import _run_and_check
+from pisceslx_amd.workloads import LayerSpec, make_workload
+
+pytestmark = pytest.mark.gpu
+
+# rows per expert: the edges of the 32-, 64-, 96- and 128-row variants, an empty expert and an
+# expert of two tiles; the first list is mean 56 (128-row tiles), the second 30 (64-row tiles on
+# these small layers)
+WIDE = [0, 1, 15, 17, 32, 33, 63, 65, 96, 97, 128, 129]
+NARROW = [1, 16, 31, 33, 64, 65, 0, 30]
+
+
+def forced_rows(spec, counts, seed=7):
+    """A workload whose expert e receives exactly counts[e] tokens (one-hot gate rows, top-1)."""
+    N, E, H = sum(counts), len(counts), spec.hidden
+    w = make_workload(spec, device="cuda", lengths=[N])
+    g = torch.Generator().manual_seed(seed)
+    expert = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(N, generator=g)]
+    x = torch.randn(N, H, generator=g) * 0.5
+    x[torch.arange(N), expert] += 8.0
+    gate = torch.zeros(E, H)
+    gate[torch.arange(E), torch.arange(E)] = 1.0
+    w.x = x.to(torch.bfloat16).cuda()
+    w.gate_weight = gate.to(torch.bfloat16).cuda()
+    return w
+
+
+@pytest.mark.parametrize("counts", [WIDE, NARROW], ids=["rows128", "rows64"])
+@pytest.mark.parametrize("fmt,hidden,ffn", [
+    ("int8", 192, 320),    # 3 and 5 k-steps; 1.5 down column groups
+    ("bf16", 64, 192),     # a single k-step
+    ("int8", 1024, 1088),  # 16 and 17 k-steps (ring remainders 0 and 1), 17 gate/up groups
+    ("int4", 128, 384),
+    ("fp8", 384, 128),
+    ("int4", 8320, 128),   # K past one scale table
+    ("fp8", 8320, 128),
+])
+def test_segment_edges(cuda, oracle, fmt, hidden, ffn, counts):
+    from pisceslx_amd import _lib
+    spec = LayerSpec("mid", hidden, ffn, len(counts), 1, 1, getattr(_lib, "W_" + fmt.upper()),
+                     torch.bfloat16, fixed_shape_mode=True)
+    w = forced_rows(spec, counts)
+    _, _, routing = _run_and_check(oracle, w, label=f"mid {fmt} H={hidden} F={ffn} N={sum(counts)}")
+    assert routing.counts.cpu().tolist() == counts
+
+
+@pytest.mark.parametrize("n", [10, 11, 85, 86, 193, 512])
+def test_form_boundaries(cuda, oracle, n):
+    """Token counts on both sides of the rules' lines (8 experts' rows at top-6 of 8)."""
+    from pisceslx_amd import _lib
+    spec = LayerSpec("midline", 512, 256, 8, 6, 1, _lib.W_INT8, torch.bfloat16)
+    _run_and_check(oracle, make_workload(spec, device="cuda", lengths=[n]), label=f"mid line N={n}")
