@@ -1900,25 +1900,16 @@ __global__ __launch_bounds__(256, (MAXMRB == 8 ? 3 : 4) - (WF == YVMOE_W_INT4 ? 
     mid_item<WF, EPI, 2, MAXMRB>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
 }
 
-// ------------------------------------------------------------------ fp32 activations
-// fp32 activations and fp32 weights (the reference's fp32 configuration).
-template <int EPI, int NCB>
+// ------------------------------------------------------------------ fp32, dense
+// out[r][n] (+ split z at z * split_stride) = A · Wᵀ in fp32 (the router's and the YvMoEGate's
+// projections of fp32 activations): 64-row tiles, NCB 16-column blocks per wavefront.
+template <int NCB>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmParams p) {
-    constexpr int NM = NMat<EPI>::value;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    int e = 0, row0, seg_end;
-    if (p.tile_seg != nullptr) {
-        const int tile = blockIdx.x;
-        if (tile >= *p.ntiles) return;
-        e = p.tile_seg[tile];
-        row0 = p.tile_row0[tile];
-        seg_end = p.seg_start[e + 1];
-    } else {
-        row0 = blockIdx.x * kTileRows;
-        if (row0 >= p.nrows) return;
-        seg_end = p.nrows;
-    }
+    const int row0 = blockIdx.x * kTileRows;
+    if (row0 >= p.nrows) return;
+    const int seg_end = p.nrows;
     const int col0 = (blockIdx.y * 4 + wave) * NCB * 16;
     if (col0 >= p.ncols) return;
     const int nrb = min(4, (seg_end - row0 + 15) / 16);
@@ -1930,47 +1921,37 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmParams p) {
     for (int rb = 0; rb < 4; ++rb) {
         int r = row0 + rb * 16 + (lane & 15);
         if (r >= seg_end) r = row0;
-        arow[rb] = (const float*)p.A + (long long)map_row(p, r) * p.lda + kl;
+        arow[rb] = (const float*)p.A + (long long)r * p.lda + kl;
     }
-    const long long e_off = (long long)e * p.b_stride;
-    const float* bptr[NM][NCB];
+    const float* bptr[NCB];
 #pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) {
-        const int n = col0 + cb * 16 + (lane & 15);
-        bptr[0][cb] = (const float*)p.B0 + e_off + (long long)n * p.K + kl;
-        if constexpr (NM == 2) bptr[NM - 1][cb] = (const float*)p.B1 + e_off + (long long)n * p.K + kl;
-    }
-    f32x4 acc[NM][NCB][4];
+    for (int cb = 0; cb < NCB; ++cb)
+        bptr[cb] = (const float*)p.B0 + (long long)(col0 + cb * 16 + (lane & 15)) * p.K + kl;
+    f32x4 acc[NCB][4];
 #pragma unroll
-    for (int m = 0; m < NM; ++m)
+    for (int cb = 0; cb < NCB; ++cb)
 #pragma unroll
-        for (int cb = 0; cb < NCB; ++cb)
-#pragma unroll
-            for (int rb = 0; rb < 4; ++rb) acc[m][cb][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int rb = 0; rb < 4; ++rb) acc[cb][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int k0 = kbeg; k0 < kend; k0 += 16) {
-        float4 bv[NM][NCB];
+        float4 bv[NCB];
 #pragma unroll
-        for (int m = 0; m < NM; ++m)
-#pragma unroll
-            for (int cb = 0; cb < NCB; ++cb) bv[m][cb] = *(const float4*)(bptr[m][cb] + k0);
+        for (int cb = 0; cb < NCB; ++cb) bv[cb] = *(const float4*)(bptr[cb] + k0);
         float4 av[4];
 #pragma unroll
         for (int rb = 0; rb < 4; ++rb)
             if (rb < nrb) av[rb] = *(const float4*)(arow[rb] + k0);
 #pragma unroll
-        for (int m = 0; m < NM; ++m)
+        for (int cb = 0; cb < NCB; ++cb)
 #pragma unroll
-            for (int cb = 0; cb < NCB; ++cb)
-#pragma unroll
-                for (int rb = 0; rb < 4; ++rb) {
-                    if (rb < nrb) {
-                        f32x4& d = acc[m][cb][rb];
-                        d = __builtin_amdgcn_mfma_f32_16x16x4f32(av[rb].x, bv[m][cb].x, d, 0, 0, 0);
-                        d = __builtin_amdgcn_mfma_f32_16x16x4f32(av[rb].y, bv[m][cb].y, d, 0, 0, 0);
-                        d = __builtin_amdgcn_mfma_f32_16x16x4f32(av[rb].z, bv[m][cb].z, d, 0, 0, 0);
-                        d = __builtin_amdgcn_mfma_f32_16x16x4f32(av[rb].w, bv[m][cb].w, d, 0, 0, 0);
-                    }
+            for (int rb = 0; rb < 4; ++rb) {
+                if (rb < nrb) {
+                    f32x4& d = acc[cb][rb];
+                    d = __builtin_amdgcn_mfma_f32_16x16x4f32(av[rb].x, bv[cb].x, d, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_16x16x4f32(av[rb].y, bv[cb].y, d, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_16x16x4f32(av[rb].z, bv[cb].z, d, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_16x16x4f32(av[rb].w, bv[cb].w, d, 0, 0, 0);
                 }
+            }
     }
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb) {
@@ -1981,14 +1962,338 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmParams p) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int r = row0 + rb * 16 + (lane >> 4) * 4 + i;
-                    if (r < seg_end) {
-                        float v;
-                        if constexpr (EPI == EPI_SWIGLU) v = silu(acc[0][cb][rb][i]) * acc[NM - 1][cb][rb][i];
-                        else if constexpr (EPI == EPI_F32) v = f32_out(p, acc[0][cb][rb][i], n, blockIdx.z);
-                        else v = acc[0][cb][rb][i];
-                        ((float*)p.out)[blockIdx.z * p.split_stride + (long long)r * p.ldo + n] = v;
-                    }
+                    if (r < seg_end)
+                        ((float*)p.out)[blockIdx.z * p.split_stride + (long long)r * p.ldo + n] =
+                            f32_out(p, acc[cb][rb][i], n, blockIdx.z);
                 }
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------ fp32, few rows per expert
+// Expert GEMM of fp32 activations and weights on the fp32 MFMAs, up to 64 rows of one expert
+// against 16 columns (gate/up: the gate and the up rows of 16 columns).
+//
+// What bounds it: HBM (the weights are 4 bytes), and at one or a few tokens the serial chain over
+// K. The four wavefronts of a work-group share the columns and deal out K in chunks of 32, so a
+// work-group streams four chunks at once and a chain is a quarter of K; each wavefront loads its
+// next chunk during the current one's MFMAs, straight to registers (the activations come through
+// L2), and the four partial sums meet in LDS in wavefront order. A tile runs the copy for its row
+// blocks. Measured (H 1024, 8 experts of
+// 2816, 2 + 1 per token; FFN, against 64-row tiles with the whole of K per wavefront): 1 token
+// 171 -> 35 us, 16 196 -> 88, 64 273 -> 127, 128 360 -> 166.
+template <int EPI, int RB>
+__device__ __forceinline__ void f32_stream_item(const GemmParams& p, int e, int row0, int seg_end, int cgroup,
+                                                f32x4* red) {
+    constexpr int NM = NMat<EPI>::value;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 4, i16 = lane & 15;
+    const int nch = p.K / 32;
+    const float* arow[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+        const int r = row0 + rb * 16 + i16;
+        arow[rb] = (const float*)p.A + (long long)map_row(p, r < seg_end ? r : row0) * p.lda + g * 4;
+    }
+    const float* wrow[NM];
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+        wrow[m] = (const float*)(m ? p.B1 : p.B0) + (long long)e * p.b_stride +
+                  (long long)(cgroup * 16 + i16) * p.K + g * 4;
+    f32x4 acc[NM][RB];
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) acc[m][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    struct Chunk {
+        f32x4 w[NM][2], a[RB][2];
+    };
+    auto load = [&](int c, Chunk& q) {  // past the end: the last chunk again, not used
+        const int k0 = min(c, nch - 1) * 32;
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) q.w[m][j] = __builtin_nontemporal_load((const f32x4*)(wrow[m] + k0 + 16 * j));
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) q.a[rb][j] = *(const f32x4*)(arow[rb] + k0 + 16 * j);
+    };
+    auto mma = [&](const Chunk& q) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int m = 0; m < NM; ++m)
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb)
+                        acc[m][rb] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.w[m][j][i], q.a[rb][j][i], acc[m][rb], 0, 0, 0);
+    };
+    Chunk q0, q1;
+    load(wave, q0);
+    int c = wave;
+    for (; c + 4 < nch; c += 8) {
+        load(c + 4, q1);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(q0);
+        load(c + 8, q0);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(q1);
+    }
+    if (c < nch) mma(q0);
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) red[((wave * NM + m) * RB + rb) * 64 + lane] = acc[m][rb];
+    __syncthreads();
+    if (wave >= RB) return;
+    // row block `wave`: the four partial sums in wavefront order; weights are the first operand, so
+    // a lane holds row i16 and 4 consecutive columns
+    f32x4 sum[NM];
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+        sum[m] = red[(m * RB + wave) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) {
+            const f32x4 v = red[((w * NM + m) * RB + wave) * 64 + lane];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum[m][i] = sum[m][i] + v[i];
+        }
+    }
+    const int r = row0 + wave * 16 + i16;
+    if (r >= seg_end) return;
+    if constexpr (EPI == EPI_SWIGLU) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum[0][i] = silu(sum[0][i]) * sum[NM - 1][i];
+    }
+    *(f32x4*)((float*)p.out + (long long)r * p.ldo + cgroup * 16 + 4 * g) = sum[0];
+}
+
+template <int EPI>
+__global__ __launch_bounds__(256, 3) void gemm_f32_stream_kernel(GemmParams p, int ngroups) {
+    __shared__ f32x4 red[4 * NMat<EPI>::value * 4 * 64];
+    // the mid-sized form's order of tiles and column groups over the XCDs
+    const int local = blockIdx.x / 8, x = blockIdx.x % 8;
+    const int per_tile = (ngroups + 7) / 8;
+    const int tile = *p.ntiles - 1 - local / per_tile;
+    if (tile < 0) return;
+    const int e = p.tile_seg[tile], row0 = p.tile_row0[tile];
+    const int cgroup = ((x + e) & 7) + 8 * (local % per_tile);
+    if (cgroup >= ngroups) return;
+    const int seg_end = min(p.seg_start[e + 1], row0 + kTileRows);
+    const int rows = seg_end - row0;
+    if (rows > 48) f32_stream_item<EPI, 4>(p, e, row0, seg_end, cgroup, red);
+    else if (rows > 32) f32_stream_item<EPI, 3>(p, e, row0, seg_end, cgroup, red);
+    else if (rows > 16) f32_stream_item<EPI, 2>(p, e, row0, seg_end, cgroup, red);
+    else f32_stream_item<EPI, 1>(p, e, row0, seg_end, cgroup, red);
+}
+
+// ------------------------------------------------------------------ fp32 on the bf16 MFMAs
+// Expert GEMM of fp32 activations and weights, up to 128 rows of one expert against 128 weight
+// rows (gate/up: 64 gate and the 64 up rows of the same columns), over K in chunks of 32.
+//
+// What bounds it: v_mfma_f32_16x16x4_f32 runs at 1/16 of the bf16 rate, so every operand is
+// split into three bf16 terms, hi + mid + lo = x exactly (round to nearest, 24 bits together),
+// and a product is the six MFMAs whose terms reach fp32's last bits: h h, h m, m h, m m, h l,
+// l h (the rest is below 2^-24 of the product), summed in fp32 smallest first. A chunk's operands
+// are loaded as fp32 into registers a chunk ahead, split once per work-group (5.5 VALU
+// instructions per element) and written to LDS as three planes of 16-row blocks in fragment
+// order (a lane's 16 bytes at 16 x lane: contiguous, conflict-free both ways); each wavefront
+// owns 64 x 64 outputs and reads 24 KB for its 96 MFMAs. 48 KB of LDS: the work-groups of a CU
+// overlap one's split with another's MFMAs.
+//
+// A term of a non-finite (or all but overflowing) operand is NaN, so a work-group that ends with
+// a non-finite sum computes its tile again on the fp32 MFMAs (f32_tile_direct): infinities and
+// NaN come out as that form gives them. Operands below 2^-110 lose low bits to bf16's range.
+// Error against 64 bits (relative 2-norm of the FFN's output): 1.11e-6 at H 1024, F 2816 and 1.63e-6
+// at H 4096, F 1408, where single fp32 MFMA sums over K have 1.29e-6 and 1.86e-6.
+// Measured (H 1024, 8 experts of 2816, 2 + 1 per token; FFN, against 64-row tiles on the fp32 MFMAs
+// without LDS): 2,052 tokens 1361 -> 663 us (160 TFLOP/s; a large fp32 matrix product reaches
+// 154), 512 438 -> 300 us. A lone work-group on a CU takes about 3,000 cycles per chunk (load,
+// split, write, barrier, read, MFMA in turn), which is what bounds small grids; a double-buffered
+// 8-wavefront form of 256 weight rows (one barrier per chunk) measured 702 us at 2,052 tokens.
+__device__ __forceinline__ void split_bf16x3(const float (&v)[8], uint4 (&o)[3]) {
+    unsigned h[4], m[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = v[2 * i], b = v[2 * i + 1];
+        h[i] = pack_bf16(a, b);
+        const float a1 = a - __uint_as_float(h[i] << 16), b1 = b - __uint_as_float(h[i] & 0xffff0000u);
+        m[i] = pack_bf16(a1, b1);
+        const float a2 = a1 - __uint_as_float(m[i] << 16), b2 = b1 - __uint_as_float(m[i] & 0xffff0000u);
+        l[i] = pack_bf16(a2, b2);
+    }
+    o[0] = make_uint4(h[0], h[1], h[2], h[3]);
+    o[1] = make_uint4(m[0], m[1], m[2], m[3]);
+    o[2] = make_uint4(l[0], l[1], l[2], l[3]);
+}
+
+// The 64 x 16 NBW outputs of one wavefront on the fp32 MFMAs, straight from memory (the operands'
+// rows as the caller's lanes hold them): the accumulator layout of gemm_f32x3_kernel.
+template <int NBW>
+__device__ __forceinline__ void f32_tile_direct(const float* const (&arow)[4], const float* const (&brow)[NBW],
+                                                int K, f32x4 (&acc)[4][NBW]) {
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NBW; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < K; k0 += 16) {
+        float4 av[4], bv[NBW];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) av[i] = *(const float4*)(arow[i] + k0);
+#pragma unroll
+        for (int i = 0; i < NBW; ++i) bv[i] = *(const float4*)(brow[i] + k0);
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+            for (int nb = 0; nb < NBW; ++nb) {
+                f32x4& d = acc[mb][nb];
+                d = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[nb].x, av[mb].x, d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[nb].y, av[mb].y, d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[nb].z, av[mb].z, d, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[nb].w, av[mb].w, d, 0, 0, 0);
+            }
+    }
+}
+
+// NBW: 16-row weight blocks per wavefront, 4 (128 weight rows per work-group) or 2 (64).
+template <int EPI, int NBW>
+__global__ __launch_bounds__(256, NBW == 4 ? 2 : 3) void gemm_f32x3_kernel(GemmParams p, int ngroups) {
+    constexpr bool SWIGLU = EPI == EPI_SWIGLU;
+    constexpr int NBLK = 8 + 2 * NBW, PER = NBLK / 4;  // 16-row blocks of a chunk; per wavefront to stage
+    constexpr int WCOLS = SWIGLU ? 16 * NBW / 2 : 16 * NBW;  // output columns per wavefront
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[3][NBLK * 1024];  // plane, block (8 A, then W)
+    // the mid-sized form's order of tiles and column groups over the XCDs
+    const int local = blockIdx.x / 8, x = blockIdx.x % 8;
+    const int per_tile = (ngroups + 7) / 8;
+    const int tile = *p.ntiles - 1 - local / per_tile;
+    if (tile < 0) return;
+    const int e = p.tile_seg[tile], row0 = p.tile_row0[tile];
+    const int cgroup = ((x + e) & 7) + 8 * (local % per_tile);
+    if (cgroup >= ngroups) return;
+    const int seg_end = min(p.seg_start[e + 1], row0 + 128);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wr = wave >> 1, wc = wave & 1;  // half of the rows, half of the weight rows
+    const int g = lane >> 4, i16 = lane & 15;
+    const int K = p.K;
+    const float* W0 = (const float*)p.B0 + (long long)e * p.b_stride;
+    const float* W1 = (const float*)p.B1 + (long long)e * p.b_stride;
+    // row i16 of 16-row block b of the tile's activations; weight row i16 of block b (blocks NBW wc
+    // .. + NBW - 1 are wavefront column wc's: gate/up the gate blocks, then the up blocks of their
+    // columns)
+    auto a_row = [&](int b) {
+        const int r = row0 + b * 16 + i16;
+        return (const float*)p.A + (long long)map_row(p, r < seg_end ? r : row0) * p.lda;
+    };
+    auto w_row = [&](int b) {
+        if constexpr (SWIGLU) {
+            const int q = b % NBW, n = cgroup * 2 * WCOLS + (b / NBW) * WCOLS + (q % (NBW / 2)) * 16 + i16;
+            return (q >= NBW / 2 ? W1 : W0) + (long long)n * K;
+        } else {
+            const int n = min(cgroup * 2 * WCOLS + b * 16, p.ncols - 16) + i16;  // past the end: not stored
+            return W0 + (long long)n * K;
+        }
+    };
+    // staging: PER blocks per wavefront; a lane takes 8 consecutive k (8 g ..) of its row
+    const float* src[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int b = wave * PER + j;
+        src[j] = (b < 8 ? a_row(b) : w_row(b - 8)) + g * 8;
+    }
+    // row blocks of the tile that hold rows; this wavefront's
+    const int nblk = (seg_end - row0 + 15) / 16;
+    const int live = min(4, max(0, nblk - wr * 4));
+
+    f32x4 acc[4][NBW];
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NBW; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    float4 raw[PER][2];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            raw[j][0] = *(const float4*)(src[j] + k0);
+            raw[j][1] = *(const float4*)(src[j] + k0 + 4);
+        }
+    };
+    load(0);
+    for (int k0 = 0; k0 < K; k0 += 32) {
+        __syncthreads();  // every wavefront has read the chunk before
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const float v[8] = {raw[j][0].x, raw[j][0].y, raw[j][0].z, raw[j][0].w,
+                                raw[j][1].x, raw[j][1].y, raw[j][1].z, raw[j][1].w};
+            uint4 pl[3];
+            split_bf16x3(v, pl);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) *(uint4*)(&lds[q][(wave * PER + j) * 1024 + lane * 16]) = pl[q];
+            __builtin_amdgcn_sched_barrier(0);  // one block's terms in registers at a time
+        }
+        load(min(k0 + 32, K - 32));
+        __syncthreads();
+        bf16x8 w[NBW][3];
+#pragma unroll
+        for (int nb = 0; nb < NBW; ++nb)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) w[nb][q] = *(const bf16x8*)(&lds[q][(8 + wc * NBW + nb) * 1024 + lane * 16]);
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb) {
+            if (mb < live) {
+                bf16x8 a[3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q) a[q] = *(const bf16x8*)(&lds[q][(wr * 4 + mb) * 1024 + lane * 16]);
+                constexpr int WT[6] = {2, 0, 1, 1, 0, 0}, AT[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+                for (int t = 0; t < 6; ++t)
+#pragma unroll
+                    for (int nb = 0; nb < NBW; ++nb)
+                        acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[nb][WT[t]], a[AT[t]], acc[mb][nb], 0, 0, 0);
+            }
+        }
+    }
+    // a non-finite sum: the tile again on the fp32 MFMAs
+    bool bad = false;
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NBW; ++nb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bad |= !(fabsf(acc[mb][nb][i]) < __builtin_inff());
+    if (__any(bad)) {
+        const float *ar[4], *br[NBW];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ar[i] = a_row(wr * 4 + i) + g * 4;
+#pragma unroll
+        for (int i = 0; i < NBW; ++i) br[i] = w_row(wc * NBW + i) + g * 4;
+        f32_tile_direct<NBW>(ar, br, K, acc);
+    }
+    // weights are the first operand: a lane holds row i16 of each row block and 4 consecutive
+    // columns (4 g ..) of each weight block
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) {
+        const int r = row0 + (wr * 4 + mb) * 16 + i16;
+        if (r >= seg_end) continue;
+        float* o = (float*)p.out + (long long)r * p.ldo;
+        if constexpr (SWIGLU) {
+#pragma unroll
+            for (int nb = 0; nb < NBW / 2; ++nb) {
+                f32x4 v;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = silu(acc[mb][nb][i]) * acc[mb][nb + NBW / 2][i];
+                *(f32x4*)(o + cgroup * 2 * WCOLS + wc * WCOLS + nb * 16 + 4 * g) = v;
+            }
+        } else {
+#pragma unroll
+            for (int nb = 0; nb < NBW; ++nb) {
+                const int n = cgroup * 2 * WCOLS + wc * WCOLS + nb * 16;
+                if (n < p.ncols) *(f32x4*)(o + n + 4 * g) = acc[mb][nb];
             }
         }
     }
@@ -2276,6 +2581,33 @@ int stream_dispatch(int wf, const GemmParams& p, int ntiles_max, hipStream_t st,
     return YVMOE_OK;
 }
 
+// fp32 with few rows per expert: 64-row tiles of the tile table, 16 columns per work-group.
+template <int EPI>
+int f32_stream_dispatch(const GemmParams& p, int ntiles_max, hipStream_t st, const char* name) {
+    const int ngroups = p.ncols / 16;
+    const long long items = 8LL * ntiles_max * ceil_div(ngroups, 8);
+    if (items <= 0) return YVMOE_OK;
+    gemm_f32_stream_kernel<EPI><<<(unsigned)items, 256, 0, st>>>(p, ngroups);
+    YV_LAUNCH_CHECK(name);
+    return YVMOE_OK;
+}
+
+// fp32 on the bf16 MFMAs: 128-row tiles of the tile table, the mid-sized form's grid. Work-groups
+// of 64 weight rows where those of 128 would leave CUs without one (H 1024, 8 experts of 2816,
+// down: 1,024 tokens 174 us on 128 weight rows, 146 on 64; 2,052 tokens 222 and 282).
+template <int EPI>
+int f32x3_dispatch(const GemmParams& p, int ntiles_max, hipStream_t st, const char* name) {
+    const int cols = EPI == EPI_SWIGLU ? 64 : 128;  // of 128 weight rows
+    const bool half = (long long)ntiles_max * ceil_div(p.ncols, cols) <= 256;
+    const int ngroups = ceil_div(p.ncols, half ? cols / 2 : cols);
+    const long long items = 8LL * ntiles_max * ceil_div(ngroups, 8);
+    if (items <= 0) return YVMOE_OK;
+    if (half) gemm_f32x3_kernel<EPI, 2><<<(unsigned)items, 256, 0, st>>>(p, ngroups);
+    else gemm_f32x3_kernel<EPI, 4><<<(unsigned)items, 256, 0, st>>>(p, ngroups);
+    YV_LAUNCH_CHECK(name);
+    return YVMOE_OK;
+}
+
 // Mid-sized form: tile_rows-row (64 or 128) tiles of the tile table; the grid covers 8 XCDs x
 // (the most tiles the batch can have) x column groups per XCD.
 template <int EPI>
@@ -2388,27 +2720,22 @@ int tile_launch(int wf, const GemmParams& p, int ntiles_max, hipStream_t st, con
     return YVMOE_OK;
 }
 
-// Launches one GEMM: grid (tiles, column groups, K splits); NCB 16-column blocks per wave. bf16
-// activations: the dense fp32-output form only (the expert GEMMs have forms of their own).
-template <int EPI>
-int gemm_dispatch(int act, GemmParams p, int ntiles_max, int ncb, int ksplit, hipStream_t st,
-                  const char* name) {
-    if (ntiles_max <= 0) return YVMOE_OK;
+// Dense fp32-output GEMM on 64-row tiles: grid (tiles, column groups, K splits); NCB 16-column
+// blocks per wavefront.
+int gemm_dispatch(int act, GemmParams p, int ntiles, int ncb, int ksplit, hipStream_t st, const char* name) {
+    if (ntiles <= 0) return YVMOE_OK;
     if (p.ncols % (16 * ncb) != 0) {
         set_error("%s: %d columns are not a multiple of %d", name, p.ncols, 16 * ncb);
         return YVMOE_ERR_SHAPE;
     }
     const int cols_per_wg = 4 * ncb * 16;
-    dim3 grid(ntiles_max, (p.ncols + cols_per_wg - 1) / cols_per_wg, ksplit);
+    dim3 grid(ntiles, (p.ncols + cols_per_wg - 1) / cols_per_wg, ksplit);
     if (act == YVMOE_ACT_F32) {
-        if (ncb == 2) gemm_f32_kernel<EPI, 2><<<grid, 256, 0, st>>>(p);
-        else gemm_f32_kernel<EPI, 1><<<grid, 256, 0, st>>>(p);
-    } else if constexpr (EPI == EPI_F32) {
+        if (ncb == 2) gemm_f32_kernel<2><<<grid, 256, 0, st>>>(p);
+        else gemm_f32_kernel<1><<<grid, 256, 0, st>>>(p);
+    } else {
         if (ncb == 2) gemm_bf16_kernel<2><<<grid, 256, 0, st>>>(p);
         else gemm_bf16_kernel<1><<<grid, 256, 0, st>>>(p);
-    } else {
-        set_error("%s: bf16 activations take another form", name);
-        return YVMOE_ERR_UNSUPPORTED;
     }
     YV_LAUNCH_CHECK(name);
     return YVMOE_OK;
@@ -2438,12 +2765,12 @@ int dense_gemm_launch(const void* x, int act, int N, int K, const void* w, int n
     if (ks == 1 || partials == nullptr) {
         p.kchunk = K;
         p.out = out;
-        return gemm_dispatch<EPI_F32>(act, p, ceil_div(N, kTileRows), ncb, 1, st, name);
+        return gemm_dispatch(act, p, ceil_div(N, kTileRows), ncb, 1, st, name);
     }
     p.kchunk = K / ks;
     p.out = partials;
     p.split_stride = (long long)N * ld;
-    int rc = gemm_dispatch<EPI_F32>(act, p, ceil_div(N, kTileRows), ncb, ks, st, name);
+    int rc = gemm_dispatch(act, p, ceil_div(N, kTileRows), ncb, ks, st, name);
     if (rc) return rc;
     return reduce_splits_launch(partials, ks, (long long)N * ld, out, st, "dense_gemm_reduce");
 }
@@ -2476,7 +2803,7 @@ int dense_partials_launch(const void* x, int act, int N, int K, const void* w, i
         // or needing more partial sums)
         return stream_dispatch<EPI_F32, 1, 1, 4, YV_DPF>(YVMOE_W_BF16, p, 1, st, name, ks);
     }
-    return gemm_dispatch<EPI_F32>(act, p, ceil_div(N, kTileRows), (ncols % 32 == 0) ? 2 : 1, ks,
+    return gemm_dispatch(act, p, ceil_div(N, kTileRows), (ncols % 32 == 0) ? 2 : 1, ks,
                                   st, name);
 }
 
@@ -2512,7 +2839,7 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
         p.kchunk = r->hidden;
         p.out = out;
         const int ncb = (p.ncols % 32 == 0) ? 2 : 1;
-        return gemm_dispatch<EPI_F32>(act, p, ceil_div(N, kTileRows), ncb, 1, st, "router_gemm");
+        return gemm_dispatch(act, p, ceil_div(N, kTileRows), ncb, 1, st, "router_gemm");
     }
     p.out = partials;
     p.split_stride = (long long)N * ld;
@@ -2523,13 +2850,15 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
     if (dense_streamed(act, N, p.ncols, r->hidden))
         rc = stream_dispatch<EPI_F32, 4, 1, 1>(YVMOE_W_BF16, p, ceil_div(N, 16), st, "router_gemm", ks);
     else
-        rc = gemm_dispatch<EPI_F32>(act, p, ceil_div(N, kTileRows), 1, ks, st, "router_gemm");
+        rc = gemm_dispatch(act, p, ceil_div(N, kTileRows), 1, ks, st, "router_gemm");
     if (rc || !reduce) return rc;
     return reduce_splits_launch(partials, ks, (long long)N * ld, out, st, "router_reduce");
 }
 
 // Rows per tile of the expert GEMMs, which is also their form, by the mean rows per expert (slots
-// / E) and the weight format (bf16 activations; fp32 has its own kernel on 64-row tiles):
+// / E) and the weight format. fp32 activations: 64-row tiles on the fp32 MFMAs up to 48 rows (32 /
+// 50 / 64 rows: 166 / 226 / 287 us against 223 / 222 / 232), 128-row tiles on the bf16 MFMAs above.
+// bf16 activations:
 // * 16: weight streaming, up to 8 rows (int4: 4). It reads a tile's weights once per 16 rows;
 //   int8 6 / 9 / 12 rows: 191 / 205 / 220 us against 197 / 200 / 204 on the mid form (H 4096, 64
 //   experts); int4 6 rows: 190 against 171 (its 8-byte weight loads want the mid form's ring).
@@ -2545,8 +2874,8 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
 //   3823), and any number of rows where the 256-row form does not take the shape.
 // * 256: the LDS-tiled form above that.
 int ffn_tile_rows(int act, int N, int k, int E, int H, int F, int wf) {
-    if (act != YVMOE_ACT_BF16) return kTileRows;
     const long long slots = (long long)N * k;
+    if (act != YVMOE_ACT_BF16) return slots < 48LL * E ? kTileRows : 128;
     if (slots < (wf == YVMOE_W_INT4 ? 4LL : 8LL) * E) return 16;
     const bool tiles = F % (TBN / 2) == 0 && H % TBN == 0 &&
                        (wf == YVMOE_W_INT8 || wf == YVMOE_W_BF16 || (H <= 8192 && F <= 8192));
@@ -2640,12 +2969,14 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
     p.out = hbuf;
     p.ldo = F;
     p.kchunk = H;
-    int rc = mid ? mid_dispatch<EPI_SWIGLU>(wf, p, T, tile_rows, st, "expert_gemm1")
+    const bool f3 = act != YVMOE_ACT_BF16 && tile_rows == 128;
+    int rc = f3 ? f32x3_dispatch<EPI_SWIGLU>(p, T, st, "expert_gemm1")
+           : mid ? mid_dispatch<EPI_SWIGLU>(wf, p, T, tile_rows, st, "expert_gemm1")
            : tiled ? tile_dispatch<EPI_SWIGLU>(wf, p, T, st, "expert_gemm1", tt.fold > 0)
            : streaming ? (S > 0
                               ? stream_dispatch<EPI_SWIGLU, YV_U1, YV_NB1, 1, YV_PF1, YV_WV1, true>(wf, p, T, st, "expert_gemm1")
                               : stream_dispatch<EPI_SWIGLU, YV_U1, YV_NB1, 1, YV_PF1, YV_WV1>(wf, p, T, st, "expert_gemm1"))
-                       : gemm_dispatch<EPI_SWIGLU>(act, p, T, (F % 32 == 0) ? 2 : 1, 1, st, "expert_gemm1");
+                       : f32_stream_dispatch<EPI_SWIGLU>(p, T, st, "expert_gemm1");
     if (rc != YVMOE_OK) return rc;
     if (tt.light > 0) {
         rc = light_launch(p, std::integral_constant<int, EPI_SWIGLU>{}, "expert_gemm1_light");
@@ -2673,11 +3004,12 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
         if (rc != YVMOE_OK || tt.light == 0) return rc;
         return light_launch(p, std::integral_constant<int, EPI_DOWN>{}, "expert_gemm2_light");
     }
+    if (f3) return f32x3_dispatch<EPI_DOWN>(p, T, st, "expert_gemm2");
     if (mid) return mid_dispatch<EPI_DOWN>(wf, p, T, tile_rows, st, "expert_gemm2");
     return streaming ? (S > 0
                             ? stream_dispatch<EPI_DOWN, YV_U2, YV_NB2, 1, YV_PF2, YV_WV2, true>(wf, p, T, st, "expert_gemm2")
                             : stream_dispatch<EPI_DOWN, YV_U2, YV_NB2, 1, YV_PF2, YV_WV2>(wf, p, T, st, "expert_gemm2"))
-                     : gemm_dispatch<EPI_DOWN>(act, p, T, (H % 32 == 0) ? 2 : 1, 1, st, "expert_gemm2");
+                     : f32_stream_dispatch<EPI_DOWN>(p, T, st, "expert_gemm2");
 }
 
 int combine_launch(const void* y, int act, int N, int H, int k, int S, const yvmoe_routing* routing,

@@ -1,0 +1,69 @@
+"""The fp32 expert GEMMs: the K-split form for few rows per expert and the split-operand form on
+the bf16 MFMAs, at the edges of their tiles and row blocks and of K, against the CPU oracle;
+infinities, NaN and values next to fp32's largest come out as plain fp32 arithmetic gives them."""
+import pytest
+import torch
+
+from pisceslx_amd import _lib
+from pisceslx_amd import functional as yvf
+from pisceslx_amd.quant import pack_experts
+from pisceslx_amd.workloads import LayerSpec, make_workload
+from test_gpu_layer import _run_and_check
+
+pytestmark = pytest.mark.gpu
+
+
+def forced_rows(spec, counts):
+    N, E, H = sum(counts), len(counts), spec.hidden
+    w = make_workload(spec, device="cuda", lengths=[N])
+    g = torch.Generator().manual_seed(9)
+    expert = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(N, generator=g)]
+    x = torch.randn(N, H, generator=g) * 0.5
+    x[torch.arange(N), expert] += 8.0
+    gate = torch.zeros(E, H)
+    gate[torch.arange(E), torch.arange(E)] = 1.0
+    w.x, w.gate_weight = x.cuda(), gate.cuda()
+    return w
+
+
+@pytest.mark.parametrize("counts", [[0, 1, 15, 16, 17, 33, 48, 49, 64, 65],            # mean 31
+                                    [0, 1, 16, 63, 64, 65, 80, 127, 128, 129, 200]],  # mean 79
+                         ids=["few_rows", "many_rows"])
+@pytest.mark.parametrize("hidden,ffn", [(64, 64), (192, 320), (1024, 1088), (4160, 192)])
+def test_segment_edges(cuda, oracle, hidden, ffn, counts):
+    spec = LayerSpec("f32", hidden, ffn, len(counts), 1, 1, _lib.W_F32, torch.float32, fixed_shape_mode=True)
+    w = forced_rows(spec, counts)
+    _, _, routing = _run_and_check(oracle, w, label=f"f32 H={hidden} F={ffn} N={sum(counts)}")
+    assert routing.counts.cpu().tolist() == counts
+
+
+@pytest.mark.parametrize("tokens", [40, 400])  # per expert: both forms
+def test_non_finite_and_largest_values(cuda, tokens):
+    """Positive weights, so a row with +inf gives +inf and one with NaN gives NaN in every output;
+    a row whose largest element rounds past bf16's range stays finite. Each poisons no other row."""
+    H, F, E = 128, 192, 2
+    g = torch.Generator(device="cuda").manual_seed(3)
+    ws = [tuple(torch.rand(o, i, device="cuda", generator=g).clamp(min=0.1) for o, i in ((F, H), (F, H), (H, F)))
+          for _ in range(E)]
+    for w in ws:
+        for m in w[:2]:
+            m[:, 5] = 1e-38
+    N = tokens * E
+    x = torch.rand(N, H, device="cuda", generator=g)
+    x[3, 7], x[60 % N, 9] = float("inf"), float("nan")
+    x[10, 5] = torch.finfo(torch.float32).max
+    idx = (torch.arange(N, device="cuda") % E).view(N, 1)
+    out = yvf.dispatch(x, torch.ones(N, 1, device="cuda"), idx, pack_experts(ws, E, _lib.W_F32))[0]
+    want = torch.empty(N, H, dtype=torch.float64, device="cuda")
+    for e, w in enumerate(ws):
+        a, b, d = (m.double() for m in w)
+        xs = x[e::E].double()
+        want[e::E] = (torch.nn.functional.silu(xs @ a.t()) * (xs @ b.t())) @ d.t()
+    assert torch.isposinf(out[3]).all() and torch.isnan(out[60 % N]).all()
+    keep = torch.ones(N, dtype=torch.bool, device="cuda")
+    keep[3] = keep[60 % N] = False
+    assert torch.isfinite(out[keep]).all()
+    # positive terms only: relative error of an fp32 sum of K terms is below K * 2^-24; three sums
+    # and the product of two of them
+    bound = (2 * H + F + 8) * 2.0 ** -24
+    assert float(((out[keep].double() - want[keep]).abs() / want[keep]).max()) < bound
