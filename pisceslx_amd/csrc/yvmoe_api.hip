@@ -309,8 +309,8 @@ int32_t yvmoe_forward(const void* x, int32_t act_dtype, int32_t n_tokens,
     const int S = experts->num_shared;
     TileTable tiles{};
     if (small)
-        tiles = ffn_tile_table(N, k, E, S, experts->ffn, act_dtype,
-                               ffn_tile_rows(act_dtype, N, k, E, experts->hidden, experts->ffn,
+        tiles = ffn_tile_table(N, k, E, S, experts->ffn, act_dtype, experts->format,
+                               ffn_tile_rows(act_dtype, N, k, E, S, experts->hidden, experts->ffn,
                                              experts->format),
                                ws);
     // the routing kernel builds the tile table unless it has a light part (the FFN builds that)
@@ -557,8 +557,8 @@ int32_t yvmoe_forward_moegate(const void* x, int32_t act_dtype, int32_t n_tokens
     r.fixed_shape_mode = 1;
     TileTable tiles{};
     if (small)
-        tiles = ffn_tile_table(N, k, E, S, experts->ffn, act_dtype,
-                               ffn_tile_rows(act_dtype, N, k, E, experts->hidden, experts->ffn,
+        tiles = ffn_tile_table(N, k, E, S, experts->ffn, act_dtype, experts->format,
+                               ffn_tile_rows(act_dtype, N, k, E, S, experts->hidden, experts->ffn,
                                              experts->format),
                                ws);
     const float* lsrc = route_logits != nullptr ? route_logits : logits;

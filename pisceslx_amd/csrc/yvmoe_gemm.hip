@@ -2302,18 +2302,20 @@ __global__ __launch_bounds__(256, NBW == 4 ? 2 : 3) void gemm_f32x3_kernel(GemmP
 // --------------------------------------------------------------- tile schedule
 // Segments: routed experts [0, E) from the routing offsets, then S shared experts of N
 // rows each after the N*k routed rows. Every segment is cut into tile_rows-row tiles (seg_tiles);
-// with light > 0 a remainder of at most light rows goes to the light table instead (seg_light).
+// with light > 0 a remainder of at most light rows goes to the light table instead (seg_light) if
+// there are at least light_min such remainders, else one of at most light_few rows does.
 __global__ __launch_bounds__(512) void build_tiles_kernel(const int* __restrict__ offsets, int E,
                                                           int S, int N, int k, int tile_rows,
                                                           int fold, int* __restrict__ seg,
                                                           int* __restrict__ tile_seg,
                                                           int* __restrict__ tile_row0,
                                                           int* __restrict__ ntiles, int light,
+                                                          int light_min, int light_few,
                                                           int* __restrict__ ltile_seg,
                                                           int* __restrict__ ltile_row0,
                                                           int* __restrict__ lntiles) {
-    __shared__ int sc[512];
-    __shared__ int lc[512];
+    __shared__ int sc[512];  // tiles with every remainder in the main table
+    __shared__ int lc[512];  // light remainders: of up to light_few rows above bit 16, all below
     const int tid = threadIdx.x;
     const int nseg = E + S;
     int s0 = 0, s1 = 0, nt = 0, nl = 0;
@@ -2327,8 +2329,9 @@ __global__ __launch_bounds__(512) void build_tiles_kernel(const int* __restrict_
         }
         seg[tid] = s0;
         if (tid == nseg - 1) seg[nseg] = s1;
-        nt = seg_tiles(s1 - s0, tile_rows, fold, light);
-        nl = seg_light(s1 - s0, tile_rows, fold, light);
+        nt = seg_tiles(s1 - s0, tile_rows, fold);
+        nl = seg_light(s1 - s0, tile_rows, fold, light) |
+             (seg_light(s1 - s0, tile_rows, fold, light_few) << 16);
     }
     sc[tid] = nt;
     lc[tid] = nl;
@@ -2341,20 +2344,25 @@ __global__ __launch_bounds__(512) void build_tiles_kernel(const int* __restrict_
         lc[tid] += u;
         __syncthreads();
     }
+    // a light remainder takes one tile less of the main table, for this and every later segment
+    const int sh = (lc[511] & 0xffff) >= light_min ? 0 : 16;
+    const int total = (lc[511] >> sh) & 0xffff, lend = (lc[tid] >> sh) & 0xffff;
+    nl = (nl >> sh) & 0xffff;
     if (tid < nseg) {
-        const int start = sc[tid] - nt;
+        const int start = (sc[tid] - nt) - (lend - nl);
+        nt -= nl;
         for (int q = 0; q < nt; ++q) {
             tile_seg[start + q] = tid;
             tile_row0[start + q] = s0 + q * tile_rows;
         }
         if (nl) {  // the remainder after the segment's full tiles
-            ltile_seg[lc[tid] - 1] = tid;
-            ltile_row0[lc[tid] - 1] = s0 + ((s1 - s0) / tile_rows) * tile_rows;
+            ltile_seg[lend - 1] = tid;
+            ltile_row0[lend - 1] = s0 + ((s1 - s0) / tile_rows) * tile_rows;
         }
     }
     if (tid == 511) {
-        *ntiles = sc[511];
-        if (light > 0) *lntiles = lc[511];
+        *ntiles = sc[511] - total;
+        if (light > 0) *lntiles = total;
     }
 }
 
@@ -2867,25 +2875,28 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
 //   against 246), and any format up to 48 rows when 128-row tiles would leave the down
 //   projection under two work-groups per CU (H 1024, 8 experts of 16 / 32 rows: 48.5 / 48.7 us
 //   against 48.2 / 58.3).
-// * 128: the mid form, up to 144 rows for int8 and int4 and 112 for bf16 and fp8, from where an
+// * 128: the mid form, up to 150 rows for int8 and int4 and 112 for fp8 and bf16, from where an
 //   expert's rows past 128 cost a second pass over its weights (H 4096, 64 experts, 96 / 131 /
-//   159 rows: int8 386 / 546 / 696 us against 576 / 601 / 669 on 256-row tiles, bf16 546 / 817 /
+//   159 rows: int8 386 / 546 / 690 us against 576 / 601 / 686 on 256-row tiles, bf16 546 / 817 /
 //   1038 against 646 / 653 / 680; fp8 H 7168, 256 experts, 94 / 128 rows 2864 / 4203 against 3309 /
-//   3823), and any number of rows where the 256-row form does not take the shape.
+//   3823); any number of rows where the 256-row form does not take
+//   the shape; and where 256-row tiles would be under two work-groups per CU (H 1024, 8 experts, 256
+//   / 375 rows: bf16 100 / 150 us against 127 / 134, int8 95 / 130 against 138 / 141).
 // * 256: the LDS-tiled form above that.
-int ffn_tile_rows(int act, int N, int k, int E, int H, int F, int wf) {
+int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf) {
     const long long slots = (long long)N * k;
     if (act != YVMOE_ACT_BF16) return slots < 48LL * E ? kTileRows : 128;
     if (slots < (wf == YVMOE_W_INT4 ? 4LL : 8LL) * E) return 16;
     const bool tiles = F % (TBN / 2) == 0 && H % TBN == 0 &&
                        (wf == YVMOE_W_INT8 || wf == YVMOE_W_BF16 || (H <= 8192 && F <= 8192));
-    const long long most = wf == YVMOE_W_INT8 || wf == YVMOE_W_INT4 ? 144 : 112;
-    if (tiles && slots >= most * E) return TBM;
+    const long long most = wf == YVMOE_W_INT8 || wf == YVMOE_W_INT4 ? 150 : 112;
+    const long long items = (long long)max_tiles(N, k, E, S, TBM) * ceil_div(F, TBN / 2);
+    if (tiles && slots >= most * E && items > 448) return TBM;
     if (slots <= 48LL * E && (wf == YVMOE_W_INT4 || (long long)E * ceil_div(H, 128) < 512)) return 64;
     return 128;
 }
 
-TileTable ffn_tile_table(int N, int k, int E, int S, int F, int act, int tile_rows, char* ws) {
+TileTable ffn_tile_table(int N, int k, int E, int S, int F, int act, int wf, int tile_rows, char* ws) {
     const RouteWs RL = route_ws(N, E, k);
     const FfnWs FL = ffn_ws(N, k, E, S, F, act);
     char* fws = ws + RL.bytes;
@@ -2897,7 +2908,9 @@ TileTable ffn_tile_table(int N, int k, int E, int S, int F, int act, int tile_ro
     t.S = S;
     t.tile_rows = tile_rows;
     t.fold = tile_rows == TBM ? tile_fold(N, k, E) : 0;
-    t.light = tile_rows == TBM ? tile_light(N, k, E, t.fold) : 0;
+    t.light = tile_rows == TBM ? tile_light(N, k, E, S, F, wf) : 0;
+    t.light_min = kLightGroups / ceil_div(F, 64);
+    t.light_few = t.light > 0 ? tile_light_few(N, k, E, t.fold) : 0;
     t.ltile_seg = (int*)(fws + FL.lseg);
     t.ltile_row0 = (int*)(fws + FL.lrow0);
     t.lntiles = (int*)(fws + FL.lntiles);
@@ -2911,10 +2924,10 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
     const FfnWs FL = ffn_ws(N, k, E, S, F, act);
     char* fws = ws + RL.bytes;
     void* hbuf = fws + FL.h;
-    const int tile_rows = ffn_tile_rows(act, N, k, E, H, F, w->format);
+    const int tile_rows = ffn_tile_rows(act, N, k, E, S, H, F, w->format);
     const bool tiled = tile_rows == TBM, streaming = tile_rows == 16;
     const bool mid = act == YVMOE_ACT_BF16 && !tiled && !streaming;
-    const TileTable tt = ffn_tile_table(N, k, E, S, F, act, tile_rows, ws);
+    const TileTable tt = ffn_tile_table(N, k, E, S, F, act, w->format, tile_rows, ws);
     int* seg = tt.seg;
     int* tile_seg = tt.tile_seg;
     int* tile_row0 = tt.tile_row0;
@@ -2922,26 +2935,21 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
     const int T = max_tiles(N, k, E, S, tile_rows);
     if (!tiles_ready) {
         build_tiles_kernel<<<1, 512, 0, st>>>(routing->offsets, E, S, N, k, tile_rows, tt.fold, seg,
-                                              tile_seg, tile_row0, ntiles, tt.light, tt.ltile_seg,
-                                              tt.ltile_row0, tt.lntiles);
+                                              tile_seg, tile_row0, ntiles, tt.light, tt.light_min,
+                                              tt.light_few, tt.ltile_seg, tt.ltile_row0, tt.lntiles);
         YV_LAUNCH_CHECK("build_tiles");
     } else if (tt.light > 0) {
         set_error("internal: a light tile table is built by the FFN launch itself");
         return YVMOE_ERR_ARG;
     }
     const int wf = w->format;
-    // the light table's remainders (at most tt.light rows, one per segment) on the streaming
-    // form with tt.light-row tiles, after the main table's launch of the same GEMM; 32-row
-    // tiles with four 16-column blocks per wavefront (a quarter of the activation staging per
-    // weight byte: cfg5 FFN -1.9 % against one block), 64-row tiles with one (1, 2 and 4
-    // blocks measured alike at cfg4)
+    // the light table's remainders (at most tt.light rows, one per segment) on the mid-sized form,
+    // after the main table's launch of the same GEMM
     auto light_launch = [&](GemmParams q, auto epi, const char* name) {
-        constexpr int EPIV = decltype(epi)::value;
         q.tile_seg = tt.ltile_seg;
         q.tile_row0 = tt.ltile_row0;
         q.ntiles = tt.lntiles;
-        if (tt.light > 32) return stream_dispatch<EPIV, 2, 1, 4, true, 4>(wf, q, E + S, st, name);
-        return stream_dispatch<EPIV, 2, 4, 2, true, 4>(wf, q, E + S, st, name);
+        return mid_dispatch<decltype(epi)::value>(wf, q, E + S, 128, st, name);
     };
     GemmParams p{};
     p.tile_seg = tile_seg;

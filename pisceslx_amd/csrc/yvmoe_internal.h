@@ -220,7 +220,7 @@ inline DispatchWs dispatch_ws(int N, int k, int E, int H, int F, int act) {
 // holds tile_rows + remainder rows) instead of taking a tile of its own. With light > 0 a
 // remainder of at most light rows that is not folded takes no tile of the main table but one of
 // the light table (ltile_seg, ltile_row0, lntiles: at most one per segment), which the
-// weight-streaming GEMM form runs with light-row tiles (32 or 64).
+// mid-sized GEMM form runs; with fewer than light_min of them only those of at most light_few.
 struct TileTable {
     int* seg;
     int* tile_seg;
@@ -230,6 +230,7 @@ struct TileTable {
     int tile_rows;
     int fold;
     int light;
+    int light_min, light_few;
     int* ltile_seg;
     int* ltile_row0;
     int* lntiles;
@@ -257,19 +258,35 @@ __host__ __device__ inline int seg_tiles(int rows, int tile_rows, int fold, int 
     return n + ((rem > 0 && !seg_folds(rows, tile_rows, fold) && !seg_light(rows, tile_rows, fold, light)) ? 1 : 0);
 }
 
-// Whether, and up to how many rows, the LDS-tiled expert GEMMs send remainders to the
-// weight-streaming form (light tiles of 32 or 64 rows, the light value): when experts hold few
-// tiles each (a mean under two 256-row tiles). A 256-row tile that holds a few dozen rows still
-// streams and dequantizes the expert's weights through LDS, at about half the cost of a full
-// tile; the streaming form reads them once from HBM with no LDS round trip for the weights.
-// Without folding: remainders of at most 32 rows (cfg5 FFN, one box: 256-row tiles only
-// 7.62-7.65 ms; light tiles of 16, 32, 64 rows 7.45-7.50, 7.19-7.21, 7.37 ms). With folding
-// (remainders of at most kTileFold rows join their last full tile): the remainders of
-// kTileFold + 1 .. 64 rows.
-inline int tile_light(int N, int k, int E, int fold) {
+// Up to how many rows the LDS-tiled expert GEMMs send remainders to the mid-sized form (0: none). A
+// 256-row tile that holds a few dozen rows still streams and dequantizes the expert's weights
+// through LDS, at about half the cost of a full tile; the mid-sized form's cost falls with the
+// rows, and at 96 the two are about even. Measured (FFN, light remainders up to 96 rows against up
+// to 32 or 64 rows on the weight-streaming form below 512 mean rows and none above): fp8 H 7168,
+// 256 experts, skewed, mean 256 / 125 rows 6995 -> 6661 / 4338 -> 4044 us; int8 H 4096, 64 experts,
+// mean 768 / 1567 2316 -> 2194 / 4467 -> 4414. bf16 tiles, which convert nothing, gain below 512
+// rows only (mean 131 / 562: 647 -> 612 / 1823 -> 1896 us). int4, whose mid-sized form has two
+// work-groups per CU instead of three, takes 64 (H 5120, 128 experts, mean 375: 2936 us on 32 rows,
+// 2915 on 64, 2985 on 96).
+// The light launches need about two work-groups per CU (kLightGroups of the gate/up launch's) or
+// they end as a chain over K on a few CUs: with 3 light experts, mean 159 rows, 686 -> 745 us; at
+// H 1024, 8 experts of 256 rows 127 -> 167 us. Layers that cannot have so many have no light table;
+// for the others the tile table's kernel decides from the routing, and where it finds fewer, only
+// remainders short enough to pay for themselves one by one leave the tiles (tile_light_few).
+constexpr int kLightRows = 96, kLightGroups = 512;
+inline int tile_light(int N, int k, int E, int S, int F, int wf) {
     const long long mean = (long long)N * k / (E > 0 ? E : 1);
-    if (mean >= 512) return 0;
-    return fold > 0 ? 64 : 32;
+    if (wf == YVMOE_W_BF16 && mean >= 512) return 0;
+    if ((E + S) * ceil_div(F, 64) < kLightGroups) return 0;
+    return wf == YVMOE_W_INT4 ? 64 : kLightRows;
+}
+
+// Remainders that leave the 256-row tiles however few there are: of up to 32 rows, or beside
+// folding (which takes those) 64, when experts hold under two tiles each. (int4 H 4096, 64 experts,
+// mean 244 / 281 rows: 887 / 976 us against 912 / 996 with every remainder in a tile.)
+inline int tile_light_few(int N, int k, int E, int fold) {
+    const long long mean = (long long)N * k / (E > 0 ? E : 1);
+    return mean >= 512 ? 0 : fold > 0 ? 64 : 32;
 }
 
 // Whether the LDS-tiled expert GEMMs fold remainders: when the mean expert holds one tile and
@@ -329,8 +346,8 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
                        int ld, float* partials, hipStream_t st, bool reduce = true);
 // Rows per tile of the expert GEMMs for this batch and layer, and the tile table's location
 // in the workspace.
-int ffn_tile_rows(int act, int N, int k, int E, int H, int F, int wf);
-TileTable ffn_tile_table(int N, int k, int E, int S, int F, int act, int tile_rows, char* ws);
+int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf);
+TileTable ffn_tile_table(int N, int k, int E, int S, int F, int act, int wf, int tile_rows, char* ws);
 int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_weights* w,
                       const yvmoe_routing* routing, void* y, char* ws, hipStream_t st,
                       bool tiles_ready = false);

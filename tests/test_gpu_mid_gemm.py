@@ -57,3 +57,23 @@ def test_form_boundaries(cuda, oracle, n):
     from pisceslx_amd import _lib
     spec = LayerSpec("midline", 512, 256, 8, 6, 1, _lib.W_INT8, torch.bfloat16)
     _run_and_check(oracle, make_workload(spec, device="cuda", lengths=[n]), label=f"mid line N={n}")
+
+
+@pytest.mark.parametrize("fmt,light", [("int8", 64), ("int8", 63), ("int4", 64), ("fp8", 64), ("bf16", 64)])
+def test_light_remainders_of_many_experts(cuda, oracle, fmt, light):
+    """Prefill-sized skewed batches of many experts: remainders of 1 .. 96 rows leave the 256-row
+    tiles for the mid-sized form when there are enough of them (64 at ffn 512; the tile table's
+    kernel decides), whole experts and tails after full tiles alike; 97 rows keep a tile. (int4
+    takes up to 64 rows, so here too few and only those of up to 32.)"""
+    from pisceslx_amd import _lib
+    counts = [1 + (e * 37) % 96 for e in range(light - 8)] + [256 + 96, 512 + 1] * 4
+    counts += [97, 0, 256, 700, 3 * 256 + 200] * 5
+    counts.append((128 - sum(counts)) % 256 + 512)  # the shared segment ends in 128 rows: not light
+    counts[-1] += 97 if 0 < counts[-1] % 256 <= 96 else 0
+    assert sum(0 < c % 256 <= 96 for c in counts) == light and not 0 < sum(counts) % 256 <= 96
+    assert sum(counts) >= 150 * len(counts)         # the rule's line for the 256-row form
+    spec = LayerSpec("manylight", 256, 512, len(counts), 1, 1, getattr(_lib, "W_" + fmt.upper()),
+                     torch.bfloat16, fixed_shape_mode=True)
+    w = forced_rows(spec, counts)
+    _, _, routing = _run_and_check(oracle, w, label=f"many light {fmt} N={sum(counts)} E={len(counts)}")
+    assert routing.counts.cpu().tolist() == counts
