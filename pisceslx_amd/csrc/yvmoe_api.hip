@@ -309,7 +309,7 @@ int32_t yvmoe_forward(const void* x, int32_t act_dtype, int32_t n_tokens,
     const int S = experts->num_shared;
     TileTable tiles{};
     if (small)
-        tiles = ffn_tile_table(N, k, E, S, experts->ffn, act_dtype, experts->format,
+        tiles = ffn_tile_table(N, k, E, S, experts->hidden, experts->ffn, act_dtype, experts->format,
                                ffn_tile_rows(act_dtype, N, k, E, S, experts->hidden, experts->ffn,
                                              experts->format),
                                ws);
@@ -557,7 +557,7 @@ int32_t yvmoe_forward_moegate(const void* x, int32_t act_dtype, int32_t n_tokens
     r.fixed_shape_mode = 1;
     TileTable tiles{};
     if (small)
-        tiles = ffn_tile_table(N, k, E, S, experts->ffn, act_dtype, experts->format,
+        tiles = ffn_tile_table(N, k, E, S, experts->hidden, experts->ffn, act_dtype, experts->format,
                                ffn_tile_rows(act_dtype, N, k, E, S, experts->hidden, experts->ffn,
                                              experts->format),
                                ws);

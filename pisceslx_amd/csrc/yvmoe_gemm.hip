@@ -851,9 +851,15 @@ static_assert(kTileFold * TBK * 2 == 256 * (TTHREADS / 64), "one dword load per 
 // rows. Such a launch holds two copies of the tile loop and each work-group runs the one its
 // tile needs: the copy without folded rows keeps the register use and schedule of a plain
 // tile. Launches without folding (FOLD = false) carry only that copy.
-template <int WF, int EPI, int S4K = 8192, bool FOLD = false, int NW = 16>
+// RAG: the last column block may end early, at ncols (a multiple of 64; fp32 output: of 16): its
+// wavefronts past the end load the last columns again, multiply and store nothing. A form of its
+// own, so that whole column blocks keep their registers. Measured (64 experts, 6 + 2 per token,
+// 8,000 tokens; FFN, against 64-row tiles without LDS): int8 H 3008, ffn 1344 3999 -> 1582 us; bf16 H
+// 2880, ffn 1152 3827 -> 1274; int4 H 2944 3662 -> 1393 (on the mid-sized form 1790, 2152 and 1572).
+template <int WF, int EPI, int S4K = 8192, bool FOLD = false, int NW = 16, bool RAG = EPI == EPI_F32>
 __global__ __launch_bounds__(64 * NW) void gemm_tile_kernel(GemmParams p, int ncb) {
     typedef TileCfg<WF, S4K, FOLD, NW> C;
+    static_assert(!RAG || !FOLD, "partial column blocks without folded rows only");
     constexpr int MBW = C::MBW;
     constexpr bool SWIGLU = EPI == EPI_SWIGLU;
     constexpr bool WFIRST = WF != YVMOE_W_BF16;  // weights as the MFMA's first operand
@@ -935,9 +941,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_tile_kernel(GemmParams p, int nc
             const int r16 = rb * 16;
             const void* B = (SWIGLU && r16 >= TBN / 2) ? p.B1 : p.B0;
             int nb16 = SWIGLU ? n0 + (r16 & (TBN / 2 - 1)) : n0 + r16;
-            // fp32 output: blocks past ncols load the last block (their wavefront skips its
-            // MFMAs and stores nothing)
-            if (EPI == EPI_F32 && nb16 >= p.ncols) nb16 = p.ncols - 16;
+            // blocks past ncols load the last block (their wavefront skips its MFMAs and stores
+            // nothing)
+            if (RAG && nb16 >= p.ncols) nb16 = p.ncols - 16;
             const long long e_bytes = C::I4 ? e_off / 2 : e_off * C::EB;
             b_src[j] = (const char*)B + e_bytes + (long long)(nb16 >> 4) * (p.K / 64) * B_CHUNK +
                        (long long)(kbeg / TBK) * B_CHUNK +
@@ -974,7 +980,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_tile_kernel(GemmParams p, int nc
             for (int nb = 0; nb < 2; ++nb) {
                 const int r = brow[nb];
                 const void* S = (SWIGLU && r >= TBN / 2) ? p.S1 : p.S0;
-                cs[nb] = b_scale<WF>(S, s_off, SWIGLU ? n0 + (r & (TBN / 2 - 1)) : n0 + r, p.K, 0);
+                const int n = SWIGLU ? n0 + (r & (TBN / 2 - 1)) : n0 + r;
+                cs[nb] = b_scale<WF>(S, s_off, RAG ? min(n, p.ncols - 1) : n, p.K, 0);
             }
         }
         if constexpr (C::I4) {
@@ -983,7 +990,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_tile_kernel(GemmParams p, int nc
             for (int i = t; i < TBN * kg; i += 64 * NW) {
                 const int r = i / kg, q = i % kg;
                 const void* S = (SWIGLU && r >= TBN / 2) ? p.S1 : p.S0;
-                const int n = SWIGLU ? n0 + (r & (TBN / 2 - 1)) : n0 + r;
+                int n = SWIGLU ? n0 + (r & (TBN / 2 - 1)) : n0 + r;
+                if (RAG) n = min(n, p.ncols - 1);
                 lds_s4[i] = ((const unsigned short*)S)[s_off + (long long)n * kg + q];
             }
             __syncthreads();
@@ -993,7 +1001,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_tile_kernel(GemmParams p, int nc
             if (t < 2 * kb) {
                 const int b = t / kb, q = t % kb;
                 const void* S = (SWIGLU && b == 1) ? p.S1 : p.S0;
-                const int n = SWIGLU ? n0 : n0 + b * 128;
+                int n = SWIGLU ? n0 : n0 + b * 128;
+                if (RAG) n = min(n, p.ncols - 1);
                 lds_s[b][q] = b_scale<WF>(S, s_off, n, p.K, q * 128);
             }
 #pragma unroll
@@ -1032,9 +1041,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_tile_kernel(GemmParams p, int nc
         // 16-row blocks of this wavefront's 128 rows that hold rows of the segment: an expert's
         // last tile skips the MFMAs of the blocks past its end (loads and barriers stay uniform)
         const int live_mb = min(MBW, max(0, (seg_end - (row0 + wr * MBW * 16) + 15) / 16));
-        // fp32 output: a wavefront whose 32 columns lie past ncols skips every MFMA (a separate
-        // flag: folding it into live_mb made the compiler spill 59 VGPRs of this kernel)
-        const bool colive = EPI != EPI_F32 || n0 + wc * 32 < p.ncols;
+        // a wavefront whose columns lie past ncols skips every MFMA (a separate flag: folding it
+        // into live_mb made the compiler spill 59 VGPRs of this kernel)
+        const bool colive = !RAG || n0 + wc * (SWIGLU ? 16 : 32) < p.ncols;
         // folded rows: wavefront row wr computes row block 256 + 16 wr .. + 15 when it holds rows
         const bool xlive = XT && ext > 16 * wr;
         f32x4 accx[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
@@ -1208,6 +1217,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_tile_kernel(GemmParams p, int nc
         // stores), down 8 (16-byte stores)
         // one 16-row block at row rb: WFIRST, lane row rb + l % 16; else rows rb + 4 (l / 16) + i
         auto store_block = [&](int rb, f32x4 c0, f32x4 c1) {
+            if (RAG && EPI != EPI_F32 && !colive) return;
             if constexpr (!WFIRST) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -2658,12 +2668,17 @@ int tile_dispatch(int wf, const GemmParams& p, int ntiles_max, hipStream_t st, c
 template <int EPI, bool FOLD>
 int tile_launch(int wf, const GemmParams& p, int ntiles_max, hipStream_t st, const char* name) {
     const int cols = (EPI == EPI_SWIGLU) ? TBN / 2 : TBN;
-    // the fp32-output form takes any multiple of 16 columns (a partial last column block) and
-    // K splits of kchunk (a multiple of 64; the last split may be shorter)
-    const int cmul = EPI == EPI_F32 ? 16 : cols;
+    // a partial last column block: any multiple of 64 columns without folded rows; the fp32-output
+    // form takes any multiple of 16 and K splits of kchunk (a multiple of 64; the last may be shorter)
+    const int cmul = EPI == EPI_F32 ? 16 : FOLD ? cols : 64;
+    const bool rag = !FOLD && p.ncols % cols != 0;
     if (p.ncols % cmul != 0 || p.K % TBK != 0 || (EPI == EPI_F32 && (p.kchunk <= 0 || p.kchunk % TBK != 0))) {
         set_error("%s: tiled form needs columns %% %d == 0 and K %% %d == 0 (K=%d, kchunk=%d)", name,
                   cmul, TBK, p.K, p.kchunk);
+        return YVMOE_ERR_SHAPE;
+    }
+    if (wf == YVMOE_W_INT4 && p.K > 8192) {  // the group-scale table in LDS holds K / 128 <= 64 groups
+        set_error("%s: tiled int4 form needs K <= 8192 (K=%d)", name, p.K);
         return YVMOE_ERR_SHAPE;
     }
     if (ntiles_max <= 0) return YVMOE_OK;
@@ -2683,6 +2698,18 @@ int tile_launch(int wf, const GemmParams& p, int ntiles_max, hipStream_t st, con
             gemm_wide_kernel<<<(unsigned)blocks, 256, 0, st>>>(p, ncb);
         else
             gemm_tile_kernel<YVMOE_W_BF16, EPI><<<(unsigned)blocks, TTHREADS, 0, st>>>(p, ncb);
+    } else if (rag) {
+        if constexpr (!FOLD) {
+#define YV_RAG(WFV) gemm_tile_kernel<WFV, EPI, 8192, false, 16, true><<<(unsigned)blocks, TTHREADS, 0, st>>>(p, ncb)
+            switch (wf) {
+                case YVMOE_W_BF16: YV_RAG(YVMOE_W_BF16); break;
+                case YVMOE_W_INT8: YV_RAG(YVMOE_W_INT8); break;
+                case YVMOE_W_FP8: YV_RAG(YVMOE_W_FP8); break;
+                case YVMOE_W_INT4: YV_RAG(YVMOE_W_INT4); break;
+                default: set_error("%s: no tiled form for weight format %d", name, wf); return YVMOE_ERR_DTYPE;
+            }
+#undef YV_RAG
+        }
     } else {
         switch (wf) {
             case YVMOE_W_BF16: gemm_tile_kernel<YVMOE_W_BF16, EPI, 8192, FOLD><<<(unsigned)blocks, TTHREADS, 0, st>>>(p, ncb); break;
@@ -2708,10 +2735,6 @@ int tile_launch(int wf, const GemmParams& p, int ntiles_max, hipStream_t st, con
                 gemm_tile_kernel<YVMOE_W_FP8, EPI, 8192, FOLD><<<(unsigned)blocks, TTHREADS, 0, st>>>(p, ncb);
                 break;
             case YVMOE_W_INT4:
-                if (p.K > 8192) {  // the group-scale table in LDS holds K / 128 <= 64 groups
-                    set_error("%s: tiled int4 form needs K <= 8192 (K=%d)", name, p.K);
-                    return YVMOE_ERR_SHAPE;
-                }
                 if constexpr (FOLD) {
                     if (p.K <= 5120)  // 40 scale groups beside a 3-stage ring
                         gemm_tile_kernel<YVMOE_W_INT4, EPI, 5120, true><<<(unsigned)blocks, TTHREADS, 0, st>>>(p, ncb);
@@ -2875,28 +2898,27 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
 //   against 246), and any format up to 48 rows when 128-row tiles would leave the down
 //   projection under two work-groups per CU (H 1024, 8 experts of 16 / 32 rows: 48.5 / 48.7 us
 //   against 48.2 / 58.3).
-// * 128: the mid form, up to 150 rows for int8 and int4 and 112 for fp8 and bf16, from where an
+// * 128: the mid form, up to 150 rows for int8 and int4, 125 for fp8 and 112 for bf16, from where an
 //   expert's rows past 128 cost a second pass over its weights (H 4096, 64 experts, 96 / 131 /
 //   159 rows: int8 386 / 546 / 690 us against 576 / 601 / 686 on 256-row tiles, bf16 546 / 817 /
 //   1038 against 646 / 653 / 680; fp8 H 7168, 256 experts, 94 / 128 rows 2864 / 4203 against 3309 /
-//   3823); any number of rows where the 256-row form does not take
-//   the shape; and where 256-row tiles would be under two work-groups per CU (H 1024, 8 experts, 256
+//   3823, H 2944, 64 experts, 122 rows 305 against 389); any number of rows where the 256-row form's scale tables
+//   (fp8, int4: 8192 of K) do not hold the shape; and where 256-row tiles would be under two work-groups per CU (H 1024, 8 experts, 256
 //   / 375 rows: bf16 100 / 150 us against 127 / 134, int8 95 / 130 against 138 / 141).
 // * 256: the LDS-tiled form above that.
 int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf) {
     const long long slots = (long long)N * k;
     if (act != YVMOE_ACT_BF16) return slots < 48LL * E ? kTileRows : 128;
     if (slots < (wf == YVMOE_W_INT4 ? 4LL : 8LL) * E) return 16;
-    const bool tiles = F % (TBN / 2) == 0 && H % TBN == 0 &&
-                       (wf == YVMOE_W_INT8 || wf == YVMOE_W_BF16 || (H <= 8192 && F <= 8192));
-    const long long most = wf == YVMOE_W_INT8 || wf == YVMOE_W_INT4 ? 150 : 112;
+    const bool tiles = wf == YVMOE_W_INT8 || wf == YVMOE_W_BF16 || (H <= 8192 && F <= 8192);
+    const long long most = wf == YVMOE_W_INT8 || wf == YVMOE_W_INT4 ? 150 : wf == YVMOE_W_FP8 ? 125 : 112;
     const long long items = (long long)max_tiles(N, k, E, S, TBM) * ceil_div(F, TBN / 2);
     if (tiles && slots >= most * E && items > 448) return TBM;
     if (slots <= 48LL * E && (wf == YVMOE_W_INT4 || (long long)E * ceil_div(H, 128) < 512)) return 64;
     return 128;
 }
 
-TileTable ffn_tile_table(int N, int k, int E, int S, int F, int act, int wf, int tile_rows, char* ws) {
+TileTable ffn_tile_table(int N, int k, int E, int S, int H, int F, int act, int wf, int tile_rows, char* ws) {
     const RouteWs RL = route_ws(N, E, k);
     const FfnWs FL = ffn_ws(N, k, E, S, F, act);
     char* fws = ws + RL.bytes;
@@ -2907,7 +2929,8 @@ TileTable ffn_tile_table(int N, int k, int E, int S, int F, int act, int wf, int
     t.ntiles = (int*)(fws + FL.ntiles);
     t.S = S;
     t.tile_rows = tile_rows;
-    t.fold = tile_rows == TBM ? tile_fold(N, k, E) : 0;
+    // folded rows and partial column blocks do not meet in one kernel
+    t.fold = tile_rows == TBM && F % (TBN / 2) == 0 && H % TBN == 0 ? tile_fold(N, k, E) : 0;
     t.light = tile_rows == TBM ? tile_light(N, k, E, S, F, wf) : 0;
     t.light_min = kLightGroups / ceil_div(F, 64);
     t.light_few = t.light > 0 ? tile_light_few(N, k, E, t.fold) : 0;
@@ -2927,7 +2950,7 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
     const int tile_rows = ffn_tile_rows(act, N, k, E, S, H, F, w->format);
     const bool tiled = tile_rows == TBM, streaming = tile_rows == 16;
     const bool mid = act == YVMOE_ACT_BF16 && !tiled && !streaming;
-    const TileTable tt = ffn_tile_table(N, k, E, S, F, act, w->format, tile_rows, ws);
+    const TileTable tt = ffn_tile_table(N, k, E, S, H, F, act, w->format, tile_rows, ws);
     int* seg = tt.seg;
     int* tile_seg = tt.tile_seg;
     int* tile_row0 = tt.tile_row0;

@@ -77,3 +77,23 @@ def test_light_remainders_of_many_experts(cuda, oracle, fmt, light):
     w = forced_rows(spec, counts)
     _, _, routing = _run_and_check(oracle, w, label=f"many light {fmt} N={sum(counts)} E={len(counts)}")
     assert routing.counts.cpu().tolist() == counts
+
+
+# a mean of 283 rows per expert on grids large enough for the 256-row form; each list entry is six
+# experts: remainders of none, 1 .. 32 (folded), 33 .. 96, more, and an expert under one tile
+MANY = [256, 257, 272, 273, 288, 289, 320, 321, 544, 16] * 6
+
+
+@pytest.mark.parametrize("fmt,hidden,ffn", [
+    ("int8", 256, 512), ("int4", 256, 512), ("fp8", 256, 512), ("bf16", 256, 512),  # folded rows
+    ("int8", 320, 448), ("bf16", 320, 448),   # partial column blocks (64 of 128, 64 of 256): no folding
+    ("int8", 64, 576), ("bf16", 448, 512),    # one k-step; gate/up whole, down partial
+    ("int4", 384, 640), ("fp8", 384, 640),    # down partial (128 of 256)
+])
+def test_tiled_forms(cuda, oracle, fmt, hidden, ffn):
+    from pisceslx_amd import _lib
+    spec = LayerSpec("tiled", hidden, ffn, len(MANY), 1, 1, getattr(_lib, "W_" + fmt.upper()),
+                     torch.bfloat16, fixed_shape_mode=True)
+    w = forced_rows(spec, MANY)
+    _, _, routing = _run_and_check(oracle, w, label=f"tiled {fmt} H={hidden} F={ffn} N={sum(MANY)}")
+    assert routing.counts.cpu().tolist() == MANY
