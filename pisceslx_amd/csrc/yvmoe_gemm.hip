@@ -1712,7 +1712,7 @@ struct MidCfg {
 };
 
 // One tile (rows row0 .. seg_end - 1, at most 16 * MRB) against column group cgroup.
-template <int WF, int EPI, int MRB, int MAXMRB>
+template <int WF, int EPI, int MRB, int MAXMRB, bool NT>
 __device__ __forceinline__ void mid_item(const GemmParams& p, int e, int row0, int seg_end, int cgroup,
                                          unsigned char (&lds_a)[3][MAXMRB * 2048], unsigned char* lds_s) {
     typedef BLoad<WF> BL;
@@ -1784,7 +1784,10 @@ __device__ __forceinline__ void mid_item(const GemmParams& p, int e, int row0, i
         // so every wait below has a fixed count
         auto load_w = [&](int c, typename BL::Raw (&dst)[2]) {
 #pragma unroll
-            for (int nb = 0; nb < 2; ++nb) BL::load_blk_nt(dst[nb], bptr[nb], kb + min(c, n - 1));
+            for (int nb = 0; nb < 2; ++nb) {
+                if constexpr (NT) BL::load_blk_nt(dst[nb], bptr[nb], kb + min(c, n - 1));
+                else BL::load_blk(dst[nb], bptr[nb], kb + min(c, n - 1));
+            }
         };
         auto issue_a = [&](int c, int st) {
             const size_t off = (size_t)(kb + min(c, n - 1)) * 128;
@@ -1863,6 +1866,17 @@ __device__ __forceinline__ void mid_item(const GemmParams& p, int e, int row0, i
     for (int mb = 0; mb < MRB; ++mb) {
         const int r = row0 + mb * 16 + i16;
         if (r >= seg_end) continue;
+        if constexpr (EPI == EPI_F32) {
+            float* o = (float*)p.out + (long long)r * p.ldo + n0 + 4 * g;
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                f32x4 v;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = f32_out(p, acc[mb][nb][i], n0 + nb * 16 + 4 * g + i, 0);
+                *(f32x4*)(o + nb * 16) = v;
+            }
+            continue;
+        }
         unsigned short* o = (unsigned short*)p.out + (long long)r * p.ldo + n0 + 4 * g;
         if constexpr (SWIGLU) {
             float hv[4];
@@ -1882,6 +1896,9 @@ __device__ __forceinline__ void mid_item(const GemmParams& p, int e, int row0, i
     }
 }
 
+// Also the dense fp32-output GEMM of mid-sized batches (EPI_F32, bf16 weights: the YvMoEGate
+// projection), where 256-row tiles would leave half of the CUs without a work-group.
+//
 // Column groups per XCD and tile: consecutive work-group ids go to different XCDs, and XCD x
 // takes the groups x - e (mod 8) of every tile of expert e. Each XCD then sees every tile (an
 // even load, although the shared experts' tiles are the fullest and stand last in the table), the
@@ -1889,25 +1906,28 @@ __device__ __forceinline__ void mid_item(const GemmParams& p, int e, int row0, i
 // run together on the tile's rows. Tiles run last to first, so the full ones do not end the
 // launch. (FFN at 64 experts of 47 rows: contiguous ranges of the items per XCD 348 us tile by
 // tile, 309 us group by group; 288 us in this order.)
-template <int WF, int EPI, int MAXMRB>
+// NT: non-temporal weight loads, where (nearly) every weight is read by one tile only.
+template <int WF, int EPI, int MAXMRB, bool NT = true>
 __global__ __launch_bounds__(256, (MAXMRB == 8 ? 3 : 4) - (WF == YVMOE_W_INT4 ? 1 : 0)) void gemm_mid_kernel(GemmParams p, int ngroups) {
     __shared__ __attribute__((aligned(1024))) unsigned char lds_a[3][MAXMRB * 2048];
     __shared__ __attribute__((aligned(16))) unsigned char lds_s[MidCfg<WF>::S_BYTES];
     const int local = blockIdx.x / 8, x = blockIdx.x % 8;
     const int per_tile = (ngroups + 7) / 8;
-    const int tile = *p.ntiles - 1 - local / per_tile;
+    const int nt = EPI == EPI_F32 ? (p.nrows + MAXMRB * 16 - 1) / (MAXMRB * 16) : *p.ntiles;
+    const int tile = nt - 1 - local / per_tile;  // dense fp32 output: one segment of nrows rows
     if (tile < 0) return;
-    const int e = p.tile_seg[tile], row0 = p.tile_row0[tile];
+    const int e = EPI == EPI_F32 ? 0 : p.tile_seg[tile];
+    const int row0 = EPI == EPI_F32 ? tile * MAXMRB * 16 : p.tile_row0[tile];
     const int cgroup = ((x + e) & 7) + 8 * (local % per_tile);
     if (cgroup >= ngroups) return;
-    const int seg_end = min(p.seg_start[e + 1], row0 + MAXMRB * 16);
+    const int seg_end = min(EPI == EPI_F32 ? p.nrows : p.seg_start[e + 1], row0 + MAXMRB * 16);
     const int rows = seg_end - row0;
     if constexpr (MAXMRB == 8) {
-        if (rows > 96) return mid_item<WF, EPI, 8, MAXMRB>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
-        if (rows > 64) return mid_item<WF, EPI, 6, MAXMRB>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
+        if (rows > 96) return mid_item<WF, EPI, 8, MAXMRB, NT>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
+        if (rows > 64) return mid_item<WF, EPI, 6, MAXMRB, NT>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
     }
-    if (rows > 32) return mid_item<WF, EPI, 4, MAXMRB>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
-    mid_item<WF, EPI, 2, MAXMRB>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
+    if (rows > 32) return mid_item<WF, EPI, 4, MAXMRB, NT>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
+    mid_item<WF, EPI, 2, MAXMRB, NT>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
 }
 
 // ------------------------------------------------------------------ fp32, dense
@@ -2774,38 +2794,6 @@ int gemm_dispatch(int act, GemmParams p, int ntiles, int ncb, int ksplit, hipStr
 
 }  // namespace
 
-int dense_gemm_launch(const void* x, int act, int N, int K, const void* w, int ncols, float* out,
-                      int ld, float* partials, hipStream_t st, const char* name) {
-    if (N <= 0) return YVMOE_OK;
-    GemmParams p{};
-    p.A = x;
-    p.lda = K;
-    p.rowmap = nullptr;
-    p.B0 = w;
-    p.K = K;
-    p.ncols = ncols;
-    p.ldo = ld;
-    p.nrows = N;
-    if (dense_tiled(act, N, ncols, K)) {
-        p.kchunk = K;
-        p.out = out;
-        return tile_dispatch<EPI_F32>(YVMOE_W_BF16, p, ceil_div(N, TBM), st, name);
-    }
-    const int ks = dense_ksplit(N, ncols, K);
-    const int ncb = (ncols % 32 == 0) ? 2 : 1;
-    if (ks == 1 || partials == nullptr) {
-        p.kchunk = K;
-        p.out = out;
-        return gemm_dispatch(act, p, ceil_div(N, kTileRows), ncb, 1, st, name);
-    }
-    p.kchunk = K / ks;
-    p.out = partials;
-    p.split_stride = (long long)N * ld;
-    int rc = gemm_dispatch(act, p, ceil_div(N, kTileRows), ncb, ks, st, name);
-    if (rc) return rc;
-    return reduce_splits_launch(partials, ks, (long long)N * ld, out, st, "dense_gemm_reduce");
-}
-
 int dense_partials_launch(const void* x, int act, int N, int K, const void* w, int ncols,
                           float* out, int ld, const float* col_bias, int col_bias_n,
                           hipStream_t st, const char* name) {
@@ -2825,7 +2813,22 @@ int dense_partials_launch(const void* x, int act, int N, int K, const void* w, i
     p.split_stride = (long long)N * ld;
     const int ks = dense_splits(act, N, ncols, K);
     p.kchunk = K / ks;
-    if (dense_tiled(act, N, ncols, K)) return tile_dispatch<EPI_F32>(YVMOE_W_BF16, p, ceil_div(N, TBM), st, name);
+    if (dense_tiled(act, N, ncols, K)) {
+        // up to 144 256 x 256 tiles, the mid-sized form: more work-groups in flight on the weights
+        // (whole gate call, H 4096, 16,896 columns: 100 / 256 / 450 tokens 120 / 143 / 162 us on
+        // 256-row tiles, 72 / 97 / 146; 700 tokens, 198 tiles: 179 and 247; H 2048, 700 tokens, 99
+        // tiles: 117 and 99). Non-temporal weight loads for a single row tile (100 tokens 79 -> 72 us;
+        // 300 tokens 122 -> 135).
+        if (ceil_div(N, TBM) * (ncols / TBN) <= 144) {
+            const int ngroups = ncols / 128;
+            const unsigned items = 8u * ceil_div(N, 128) * ceil_div(ngroups, 8);
+            if (N <= 128) gemm_mid_kernel<YVMOE_W_BF16, EPI_F32, 8><<<items, 256, 0, st>>>(p, ngroups);
+            else gemm_mid_kernel<YVMOE_W_BF16, EPI_F32, 8, false><<<items, 256, 0, st>>>(p, ngroups);
+            YV_LAUNCH_CHECK(name);
+            return YVMOE_OK;
+        }
+        return tile_dispatch<EPI_F32>(YVMOE_W_BF16, p, ceil_div(N, TBM), st, name);
+    }
     if (dense_streamed(act, N, ncols, K)) {
         if (N <= 16) return stream_dispatch<EPI_F32, 4, 1, 1>(YVMOE_W_BF16, p, 1, st, name, ks);
         // one k-step per staged chunk with the next chunk's weights in flight: the YvMoEGate

@@ -351,11 +351,8 @@ TileTable ffn_tile_table(int N, int k, int E, int S, int H, int F, int act, int 
 int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_weights* w,
                       const yvmoe_routing* routing, void* y, char* ws, hipStream_t st,
                       bool tiles_ready = false);
-// out[N][ld] (fp32) = x[N][K] · wᵀ, w [ncols][K] in the activation dtype; split-K partial
-// sums (when the rule splits) go to partials and are reduced in split order.
-int dense_gemm_launch(const void* x, int act, int N, int K, const void* w, int ncols, float* out,
-                      int ld, float* partials, hipStream_t st, const char* name);
-// The same product left as dense_splits(act, N, ncols, K) partial sums: split z at
+// out[N][ld] (fp32) = x[N][K] · wᵀ, w [ncols][K] in the activation dtype, left as
+// dense_splits(act, N, ncols, K) partial sums: split z at
 // out + z * N * ld (its K range z * K / splits ...), for the consumer to sum in split order;
 // split 0 also adds col_bias[n] to columns n < col_bias_n (col_bias may be NULL).
 int dense_partials_launch(const void* x, int act, int N, int K, const void* w, int ncols,

@@ -4,7 +4,7 @@
 // yvmoe_route (softmax, top-k, softmax of the k scores).
 //
 // Kernels:
-//   moegate_proj (dense_gemm_launch): fp32 [N][P] = x · W_projᵀ, W_proj = [dg_proj
+//   moegate_proj (dense_partials_launch): fp32 [N][P] = x · W_projᵀ, W_proj = [dg_proj
 //     (hicl_router.py:77); gate; got_cluster_proj; gate_k; gate_v; input_encoder.0; zero
 //     rows] — the LDS-tiled MFMA form for batches above 64 rows, the streaming form below.
 //   moegate_token_kernel: per token — relu(dg + dg_bias), the sel_k largest kept (radix select

@@ -79,6 +79,15 @@ def test_moegate_matches_oracle(cuda, oracle, B, S, H, E, k, scale):
     _check(g, x, oracle)
 
 
+@pytest.mark.parametrize("n", [65, 96, 97, 128, 129, 300])
+def test_projection_of_mid_sized_batches(cuda, oracle, n):
+    """Batches above the streaming form whose 256-row tiles would not fill the chip: the mid-sized
+    form's row-block variants, one and several row tiles (cached and non-temporal weights)."""
+    g = _gate(512, 48, 6, scale_heads=True, seed=n)
+    x = torch.randn(n, 1, 512, generator=torch.Generator().manual_seed(n)).to(torch.bfloat16).cuda()
+    _check(g, x, oracle)
+
+
 def test_dg_ties_and_few_positives(cuda, oracle):
     H, E = 256, 8
     g = _gate(H, E, 2, scale_heads=True, seed=1)
