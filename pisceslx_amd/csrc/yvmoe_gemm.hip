@@ -763,6 +763,130 @@ __global__ __launch_bounds__(64 * WV) void gemm_stream_kernel(GemmParams p, int 
                                                *reinterpret_cast<uint4(*)[2][16 * MAXRB * (U * 8 + 1)]>(As_raw));
 }
 
+// ------------------------------------------------------------------ bf16, a few tokens
+// Expert GEMM for batches of so few tokens that the weight-streaming form has a work-group or two
+// per CU: a tile of up to 16 rows of one expert against 16 h columns (gate/up) or 32 output
+// columns (down).
+//
+// What bounds it: the serial chain over K, since the few experts' weights leave few work-groups
+// to stream them. Half the columns per work-group and K dealt out to its four wavefronts in chunks
+// of four k-steps give twice the work-groups and a chain of a quarter of K; a wavefront has its
+// next chunk's weights and activations in flight during the current one (no LDS before the end, so
+// no barrier in the loop). The four partial sums meet in LDS in wavefront order.
+// Measured (FFN, against the weight-streaming form): H 4096, 64 experts of 1408, 6 + 2 per token, 1
+// token int8 48 -> 34 us, int4 56 -> 33, fp8 49 -> 32, bf16 58 -> 48; H 1024, 8 experts of 2816, 16
+// tokens int8 43 -> 28 us.
+template <int WF, int EPI>
+__global__ __launch_bounds__(256, 2) void gemm_few_kernel(GemmParams p, int ngroups) {
+    typedef BLoad<WF> BL;
+    constexpr bool SWIGLU = EPI == EPI_SWIGLU;
+    constexpr bool GROUPED = WF == YVMOE_W_INT4 || WF == YVMOE_W_FP8;
+    constexpr int U = WF == YVMOE_W_BF16 ? 2 : 4;  // k-steps per chunk
+    __shared__ f32x4 red[4][2][64];
+    // the mid-sized form's order of tiles and column groups over the XCDs
+    const int local = blockIdx.x / 8, x = blockIdx.x % 8;
+    const int per_tile = (ngroups + 7) / 8;
+    const int tile = *p.ntiles - 1 - local / per_tile;
+    if (tile < 0) return;
+    const int e = p.tile_seg[tile], row0 = p.tile_row0[tile];
+    const int cgroup = ((x + e) & 7) + 8 * (local % per_tile);
+    if (cgroup >= ngroups) return;
+    const int seg_end = min(p.seg_start[e + 1], row0 + 16);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 4, i16 = lane & 15;
+    const long long e_off = (long long)e * p.b_stride;
+    const long long s_off = (long long)e * p.s_stride;
+    const int n0 = cgroup * (SWIGLU ? 16 : 32);
+    const void* S[2] = {p.S0, SWIGLU ? p.S1 : p.S0};
+    const char* bptr[2];
+    int n[2];
+    float cs[2];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+        n[nb] = SWIGLU ? n0 + i16 : n0 + nb * 16 + i16;
+        bptr[nb] = BL::bptr(SWIGLU && nb ? p.B1 : p.B0, e_off, n[nb], p.K, 0, lane);
+        cs[nb] = GROUPED ? 1.0f : b_scale<WF>(S[nb], s_off, n[nb], p.K, 0);
+    }
+    const int r = row0 + i16;
+    const char* arow = (const char*)p.A + ((long long)map_row(p, r < seg_end ? r : row0) * p.lda + g * 16) * 2;
+    const int nks = p.K / 64, nch = (nks + U - 1) / U;
+
+    struct Chunk {
+        typename BL::Raw w[U][2];
+        float s[GROUPED ? U / 2 : 1][2];  // a scale group is two k-steps, and chunks start even
+        Frag16 a[U];
+    };
+    auto load = [&](int c, Chunk& q) {  // k-steps past the end: the last one again, not used
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int ks = min(c * U + u, nks - 1);
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                BL::load_blk_nt(q.w[u][nb], bptr[nb], ks);
+                if constexpr (GROUPED)
+                    if (u % 2 == 0) q.s[u / 2][nb] = b_scale<WF>(S[nb], s_off, n[nb], p.K, ks * 64);
+            }
+            const uint4* ap = (const uint4*)(arow + (size_t)ks * 128);
+            q.a[u].u[0] = ap[0];
+            q.a[u].u[1] = ap[1];
+        }
+    };
+    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    auto mma = [&](int c, const Chunk& q) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (c * U + u < nks) {
+#pragma unroll
+                for (int nb = 0; nb < 2; ++nb) {
+                    Frag16 b;
+                    BL::cvt(q.w[u][nb], GROUPED ? q.s[u / 2][nb] : cs[nb], b);
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b.v[0], q.a[u].v[0], acc[nb], 0, 0, 0);
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b.v[1], q.a[u].v[1], acc[nb], 0, 0, 0);
+                }
+            }
+        }
+    };
+    Chunk q0, q1;
+    int c = wave;
+    if (c < nch) load(c, q0);
+    for (; c + 4 < nch; c += 8) {
+        load(c + 4, q1);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(c, q0);
+        load(min(c + 8, nch - 1), q0);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(c + 4, q1);
+    }
+    if (c < nch) mma(c, q0);
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) red[wave][nb][lane] = acc[nb];
+    __syncthreads();
+    if (wave >= (SWIGLU ? 1 : 2)) return;
+    // gate/up: wavefront 0 both sums; down: wavefront nb the sum of fragment nb. Weights are the
+    // first operand: a lane holds row i16 and 4 consecutive columns
+    f32x4 sum[2];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+        sum[nb] = red[0][nb][lane];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) {
+            const f32x4 v = red[w][nb][lane];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum[nb][i] = sum[nb][i] + v[i];
+        }
+    }
+    if (r >= seg_end) return;
+    float o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if constexpr (SWIGLU) o[i] = round_bf16(silu(round_bf16(sum[0][i]))) * round_bf16(sum[1][i]);
+        else o[i] = wave ? sum[1][i] : sum[0][i];
+    }
+    *(uint2*)((unsigned short*)p.out + (long long)r * p.ldo + n0 + (SWIGLU ? 0 : wave * 16) + 4 * g) =
+        make_uint2(pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3]));
+}
+
 // ------------------------------------------------------------------ bf16, LDS-tiled form
 // Tiled form for batches whose experts hold many rows (prefill). A work-group of 16
 // wavefronts computes a 256-row x 256-column output tile over K in 64-wide chunks.
@@ -2646,6 +2770,25 @@ int f32x3_dispatch(const GemmParams& p, int ntiles_max, hipStream_t st, const ch
     return YVMOE_OK;
 }
 
+// A few tokens: 16-row tiles of the tile table.
+template <int EPI>
+int few_dispatch(int wf, const GemmParams& p, int ntiles_max, hipStream_t st, const char* name) {
+    const int ngroups = p.ncols / (EPI == EPI_SWIGLU ? 16 : 32);
+    const long long items = 8LL * ntiles_max * ceil_div(ngroups, 8);
+    if (items <= 0) return YVMOE_OK;
+#define YV_FEW(WFV) gemm_few_kernel<WFV, EPI><<<(unsigned)items, 256, 0, st>>>(p, ngroups)
+    switch (wf) {
+        case YVMOE_W_BF16: YV_FEW(YVMOE_W_BF16); break;
+        case YVMOE_W_INT8: YV_FEW(YVMOE_W_INT8); break;
+        case YVMOE_W_INT4: YV_FEW(YVMOE_W_INT4); break;
+        case YVMOE_W_FP8: YV_FEW(YVMOE_W_FP8); break;
+        default: set_error("unsupported weight format %d for bf16 activations", wf); return YVMOE_ERR_DTYPE;
+    }
+#undef YV_FEW
+    YV_LAUNCH_CHECK(name);
+    return YVMOE_OK;
+}
+
 // Mid-sized form: tile_rows-row (64 or 128) tiles of the tile table; the grid covers 8 XCDs x
 // (the most tiles the batch can have) x column groups per XCD.
 template <int EPI>
@@ -2958,7 +3101,19 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
     int* tile_seg = tt.tile_seg;
     int* tile_row0 = tt.tile_row0;
     int* ntiles = tt.ntiles;
-    const int T = max_tiles(N, k, E, S, tile_rows);
+    // every tile of the main table holds a row
+    const int T = (int)std::min<long long>(max_tiles(N, k, E, S, tile_rows),
+                                           (long long)N * k + (long long)S * ceil_div(N, tile_rows));
+    // a few tokens: by the mean rows per expert (from where the streaming form's work-groups fill
+    // the chip; H 4096, 64 experts, 4 / 6 / 8 tokens: int8 69 / 87 / 113 us there, 67 / 89 / 114 on
+    // the few-token form; 8 / 16: fp8 113 / 151 and 111 / 152; 32 / 64: bf16 350 / 367 and 338 / 371;
+    // H 5120, 128 experts, 8 / 16: int4 164 / 238 and 163 / 252), and always where a layer's experts
+    // are too few to fill it
+    const long long slots = (long long)N * k;
+    const bool few = streaming && (E * ceil_div(F, 32) <= 1024 ||
+                                   (w->format == YVMOE_W_BF16  ? slots < 3LL * E
+                                    : w->format == YVMOE_W_FP8 ? slots < E
+                                                               : 2 * slots < E));
     if (!tiles_ready) {
         build_tiles_kernel<<<1, 512, 0, st>>>(routing->offsets, E, S, N, k, tile_rows, tt.fold, seg,
                                               tile_seg, tile_row0, ntiles, tt.light, tt.light_min,
@@ -3004,7 +3159,8 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
     p.ldo = F;
     p.kchunk = H;
     const bool f3 = act != YVMOE_ACT_BF16 && tile_rows == 128;
-    int rc = f3 ? f32x3_dispatch<EPI_SWIGLU>(p, T, st, "expert_gemm1")
+    int rc = few ? few_dispatch<EPI_SWIGLU>(wf, p, T, st, "expert_gemm1")
+           : f3 ? f32x3_dispatch<EPI_SWIGLU>(p, T, st, "expert_gemm1")
            : mid ? mid_dispatch<EPI_SWIGLU>(wf, p, T, tile_rows, st, "expert_gemm1")
            : tiled ? tile_dispatch<EPI_SWIGLU>(wf, p, T, st, "expert_gemm1", tt.fold > 0)
            : streaming ? (S > 0
@@ -3038,6 +3194,7 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
         if (rc != YVMOE_OK || tt.light == 0) return rc;
         return light_launch(p, std::integral_constant<int, EPI_DOWN>{}, "expert_gemm2_light");
     }
+    if (few) return few_dispatch<EPI_DOWN>(wf, p, T, st, "expert_gemm2");
     if (f3) return f32x3_dispatch<EPI_DOWN>(p, T, st, "expert_gemm2");
     if (mid) return mid_dispatch<EPI_DOWN>(wf, p, T, tile_rows, st, "expert_gemm2");
     return streaming ? (S > 0

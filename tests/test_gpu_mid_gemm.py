@@ -97,3 +97,23 @@ def test_tiled_forms(cuda, oracle, fmt, hidden, ffn):
     w = forced_rows(spec, MANY)
     _, _, routing = _run_and_check(oracle, w, label=f"tiled {fmt} H={hidden} F={ffn} N={sum(MANY)}")
     assert routing.counts.cpu().tolist() == MANY
+
+
+@pytest.mark.parametrize("fmt,hidden,ffn", [
+    ("int8", 64, 64),      # one k-step: three wavefronts without a chunk
+    ("int8", 192, 320),    # 3 and 5 k-steps: a partial chunk, one or two wavefronts
+    ("int8", 1024, 1088),  # 16 and 17 k-steps: a chunk each, and one left over
+    ("bf16", 64, 192), ("bf16", 1152, 640),
+    ("int4", 128, 384), ("int4", 1152, 640), ("fp8", 384, 128), ("fp8", 2432, 640),
+])
+def test_a_few_rows(cuda, oracle, fmt, hidden, ffn):
+    """The few-token form (K dealt out to the wavefronts): tiles of 1, 2, 16 and 16 + 1 rows, empty
+    experts, a shared segment of several tiles, and a single token."""
+    from pisceslx_amd import _lib
+    counts = [0, 1, 2, 16, 17, 3, 1, 0]
+    spec = LayerSpec("few", hidden, ffn, len(counts), 1, 1, getattr(_lib, "W_" + fmt.upper()),
+                     torch.bfloat16, fixed_shape_mode=True)
+    w = forced_rows(spec, counts)
+    _, _, routing = _run_and_check(oracle, w, label=f"few {fmt} H={hidden} F={ffn} N={sum(counts)}")
+    assert routing.counts.cpu().tolist() == counts
+    _run_and_check(oracle, make_workload(spec, device="cuda", lengths=[1]), label=f"few {fmt} N=1")
