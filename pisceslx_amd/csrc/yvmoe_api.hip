@@ -260,11 +260,11 @@ int32_t yvmoe_combine(const void* y, int32_t act_dtype, int32_t n_tokens, int32_
                           out, shared_out, (hipStream_t)stream);
 }
 
-int32_t yvmoe_forward(const void* x, int32_t act_dtype, int32_t n_tokens,
+static int32_t forward_run(const void* x, int32_t act_dtype, int32_t n_tokens,
                       const yvmoe_router* router, const yvmoe_expert_weights* experts,
                       const float* mix, const void* skip, void* out, void* shared_out,
                       yvmoe_routing* routing, void* workspace, size_t workspace_bytes,
-                      void* stream) {
+                      void* stream, bool may_drop_split) {
     clear_error();
     int rc = check_router(router, act_dtype);
     if (rc) return rc;
@@ -276,7 +276,10 @@ int32_t yvmoe_forward(const void* x, int32_t act_dtype, int32_t n_tokens,
                YVMOE_ERR_SHAPE, "router (E=%d, H=%d) and experts (E=%d, H=%d) disagree",
                router->num_experts, router->hidden, experts->num_routed, experts->hidden);
     YV_REQUIRE(n_tokens >= 0, YVMOE_ERR_ARG, "n_tokens=%d < 0", n_tokens);
-    const size_t need = yvmoe_workspace_bytes(n_tokens, act_dtype, router, experts);
+    size_t need = yvmoe_workspace_bytes(n_tokens, act_dtype, router, experts);
+    // without room for the router's split partial sums (the last region) it runs unsplit
+    const bool drop = may_drop_split && workspace_bytes < need;
+    if (drop) need -= router_partials_bytes(n_tokens, router->num_experts, act_dtype, router->hidden);
     YV_REQUIRE(workspace != nullptr && workspace_bytes >= need, YVMOE_ERR_WORKSPACE,
                "workspace %zu bytes, need %zu", workspace_bytes, need);
     YV_REQUIRE(n_tokens == 0 || (x && out), YVMOE_ERR_ARG, "NULL pointer");
@@ -291,7 +294,7 @@ int32_t yvmoe_forward(const void* x, int32_t act_dtype, int32_t n_tokens,
     float* logits = (float*)(ws + route_ws(N, E, k).bytes +
                              ffn_ws(N, k, E, experts->num_shared, experts->ffn, act_dtype).bytes);
     void* y = (char*)logits + align_up((size_t)N * ld * 4, 256);
-    float* partials = (float*)((char*)y + y_bytes(N, k, experts->num_shared, experts->hidden, act_dtype));
+    float* partials = drop ? nullptr : (float*)((char*)y + y_bytes(N, k, experts->num_shared, experts->hidden, act_dtype));
     // The routing's top-k kernels sum the router's split-K partial sums themselves (in split
     // order, as the reduction of yvmoe_router_logits does), so the sums need no launch of their
     // own (above kSmallRouteTok tokens up to kFoldSplits splits: more, read per logit, measured
@@ -299,7 +302,7 @@ int32_t yvmoe_forward(const void* x, int32_t act_dtype, int32_t n_tokens,
     // the expert GEMM tile table.
     const bool small = N > 0 && N <= kSmallRouteTok;
     const int ks = router_ksplit(N, E, act_dtype, router->hidden);
-    const bool split = N > 0 && ks > 1 && (small || ks <= kFoldSplits);
+    const bool split = N > 0 && ks > 1 && !drop && (small || ks <= kFoldSplits);
     if (N > 0) {
         rc = router_gemm_launch(x, act_dtype, N, router, logits, ld, partials, st, !split);
         if (rc) return rc;
@@ -323,6 +326,15 @@ int32_t yvmoe_forward(const void* x, int32_t act_dtype, int32_t n_tokens,
     if (rc) return rc;
     return combine_launch(y, act_dtype, N, experts->hidden, k, experts->num_shared, routing, mix,
                           skip, out, shared_out, st);
+}
+
+int32_t yvmoe_forward(const void* x, int32_t act_dtype, int32_t n_tokens,
+                      const yvmoe_router* router, const yvmoe_expert_weights* experts,
+                      const float* mix, const void* skip, void* out, void* shared_out,
+                      yvmoe_routing* routing, void* workspace, size_t workspace_bytes,
+                      void* stream) {
+    return forward_run(x, act_dtype, n_tokens, router, experts, mix, skip, out, shared_out, routing,
+                       workspace, workspace_bytes, stream, false);
 }
 
 }  // extern "C"
@@ -371,7 +383,9 @@ int32_t yvmoe_forward_static(const void* x, int32_t act_dtype, int32_t n_tokens,
     rc = check_experts(experts, act_dtype);
     if (rc) return rc;
     YV_REQUIRE(n_tokens >= 0, YVMOE_ERR_ARG, "n_tokens=%d < 0", n_tokens);
-    const size_t need = yvmoe_workspace_bytes(n_tokens, act_dtype, router, experts);
+    // the router's split partial sums are left out where only they would not fit
+    const size_t need = yvmoe_workspace_bytes(n_tokens, act_dtype, router, experts) -
+                        router_partials_bytes(n_tokens, router->num_experts, act_dtype, router->hidden);
     YV_REQUIRE(need <= (size_t)YVMOE_STATIC_SCRATCH_BYTES, YVMOE_ERR_WORKSPACE,
                "n_tokens=%d needs %zu bytes of scratch, more than the static %zu bytes of "
                "yvmoe_forward_static (use yvmoe_forward with a workspace)",
@@ -379,8 +393,8 @@ int32_t yvmoe_forward_static(const void* x, int32_t act_dtype, int32_t n_tokens,
     void* ws = nullptr;
     rc = static_scratch(&ws);
     if (rc) return rc;
-    return yvmoe_forward(x, act_dtype, n_tokens, router, experts, mix, skip, out, shared_out,
-                         routing, ws, (size_t)YVMOE_STATIC_SCRATCH_BYTES, stream);
+    return forward_run(x, act_dtype, n_tokens, router, experts, mix, skip, out, shared_out, routing, ws,
+                       (size_t)YVMOE_STATIC_SCRATCH_BYTES, stream, true);
 }
 
 static int check_moegate(const yvmoe_moegate* g, int act) {

@@ -315,122 +315,6 @@ struct NMat {
     static constexpr int value = (EPI == EPI_SWIGLU) ? 2 : 1;
 };
 
-// ------------------------------------------------------------------ bf16, dense fp32 output
-// out[r][n] (+ split z at z * split_stride) = A · Wᵀ for bf16 weights and row counts between the
-// streaming and the tiled forms: 64-row tiles, NCB 16-column blocks per wavefront. Weight loads
-// run RB - 1 k-steps ahead of the MFMAs, activation loads RA - 1 (RA divides RB).
-template <int NCB, int RB = 4, int RA = 2>
-__global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmParams p) {
-    static_assert(RB % RA == 0, "A ring depth must divide the B ring depth");
-    constexpr int MAXRB = 4;
-    typedef BLoad<YVMOE_W_BF16> BL;
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int row0 = blockIdx.x * MAXRB * 16;
-    if (row0 >= p.nrows) return;
-    const int seg_end = p.nrows;
-    const int col0 = (blockIdx.y * 4 + wave) * NCB * 16;
-    if (col0 >= p.ncols) return;
-    const int nrb = min(MAXRB, (seg_end - row0 + 15) / 16);
-    const int kl = (lane >> 4) * 16;  // this lane's k offset inside a 64-wide k-step
-    const int kbeg = blockIdx.z * p.kchunk;
-    const int nks = (min(p.K, kbeg + p.kchunk) - kbeg) / 64;
-
-    const char* arow[MAXRB];
-#pragma unroll
-    for (int rb = 0; rb < MAXRB; ++rb) {
-        int r = row0 + rb * 16 + (lane & 15);
-        if (r >= seg_end) r = row0;
-        arow[rb] = (const char*)p.A + ((long long)r * p.lda + kbeg + kl) * 2;
-    }
-    const char* bptr[NCB];
-    int ncol[NCB];
-#pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) {
-        ncol[cb] = col0 + cb * 16 + (lane & 15);
-        bptr[cb] = BL::bptr(p.B0, 0, ncol[cb], p.K, kbeg, lane);
-    }
-
-    f32x4 acc[NCB][MAXRB];
-#pragma unroll
-    for (int cb = 0; cb < NCB; ++cb)
-#pragma unroll
-        for (int rb = 0; rb < MAXRB; ++rb) acc[cb][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    Frag16 braw[RB][NCB];
-    auto load_b = [&](int ks, Frag16 (&dst)[NCB]) {
-#pragma unroll
-        for (int cb = 0; cb < NCB; ++cb) BL::load_blk(dst[cb], bptr[cb], ks);
-    };
-    // Loads are unconditional (k-step clamped to the last one, row blocks past nrb read the
-    // tile's first row): with no branch around them the compiler can wait for exactly the
-    // oldest in-flight load instead of draining the whole ring before every MFMA.
-    auto load_a = [&](int ks, Frag16 (&af)[MAXRB]) {
-#pragma unroll
-        for (int rb = 0; rb < MAXRB; ++rb) {
-            const uint4* q = (const uint4*)(arow[rb] + (size_t)ks * 128);
-            af[rb].u[0] = q[0];
-            af[rb].u[1] = q[1];
-        }
-    };
-    auto mma = [&](const Frag16 (&bf)[NCB], const Frag16 (&af)[MAXRB]) {
-#pragma unroll
-        for (int cb = 0; cb < NCB; ++cb) {
-#pragma unroll
-            for (int rb = 0; rb < MAXRB; ++rb) {
-                if (rb < nrb) {
-                    f32x4& dst = acc[cb][rb];
-                    dst = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[rb].v[0], bf[cb].v[0], dst, 0, 0, 0);
-                    dst = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[rb].v[1], bf[cb].v[1], dst, 0, 0, 0);
-                }
-            }
-        }
-    };
-    auto kc = [&](int ks) { return ks < nks ? ks : nks - 1; };
-
-    Frag16 abuf[RA][MAXRB];
-    if (nks > 0) {
-#pragma unroll
-        for (int r = 0; r < RB - 1; ++r) load_b(kc(r), braw[r]);
-#pragma unroll
-        for (int r = 0; r < RA - 1; ++r) load_a(kc(r), abuf[r]);
-    }
-    int ks0 = 0;
-    for (; ks0 + RB <= nks; ks0 += RB) {
-#pragma unroll
-        for (int r = 0; r < RB; ++r) {
-            const int ks = ks0 + r;
-            load_b(kc(ks + RB - 1), braw[(r + RB - 1) % RB]);
-            load_a(kc(ks + RA - 1), abuf[(r + RA - 1) % RA]);
-            mma(braw[r], abuf[r % RA]);
-        }
-    }
-    // tail (fewer than RB steps): their weights are already in ring slots 0..nks-ks0-1
-#pragma unroll
-    for (int r = 0; r < RB - 1; ++r) {
-        if (ks0 + r < nks) {
-            load_a(kc(ks0 + r + RA - 1), abuf[(r + RA - 1) % RA]);
-            mma(braw[r], abuf[r % RA]);
-        }
-    }
-#pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) {
-        const int n = ncol[cb];
-#pragma unroll
-        for (int rb = 0; rb < MAXRB; ++rb) {
-            if (rb < nrb) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int r = row0 + rb * 16 + (lane >> 4) * 4 + i;
-                    if (r < seg_end)
-                        ((float*)p.out)[blockIdx.z * p.split_stride + (long long)r * p.ldo + n] =
-                            f32_out(p, acc[cb][rb][i], n, blockIdx.z);
-                }
-            }
-        }
-    }
-}
-
 // ------------------------------------------------------------------ bf16, streaming form
 // Weight-streaming form for batches whose experts hold few rows (decode). A work-group of 4
 // wavefronts owns one tile (up to 16*MAXRB rows of one expert); every wavefront streams one
@@ -2914,9 +2798,9 @@ int tile_launch(int wf, const GemmParams& p, int ntiles_max, hipStream_t st, con
     return YVMOE_OK;
 }
 
-// Dense fp32-output GEMM on 64-row tiles: grid (tiles, column groups, K splits); NCB 16-column
+// Dense GEMM of fp32 operands on 64-row tiles: grid (tiles, column groups, K splits); NCB 16-column
 // blocks per wavefront.
-int gemm_dispatch(int act, GemmParams p, int ntiles, int ncb, int ksplit, hipStream_t st, const char* name) {
+int gemm_dispatch(GemmParams p, int ntiles, int ncb, int ksplit, hipStream_t st, const char* name) {
     if (ntiles <= 0) return YVMOE_OK;
     if (p.ncols % (16 * ncb) != 0) {
         set_error("%s: %d columns are not a multiple of %d", name, p.ncols, 16 * ncb);
@@ -2924,13 +2808,8 @@ int gemm_dispatch(int act, GemmParams p, int ntiles, int ncb, int ksplit, hipStr
     }
     const int cols_per_wg = 4 * ncb * 16;
     dim3 grid(ntiles, (p.ncols + cols_per_wg - 1) / cols_per_wg, ksplit);
-    if (act == YVMOE_ACT_F32) {
-        if (ncb == 2) gemm_f32_kernel<2><<<grid, 256, 0, st>>>(p);
-        else gemm_f32_kernel<1><<<grid, 256, 0, st>>>(p);
-    } else {
-        if (ncb == 2) gemm_bf16_kernel<2><<<grid, 256, 0, st>>>(p);
-        else gemm_bf16_kernel<1><<<grid, 256, 0, st>>>(p);
-    }
+    if (ncb == 2) gemm_f32_kernel<2><<<grid, 256, 0, st>>>(p);
+    else gemm_f32_kernel<1><<<grid, 256, 0, st>>>(p);
     YV_LAUNCH_CHECK(name);
     return YVMOE_OK;
 }
@@ -2980,8 +2859,11 @@ int dense_partials_launch(const void* x, int act, int N, int K, const void* w, i
         // or needing more partial sums)
         return stream_dispatch<EPI_F32, 1, 1, 4, YV_DPF>(YVMOE_W_BF16, p, 1, st, name, ks);
     }
-    return gemm_dispatch(act, p, ceil_div(N, kTileRows), (ncols % 32 == 0) ? 2 : 1, ks,
-                                  st, name);
+    if (act != YVMOE_ACT_F32) {  // bf16: up to 64 rows streamed, more tiled (columns in 256s)
+        set_error("%s: no dense bf16 form for %d rows x %d columns", name, N, ncols);
+        return YVMOE_ERR_SHAPE;
+    }
+    return gemm_dispatch(p, ceil_div(N, kTileRows), (ncols % 32 == 0) ? 2 : 1, ks, st, name);
 }
 
 int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, float* out, int ld,
@@ -3011,24 +2893,24 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
         if (rc || !reduce) return rc;
         return reduce_splits_launch(partials, ks, (long long)N * ld, out, st, "router_reduce");
     }
-    p.kchunk = r->hidden / ks;
-    if (ks == 1 || partials == nullptr) {
-        p.kchunk = r->hidden;
-        p.out = out;
-        const int ncb = (p.ncols % 32 == 0) ? 2 : 1;
-        return gemm_dispatch(act, p, ceil_div(N, kTileRows), ncb, 1, st, "router_gemm");
-    }
-    p.out = partials;
-    p.split_stride = (long long)N * ld;
+    // ks == 1 writes the logits themselves; else the partial sums, the last split's K range shorter
+    const bool direct = ks == 1 || partials == nullptr;
+    p.kchunk = direct ? r->hidden : router_split_steps(N, r->num_experts, act, r->hidden) * 64;
+    p.out = direct ? out : partials;
+    p.split_stride = direct ? 0 : (long long)N * ld;
+    const int nz = direct ? 1 : ks;
     int rc;
-    // up to 64 rows: the weight-streaming form, in 16-row tiles (the router operand, 2 MB at
-    // E = 64, stays in L2 for the tiles that re-read it: 2.7 us less per decode step than one
-    // 64-row tile; the 138 MB YvMoEGate projection keeps 64-row tiles, which measured faster)
-    if (dense_streamed(act, N, p.ncols, r->hidden))
-        rc = stream_dispatch<EPI_F32, 4, 1, 1>(YVMOE_W_BF16, p, ceil_div(N, 16), st, "router_gemm", ks);
+    // 16-row tiles up to kSmallRouteTok tokens (the router operand, 2 MB at E = 64, stays in L2 for the
+    // tiles that re-read it: 2.7 us less per decode step at 64 tokens than one 64-row tile; the 138
+    // MB YvMoEGate projection keeps 64-row tiles, which measured faster; layer at 128 tokens 226 ->
+    // 223 us against 64-row tiles without LDS), 64-row tiles above
+    if (act == YVMOE_ACT_BF16)
+        rc = N <= kSmallRouteTok
+                 ? stream_dispatch<EPI_F32, 4, 1, 1>(YVMOE_W_BF16, p, ceil_div(N, 16), st, "router_gemm", nz)
+                 : stream_dispatch<EPI_F32, 1, 1, 4, YV_DPF>(YVMOE_W_BF16, p, ceil_div(N, 64), st, "router_gemm", nz);
     else
-        rc = gemm_dispatch(act, p, ceil_div(N, kTileRows), 1, ks, st, "router_gemm");
-    if (rc || !reduce) return rc;
+        rc = gemm_dispatch(p, ceil_div(N, kTileRows), direct && p.ncols % 32 == 0 ? 2 : 1, nz, st, "router_gemm");
+    if (rc || direct || !reduce) return rc;
     return reduce_splits_launch(partials, ks, (long long)N * ld, out, st, "router_reduce");
 }
 
@@ -3044,7 +2926,9 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
 //   against 246), and any format up to 48 rows when 128-row tiles would leave the down
 //   projection under two work-groups per CU (H 1024, 8 experts of 16 / 32 rows: 48.5 / 48.7 us
 //   against 48.2 / 58.3).
-// * 128: the mid form, up to 150 rows for int8 and int4, 125 for fp8 and 112 for bf16, from where an
+// * 128: the mid form, up to 150 rows for int8 and int4, 125 for fp8 and 112 for bf16 and for fp8
+//   layers of 128 experts and more (skewed loads, 109 / 122 rows: 3935 / 4251 us against 3720 /
+//   3994), from where an
 //   expert's rows past 128 cost a second pass over its weights (H 4096, 64 experts, 96 / 131 /
 //   159 rows: int8 386 / 546 / 690 us against 576 / 601 / 686 on 256-row tiles, bf16 546 / 817 /
 //   1038 against 646 / 653 / 680; fp8 H 7168, 256 experts, 94 / 128 rows 2864 / 4203 against 3309 /
@@ -3057,7 +2941,8 @@ int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf) {
     if (act != YVMOE_ACT_BF16) return slots < 48LL * E ? kTileRows : 128;
     if (slots < (wf == YVMOE_W_INT4 ? 4LL : 8LL) * E) return 16;
     const bool tiles = wf == YVMOE_W_INT8 || wf == YVMOE_W_BF16 || (H <= 8192 && F <= 8192);
-    const long long most = wf == YVMOE_W_INT8 || wf == YVMOE_W_INT4 ? 150 : wf == YVMOE_W_FP8 ? 125 : 112;
+    const long long most = wf == YVMOE_W_INT8 || wf == YVMOE_W_INT4 ? 150
+                           : wf == YVMOE_W_FP8 && E < 128                   ? 125 : 112;
     const long long items = (long long)max_tiles(N, k, E, S, TBM) * ceil_div(F, TBN / 2);
     if (tiles && slots >= most * E && items > 448) return TBM;
     if (slots <= 48LL * E && (wf == YVMOE_W_INT4 || (long long)E * ceil_div(H, 128) < 512)) return 64;

@@ -44,8 +44,6 @@ inline int router_ld(int E, int act) {
     return pad16(E) + (act == YVMOE_ACT_BF16 ? 3 * kPredDim : kPredDim);
 }
 
-// K splits of the router GEMM: enough work-groups to spread a small batch over the chip,
-// at least 128 of K per split (2 k-steps); partial sums are reduced in split order.
 // Batches of up to kSmallRouteTok tokens take the two-kernel small-batch routing path
 // (per-token top-k with the router's split-K reduction folded in, then everything else in
 // one work-group).
@@ -60,11 +58,16 @@ constexpr int kFoldSplits = 4;
 #define YV_ROUTER_KS_MAX 16
 #endif
 
-// Router GEMMs of more than kSmallRouteTok tokens with bf16 operands run on the LDS-tiled MFMA
-// form: 256 x 256 output tiles (the last column block may be partial), K split so that the
-// (tile, column block, split) items spread over the 256 CUs.
+// Router GEMMs with bf16 operands: the weight-streaming form (16-row tiles up to kSmallRouteTok
+// tokens, 64-row tiles and at most kFoldSplits K splits above) up to kStreamRouteTok tokens, the
+// LDS-tiled MFMA form above: 256 x 256 output tiles (the last column block may be partial), K split so
+// that the (tile, column block, split) items spread over the 256 CUs. A batch of a few tiles needs
+// many splits there, whose reduction is a launch of its own (layer, H 4096, 64 experts, 300 / 700 /
+// 3,000 tokens: 299 / 382 / 1125 us tiled, 285 / 368 / 1110 streamed; H 1024, 8 experts, 500 tokens
+// 114 and 96).
+constexpr int kStreamRouteTok = 3072;
 inline bool router_tiled(int act, int N, int ncols, int K) {
-    return act == YVMOE_ACT_BF16 && N > kSmallRouteTok && ncols % 16 == 0 && K % 64 == 0 && K > 0;
+    return act == YVMOE_ACT_BF16 && N > kStreamRouteTok && ncols % 16 == 0 && K % 64 == 0 && K > 0;
 }
 
 // k-steps (of 64) per split of the tiled router GEMM: the choice with the least estimated time,
@@ -89,16 +92,20 @@ inline int router_tiled_steps(int N, int ncols, int K) {
     return best;
 }
 
+// K splits of the other router GEMMs: enough work-groups to spread the batch over the chip, at
+// least 128 of K per split; steps (of 64) per split, the last split shorter.
+inline int router_split_steps(int N, int E, int act, int H) {
+    const int groups = ceil_div(router_ld(E, act), 64);
+    const int wgs = ceil_div(N > 0 ? N : 1, 64) * groups;
+    const int most = act == YVMOE_ACT_BF16 && N > kSmallRouteTok ? kFoldSplits : YV_ROUTER_KS_MAX;
+    int ks = 1;
+    while (ks * 2 <= most && (wgs * ks * 2 <= 512 || most == kFoldSplits) && H / (ks * 2) >= 128) ks *= 2;
+    return ceil_div(H / 64, ks);
+}
 inline int router_ksplit(int N, int E, int act, int H) {
     const int ld = router_ld(E, act);
     if (router_tiled(act, N, ld, H)) return ceil_div(H / 64, router_tiled_steps(N, ld, H));
-    const int groups = ceil_div(router_ld(E, act), 64);
-    const int wgs = ceil_div(N > 0 ? N : 1, 64) * groups;
-    int ks = 1;
-    while (ks * 2 <= YV_ROUTER_KS_MAX && wgs * ks * 2 <= 512 && H % (ks * 2 * 64) == 0 &&
-           H / (ks * 2) >= 128)
-        ks *= 2;
-    return ks;
+    return ceil_div(H / 64, router_split_steps(N, E, act, H));
 }
 
 // Dense fp32-output GEMMs of more than 64 rows with bf16 operands, 256-multiple columns and
@@ -131,9 +138,16 @@ inline int dense_splits(int act, int N, int ncols, int K) {
     return ks;
 }
 
+// Room for the split partial sums: of the tiled form's splits too where the streaming form, which
+// has fewer, runs (so a workspace never has to be larger than for that form).
 inline size_t router_partials_bytes(int N, int E, int act, int H) {
-    const int ks = router_ksplit(N, E, act, H);
-    return ks > 1 ? align_up((size_t)ks * N * router_ld(E, act) * 4, 256) : 0;
+    const int ld = router_ld(E, act);
+    int ks = router_ksplit(N, E, act, H);
+    if (act == YVMOE_ACT_BF16 && N > kSmallRouteTok && H % 64 == 0) {
+        const int tiled = ceil_div(H / 64, router_tiled_steps(N, ld, H));
+        ks = ks > tiled ? ks : tiled;
+    }
+    return ks > 1 ? align_up((size_t)ks * N * ld * 4, 256) : 0;
 }
 
 // Upper bound on the number of GEMM tiles of tile_rows rows over all segments.

@@ -39,6 +39,11 @@ def _router(E, H, dev, seed):
     (4344, 5120, 128),  # cfg4's shape: 7 splits of 12 k-steps, the last of 8
     (600, 2048, 80),    # ld 272: the last column block holds one 16-column block
     (513, 64, 16),      # K = 64: one k-step, no split
+    (70, 3008, 64),     # 47 k-steps: splits of 3, the last of 2
+    (256, 1088, 128),   # 17 k-steps
+    (258, 3008, 40),    # above the small-batch bound: splits of 12, the last of 11
+    (3072, 320, 8),     # the streaming form's last size: 5 k-steps in splits of 3 and 2
+    (3073, 1024, 64),   # and the tiled form's first
 ])
 def test_router_logits_against_float64(cuda, N, H, E):
     gw, st = _router(E, H, cuda, seed=N + H + E)
