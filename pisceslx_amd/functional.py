@@ -28,7 +28,9 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 def _stream(device: torch.device):
-    return torch.cuda.current_stream(device).cuda_stream
+    """The handle of torch's current stream on a tensor's device (without the Stream object that
+    torch.cuda.current_stream builds: 0.1 us instead of 1.9 on every call)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _require_cuda(*ts: Optional[torch.Tensor]) -> torch.device:
@@ -449,6 +451,9 @@ def moe_forward_moegate(x2d: torch.Tensor, gate: MoEGateState, top_k: int, exper
     return out, shared_out, routing, logits, loss, workspace
 
 
+_RMS_PARAMS1, _RMS_PARAMS2 = _lib.RMSNormParams * 1, _lib.RMSNormParams * 2
+
+
 def rms_norm(x: torch.Tensor, norms, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """RMSNorm over the last dimension, one or two norms in sequence in one pass.
 
@@ -458,28 +463,27 @@ def rms_norm(x: torch.Tensor, norms, out: Optional[torch.Tensor] = None) -> torc
     (opss/kernels/fused_rms_norm.py:42): fp32 sum of squares, (x / sqrt(Σx²/H + eps)) * weight
     rounded once, + bias rounded again (model/core/norms.py:998-999). ``out`` may be x.
     """
-    norms = list(norms)
+    norms = tuple(norms)
     if len(norms) not in (1, 2):
         raise ValueError("rms_norm takes one or two norms")
-    H = x.shape[-1]
-    ts = [x] + [t for w, b, _ in norms for t in (w, b)]
-    dev = _require_cuda(*ts, out)
-    act = _act(x.dtype)
-    for w, b, _ in norms:
-        for t in (w, b):
-            if t is not None and (t.dtype != x.dtype or t.numel() != H):
-                raise ValueError(f"norm weight/bias must be {x.dtype} [{H}]")
+    shape, dt = x.shape, x.dtype
+    H = shape[-1]
+    dev = _require_cuda(x, *norms[0][:2], *norms[-1][:2], out)
+    act = _act(dt)
+    params = (_RMS_PARAMS1 if len(norms) == 1 else _RMS_PARAMS2)()
+    for p, (w, b, eps) in zip(params, norms):
+        if w.dtype != dt or w.numel() != H or (b is not None and (b.dtype != dt or b.numel() != H)):
+            raise ValueError(f"norm weight/bias must be {dt} [{H}]")
+        p.weight = w.data_ptr()
+        p.bias = None if b is None else b.data_ptr()
+        p.eps = float(eps)
     if out is None:
         out = torch.empty_like(x)
-    elif out.shape != x.shape or out.dtype != x.dtype:
+    elif out.shape != shape or out.dtype != dt:
         raise ValueError("out must match x")
     N = x.numel() // H if H else 0
-    params = (_lib.RMSNormParams * len(norms))()
-    for i, (w, b, eps) in enumerate(norms):
-        params[i].weight = w.data_ptr()
-        params[i].bias = _ptr(b)
-        params[i].eps = float(eps)
-    _lib.check(_lib.lib().yvmoe_rmsnorm(x.data_ptr() if N > 0 else None, act, N, H, params,
-                                        len(norms), out.data_ptr() if N > 0 else None,
-                                        _stream(dev)), "yvmoe_rmsnorm")
+    rc = _lib.lib().yvmoe_rmsnorm(x.data_ptr() if N > 0 else None, act, N, H, params, len(norms),
+                                  out.data_ptr() if N > 0 else None, _stream(dev))
+    if rc:
+        _lib.check(rc, "yvmoe_rmsnorm")
     return out

@@ -42,7 +42,12 @@ class YvRMSNorm(nn.Module):
             nn.init.zeros_(self.bias)
 
     def norm_params(self):
-        return (self.weight.detach(), None if self.bias is None else self.bias.detach(), self.eps)
+        # straight from the parameter table where they stand there (not, say, parametrized): the
+        # attribute lookups of nn.Module take longer than the rest of this function
+        p = self._parameters
+        weight = p["weight"] if "weight" in p else self.weight
+        bias = p["bias"] if "bias" in p else self.bias
+        return (weight.detach(), None if bias is None else bias.detach(), self.eps)
 
     @torch.no_grad()
     def forward(self, x: torch.Tensor) -> torch.Tensor:
