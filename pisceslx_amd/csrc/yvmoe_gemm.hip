@@ -7,9 +7,10 @@
 //
 // Forms. Every expert GEMM runs over a table of tiles (up to 16, 64, 128 or 256 rows of one expert
 // segment: rows are expert-sorted slots, shared experts are extra segments of all N tokens) times
-// column groups: the weight-streaming form at decode, the mid-sized form for tens of rows per
-// expert, the LDS-tiled form at prefill (ffn_tile_rows draws the lines). The weights are
-// dequantized in registers to bf16; the activations are gathered through the permutation.
+// column groups: the few-token and the weight-streaming form at decode, the mid-sized form for
+// tens of rows per expert, the LDS-tiled form at prefill, two forms of their own for fp32
+// (ffn_tile_rows draws the lines). Quantized weights are dequantized in registers to bf16; the
+// activations are gathered through the permutation.
 //
 // Rounding points follow the reference's bf16 path, because the reference's own bf16
 // chain sits about 2e-2 (max-abs) from exact arithmetic at these shapes and a more exact
@@ -2927,14 +2928,14 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
 //   projection under two work-groups per CU (H 1024, 8 experts of 16 / 32 rows: 48.5 / 48.7 us
 //   against 48.2 / 58.3).
 // * 128: the mid form, up to 150 rows for int8 and int4, 125 for fp8 and 112 for bf16 and for fp8
-//   layers of 128 experts and more (skewed loads, 109 / 122 rows: 3935 / 4251 us against 3720 /
-//   3994), from where an
-//   expert's rows past 128 cost a second pass over its weights (H 4096, 64 experts, 96 / 131 /
-//   159 rows: int8 386 / 546 / 690 us against 576 / 601 / 686 on 256-row tiles, bf16 546 / 817 /
-//   1038 against 646 / 653 / 680; fp8 H 7168, 256 experts, 94 / 128 rows 2864 / 4203 against 3309 /
-//   3823, H 2944, 64 experts, 122 rows 305 against 389); any number of rows where the 256-row form's scale tables
-//   (fp8, int4: 8192 of K) do not hold the shape; and where 256-row tiles would be under two work-groups per CU (H 1024, 8 experts, 256
-//   / 375 rows: bf16 100 / 150 us against 127 / 134, int8 95 / 130 against 138 / 141).
+//   layers of 128 experts and more, from where an expert's rows past 128 cost a second pass over its
+//   weights (H 4096, 64 experts, 96 / 131 / 159 rows: int8 386 / 546 / 690 us against 576 / 601 /
+//   686 on 256-row tiles, bf16 546 / 817 / 1038 against 646 / 653 / 680; fp8 H 2944, 64 experts, 122
+//   rows 305 against 389; H 7168, 256 experts, 109 / 128 rows 3205 / 4203 against 3429 / 3823, with
+//   a skewed load 3935 / 4313 against 3720 / 4004); any number of rows where the 256-row form's scale
+//   tables (fp8, int4: 8192 of K) do not hold the shape; and where 256-row tiles would be under two
+//   work-groups per CU (H 1024, 8 experts, 256 / 375 rows: bf16 100 / 150 us against 127 / 134, int8
+//   95 / 130 against 138 / 141).
 // * 256: the LDS-tiled form above that.
 int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf) {
     const long long slots = (long long)N * k;
