@@ -102,7 +102,9 @@ inline int router_split_steps(int N, int E, int act, int H) {
     while (ks * 2 <= most && (wgs * ks * 2 <= 512 || most == kFoldSplits) && H / (ks * 2) >= 128) ks *= 2;
     return ceil_div(H / 64, ks);
 }
+// (H < 64: sizes are asked for before a shape is checked, and routing alone never reads it.)
 inline int router_ksplit(int N, int E, int act, int H) {
+    if (H < 64) return 1;
     const int ld = router_ld(E, act);
     if (router_tiled(act, N, ld, H)) return ceil_div(H / 64, router_tiled_steps(N, ld, H));
     return ceil_div(H / 64, router_split_steps(N, E, act, H));
@@ -143,7 +145,7 @@ inline int dense_splits(int act, int N, int ncols, int K) {
 inline size_t router_partials_bytes(int N, int E, int act, int H) {
     const int ld = router_ld(E, act);
     int ks = router_ksplit(N, E, act, H);
-    if (act == YVMOE_ACT_BF16 && N > kSmallRouteTok && H % 64 == 0) {
+    if (act == YVMOE_ACT_BF16 && N > kSmallRouteTok && H >= 64 && H % 64 == 0) {
         const int tiled = ceil_div(H / 64, router_tiled_steps(N, ld, H));
         ks = ks > tiled ? ks : tiled;
     }

@@ -58,6 +58,21 @@ def test_router_split_partials(N, H, E, splits):
     assert _lib.lib().yvmoe_router_workspace_bytes(N, _lib.ACT_BF16, ctypes.byref(r)) == want
 
 
+@pytest.mark.parametrize("tokens", [0, 16, 300, 5000])
+@pytest.mark.parametrize("act", [_lib.ACT_F32, _lib.ACT_BF16])
+@pytest.mark.parametrize("hidden", [0, 32, 63, 96])
+def test_sizes_for_a_hidden_the_router_gemm_rejects(hidden, act, tokens):
+    """Routing from given logits never reads the hidden size, so its workspace can be asked for
+    with any (no split partial sums there), and the GEMM refuses it with an error code."""
+    l = _lib.lib()
+    r = _lib.Router(8, hidden, 2, 1, 0, 0, 1.0, 1, None, None, None, None)
+    ld = 16 + (3 if act == _lib.ACT_BF16 else 1) * _lib.PREDICTOR_DIM
+    assert l.yvmoe_router_workspace_bytes(tokens, act, ctypes.byref(r)) == 0
+    assert l.yvmoe_workspace_bytes(tokens, act, ctypes.byref(r), None) >= tokens * ld * 4
+    rc = l.yvmoe_router_logits(1, act, tokens, ctypes.byref(r), 1, ld, 1, 1 << 30, None)
+    assert rc == (_lib.YVMOE_ERR_SHAPE if tokens else 0)
+
+
 @pytest.mark.parametrize("E,k,code", [(0, 1, _lib.YVMOE_ERR_SHAPE), (257, 2, _lib.YVMOE_ERR_SHAPE),
                                       (8, 9, _lib.YVMOE_ERR_SHAPE), (8, 0, _lib.YVMOE_ERR_SHAPE),
                                       (64, 17, _lib.YVMOE_ERR_SHAPE)])
