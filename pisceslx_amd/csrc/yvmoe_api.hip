@@ -122,8 +122,9 @@ int32_t yvmoe_router_logits(const void* x, int32_t act_dtype, int32_t n_tokens,
     const size_t need = router_partials_bytes(n_tokens, router->num_experts, act_dtype, router->hidden);
     YV_REQUIRE(need == 0 || (workspace != nullptr && workspace_bytes >= need), YVMOE_ERR_WORKSPACE,
                "workspace %zu bytes, need %zu", workspace_bytes, need);
-    return router_gemm_launch(x, act_dtype, n_tokens, router, logits_out, ld,
-                              need ? (float*)workspace : nullptr, (hipStream_t)stream);
+    return router_gemm_launch(x, act_dtype, n_tokens, router, logits_out, ld, (float*)workspace,
+                              router_split(n_tokens, router->num_experts, act_dtype, router->hidden),
+                              (hipStream_t)stream);
 }
 
 int32_t yvmoe_route(const float* logits, int32_t ld, const float* predictor, int32_t n_tokens,
@@ -260,11 +261,13 @@ int32_t yvmoe_combine(const void* y, int32_t act_dtype, int32_t n_tokens, int32_
                           out, shared_out, (hipStream_t)stream);
 }
 
+// fewer_splits: the workspace need not hold more than the partial sums of router splits of one
+// length (router_even_partials_bytes); the router then takes as many splits as there is room for.
 static int32_t forward_run(const void* x, int32_t act_dtype, int32_t n_tokens,
-                      const yvmoe_router* router, const yvmoe_expert_weights* experts,
-                      const float* mix, const void* skip, void* out, void* shared_out,
-                      yvmoe_routing* routing, void* workspace, size_t workspace_bytes,
-                      void* stream, bool may_drop_split) {
+                           const yvmoe_router* router, const yvmoe_expert_weights* experts,
+                           const float* mix, const void* skip, void* out, void* shared_out,
+                           yvmoe_routing* routing, void* workspace, size_t workspace_bytes,
+                           void* stream, bool fewer_splits) {
     clear_error();
     int rc = check_router(router, act_dtype);
     if (rc) return rc;
@@ -277,9 +280,10 @@ static int32_t forward_run(const void* x, int32_t act_dtype, int32_t n_tokens,
                router->num_experts, router->hidden, experts->num_routed, experts->hidden);
     YV_REQUIRE(n_tokens >= 0, YVMOE_ERR_ARG, "n_tokens=%d < 0", n_tokens);
     size_t need = yvmoe_workspace_bytes(n_tokens, act_dtype, router, experts);
-    // without room for the router's split partial sums (the last region) it runs unsplit
-    const bool drop = may_drop_split && workspace_bytes < need;
-    if (drop) need -= router_partials_bytes(n_tokens, router->num_experts, act_dtype, router->hidden);
+    // all but the router's split partial sums (the last region)
+    const size_t fixed = need - router_partials_bytes(n_tokens, router->num_experts, act_dtype, router->hidden);
+    if (fewer_splits)
+        need = fixed + router_even_partials_bytes(n_tokens, router->num_experts, act_dtype, router->hidden);
     YV_REQUIRE(workspace != nullptr && workspace_bytes >= need, YVMOE_ERR_WORKSPACE,
                "workspace %zu bytes, need %zu", workspace_bytes, need);
     YV_REQUIRE(n_tokens == 0 || (x && out), YVMOE_ERR_ARG, "NULL pointer");
@@ -294,17 +298,18 @@ static int32_t forward_run(const void* x, int32_t act_dtype, int32_t n_tokens,
     float* logits = (float*)(ws + route_ws(N, E, k).bytes +
                              ffn_ws(N, k, E, experts->num_shared, experts->ffn, act_dtype).bytes);
     void* y = (char*)logits + align_up((size_t)N * ld * 4, 256);
-    float* partials = drop ? nullptr : (float*)((char*)y + y_bytes(N, k, experts->num_shared, experts->hidden, act_dtype));
+    float* partials = (float*)((char*)y + y_bytes(N, k, experts->num_shared, experts->hidden, act_dtype));
     // The routing's top-k kernels sum the router's split-K partial sums themselves (in split
     // order, as the reduction of yvmoe_router_logits does), so the sums need no launch of their
     // own (above kSmallRouteTok tokens up to kFoldSplits splits: more, read per logit, measured
     // slower than the reduction launch); for small batches the fused routing kernel also builds
     // the expert GEMM tile table.
     const bool small = N > 0 && N <= kSmallRouteTok;
-    const int ks = router_ksplit(N, E, act_dtype, router->hidden);
-    const bool split = N > 0 && ks > 1 && !drop && (small || ks <= kFoldSplits);
+    const RouterSplit rs = router_split(N, E, act_dtype, router->hidden, workspace_bytes - fixed);
+    const int ks = rs.ks;
+    const bool split = N > 0 && ks > 1 && (small || ks <= kFoldSplits);
     if (N > 0) {
-        rc = router_gemm_launch(x, act_dtype, N, router, logits, ld, partials, st, !split);
+        rc = router_gemm_launch(x, act_dtype, N, router, logits, ld, partials, rs, st, !split);
         if (rc) return rc;
     }
     const float* lsrc = split ? partials : logits;
@@ -383,9 +388,10 @@ int32_t yvmoe_forward_static(const void* x, int32_t act_dtype, int32_t n_tokens,
     rc = check_experts(experts, act_dtype);
     if (rc) return rc;
     YV_REQUIRE(n_tokens >= 0, YVMOE_ERR_ARG, "n_tokens=%d < 0", n_tokens);
-    // the router's split partial sums are left out where only they would not fit
+    const int E = router->num_experts;
     const size_t need = yvmoe_workspace_bytes(n_tokens, act_dtype, router, experts) -
-                        router_partials_bytes(n_tokens, router->num_experts, act_dtype, router->hidden);
+                        router_partials_bytes(n_tokens, E, act_dtype, router->hidden) +
+                        router_even_partials_bytes(n_tokens, E, act_dtype, router->hidden);
     YV_REQUIRE(need <= (size_t)YVMOE_STATIC_SCRATCH_BYTES, YVMOE_ERR_WORKSPACE,
                "n_tokens=%d needs %zu bytes of scratch, more than the static %zu bytes of "
                "yvmoe_forward_static (use yvmoe_forward with a workspace)",

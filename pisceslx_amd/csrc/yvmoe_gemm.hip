@@ -2868,7 +2868,7 @@ int dense_partials_launch(const void* x, int act, int N, int K, const void* w, i
 }
 
 int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, float* out, int ld,
-                       float* partials, hipStream_t st, bool reduce) {
+                       float* partials, RouterSplit split, hipStream_t st, bool reduce) {
     GemmParams p{};
     p.A = x;
     p.lda = r->hidden;
@@ -2878,39 +2878,26 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
     p.ncols = router_ld(r->num_experts, act);
     p.ldo = ld;
     p.nrows = N;
-    const int ks = router_ksplit(N, r->num_experts, act, r->hidden);
-    if (router_tiled(act, N, p.ncols, r->hidden)) {
-        // large batches: the LDS-tiled MFMA form over (tile, column block, K split) items, the
-        // split partial sums reduced in split order
-        if (ks == 1 || partials == nullptr) {
-            p.kchunk = r->hidden;
-            p.out = out;
-            return tile_dispatch<EPI_F32>(YVMOE_W_BF16, p, ceil_div(N, TBM), st, "router_gemm");
-        }
-        p.kchunk = router_tiled_steps(N, p.ncols, r->hidden) * 64;
-        p.out = partials;
-        p.split_stride = (long long)N * ld;
-        int rc = tile_dispatch<EPI_F32>(YVMOE_W_BF16, p, ceil_div(N, TBM), st, "router_gemm");
-        if (rc || !reduce) return rc;
-        return reduce_splits_launch(partials, ks, (long long)N * ld, out, st, "router_reduce");
-    }
     // ks == 1 writes the logits themselves; else the partial sums, the last split's K range shorter
-    const bool direct = ks == 1 || partials == nullptr;
-    p.kchunk = direct ? r->hidden : router_split_steps(N, r->num_experts, act, r->hidden) * 64;
+    const int ks = split.ks;
+    const bool direct = ks == 1;
+    p.kchunk = direct ? r->hidden : split.steps * 64;
     p.out = direct ? out : partials;
     p.split_stride = direct ? 0 : (long long)N * ld;
-    const int nz = direct ? 1 : ks;
     int rc;
+    // large batches: the LDS-tiled MFMA form over (tile, column block, K split) items
     // 16-row tiles up to kSmallRouteTok tokens (the router operand, 2 MB at E = 64, stays in L2 for the
     // tiles that re-read it: 2.7 us less per decode step at 64 tokens than one 64-row tile; the 138
     // MB YvMoEGate projection keeps 64-row tiles, which measured faster; layer at 128 tokens 226 ->
     // 223 us against 64-row tiles without LDS), 64-row tiles above
-    if (act == YVMOE_ACT_BF16)
+    if (router_tiled(act, N, p.ncols, r->hidden))
+        rc = tile_dispatch<EPI_F32>(YVMOE_W_BF16, p, ceil_div(N, TBM), st, "router_gemm");
+    else if (act == YVMOE_ACT_BF16)
         rc = N <= kSmallRouteTok
-                 ? stream_dispatch<EPI_F32, 4, 1, 1>(YVMOE_W_BF16, p, ceil_div(N, 16), st, "router_gemm", nz)
-                 : stream_dispatch<EPI_F32, 1, 1, 4, YV_DPF>(YVMOE_W_BF16, p, ceil_div(N, 64), st, "router_gemm", nz);
+                 ? stream_dispatch<EPI_F32, 4, 1, 1>(YVMOE_W_BF16, p, ceil_div(N, 16), st, "router_gemm", ks)
+                 : stream_dispatch<EPI_F32, 1, 1, 4, YV_DPF>(YVMOE_W_BF16, p, ceil_div(N, 64), st, "router_gemm", ks);
     else
-        rc = gemm_dispatch(p, ceil_div(N, kTileRows), direct && p.ncols % 32 == 0 ? 2 : 1, nz, st, "router_gemm");
+        rc = gemm_dispatch(p, ceil_div(N, kTileRows), direct && p.ncols % 32 == 0 ? 2 : 1, ks, st, "router_gemm");
     if (rc || direct || !reduce) return rc;
     return reduce_splits_launch(partials, ks, (long long)N * ld, out, st, "router_reduce");
 }

@@ -102,12 +102,17 @@ inline int router_split_steps(int N, int E, int act, int H) {
     while (ks * 2 <= most && (wgs * ks * 2 <= 512 || most == kFoldSplits) && H / (ks * 2) >= 128) ks *= 2;
     return ceil_div(H / 64, ks);
 }
-// (H < 64: sizes are asked for before a shape is checked, and routing alone never reads it.)
-inline int router_ksplit(int N, int E, int act, int H) {
-    if (H < 64) return 1;
-    const int ld = router_ld(E, act);
-    if (router_tiled(act, N, ld, H)) return ceil_div(H / 64, router_tiled_steps(N, ld, H));
-    return ceil_div(H / 64, router_split_steps(N, E, act, H));
+// (H < 64: sizes are asked for before a shape is checked, and routing alone never reads it.) Fewer
+// splits, longer ones, where their partial sums would not fit in room bytes.
+struct RouterSplit {
+    int steps, ks;
+};
+inline RouterSplit router_split(int N, int E, int act, int H, size_t room = ~(size_t)0) {
+    if (H < 64) return {0, 1};
+    const int ld = router_ld(E, act), nks = H / 64;
+    int steps = router_tiled(act, N, ld, H) ? router_tiled_steps(N, ld, H) : router_split_steps(N, E, act, H);
+    while (steps < nks && align_up((size_t)ceil_div(nks, steps) * N * ld * 4, 256) > room) ++steps;
+    return {steps, ceil_div(nks, steps)};
 }
 
 // Dense fp32-output GEMMs of more than 64 rows with bf16 operands, 256-multiple columns and
@@ -142,14 +147,27 @@ inline int dense_splits(int act, int N, int ncols, int K) {
 
 // Room for the split partial sums: of the tiled form's splits too where the streaming form, which
 // has fewer, runs (so a workspace never has to be larger than for that form).
+inline int router_tiled_splits(int N, int E, int act, int H) {  // 1 where that form never runs
+    if (act != YVMOE_ACT_BF16 || N <= kSmallRouteTok || H < 64 || H % 64 != 0) return 1;
+    return ceil_div(H / 64, router_tiled_steps(N, router_ld(E, act), H));
+}
+inline size_t router_splits_bytes(int ks, int N, int E, int act) {
+    return ks > 1 ? align_up((size_t)ks * N * router_ld(E, act) * 4, 256) : 0;
+}
 inline size_t router_partials_bytes(int N, int E, int act, int H) {
-    const int ld = router_ld(E, act);
-    int ks = router_ksplit(N, E, act, H);
-    if (act == YVMOE_ACT_BF16 && N > kSmallRouteTok && H >= 64 && H % 64 == 0) {
-        const int tiled = ceil_div(H / 64, router_tiled_steps(N, ld, H));
-        ks = ks > tiled ? ks : tiled;
+    const int ks = router_split(N, E, act, H).ks, tiled = router_tiled_splits(N, E, act, H);
+    return router_splits_bytes(ks > tiled ? ks : tiled, N, E, act);
+}
+// The same with splits of one length only: what the static scratch's limit on the batch counts, so
+// that it does not move with the number of unequal splits (which yield to the room there is).
+inline size_t router_even_partials_bytes(int N, int E, int act, int H) {
+    int ks = router_tiled_splits(N, E, act, H);
+    if (act != YVMOE_ACT_BF16 || N <= kSmallRouteTok) {
+        const int wgs = ceil_div(N > 0 ? N : 1, 64) * ceil_div(router_ld(E, act), 64);
+        while (ks * 2 <= YV_ROUTER_KS_MAX && wgs * ks * 2 <= 512 && H % (ks * 2 * 64) == 0 && H / (ks * 2) >= 128)
+            ks *= 2;
     }
-    return ks > 1 ? align_up((size_t)ks * N * ld * 4, 256) : 0;
+    return router_splits_bytes(ks, N, E, act);
 }
 
 // Upper bound on the number of GEMM tiles of tile_rows rows over all segments.
@@ -356,10 +374,11 @@ inline bool route_small_fixed(int N) { return N > 0 && N <= kSmallRouteTok; }
 int dispatch_route_launch(const int64_t* idx, const unsigned short* w_bf16, float* w32, int N,
                           int E, int k, int* counts, int* offsets, int* perm, int* pos,
                           int* invalid, int* cap_scratch, char* ws, hipStream_t st);
-// GEMMs and combine (yvmoe_gemm.hip). With reduce = false the router GEMM leaves its split-K
-// partial sums in partials (when it splits) for the routing kernel to reduce.
-int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, float* out,
-                       int ld, float* partials, hipStream_t st, bool reduce = true);
+// GEMMs and combine (yvmoe_gemm.hip). The router GEMM's K splits are the caller's
+// router_split(). With reduce = false it leaves their partial sums in partials (when it splits) for
+// the routing kernel to reduce.
+int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, float* out, int ld,
+                       float* partials, RouterSplit split, hipStream_t st, bool reduce = true);
 // Rows per tile of the expert GEMMs for this batch and layer, and the tile table's location
 // in the workspace.
 int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf);

@@ -73,6 +73,23 @@ def test_sizes_for_a_hidden_the_router_gemm_rejects(hidden, act, tokens):
     assert rc == (_lib.YVMOE_ERR_SHAPE if tokens else 0)
 
 
+@pytest.mark.parametrize("H,E,F,k,S,act,tokens", [
+    (4096, 64, 1408, 6, 2, _lib.ACT_BF16, 636), (4096, 64, 1408, 6, 2, _lib.ACT_F32, 363),
+    (1024, 8, 2816, 2, 1, _lib.ACT_BF16, 2465), (4096, 8, 4096, 2, 0, _lib.ACT_BF16, 1430),
+    (3008, 64, 1344, 6, 2, _lib.ACT_F32, 480),  # 47 k-steps: no equal splits, so none count
+])
+def test_static_scratch_refuses_from_the_same_batch_on(H, E, F, k, S, act, tokens):
+    """The first batch that yvmoe_forward_static refuses: one for which the scratch lacks the room
+    for the partial sums of equal router splits. (Refused before any device call.)"""
+    l = _lib.lib()
+    r = _lib.Router(E, H, k, 1, 0, 0, 1.0, 1, None, None, None, None)
+    e = _lib.ExpertWeights(_lib.W_BF16 if act == _lib.ACT_BF16 else _lib.W_F32, E, S, H, F, 1, 1, 1, None, None, None)
+    o = _lib.Routing(1, 1, 1, 1, 1, 1, 1)
+    rc = l.yvmoe_forward_static(1, act, tokens, ctypes.byref(r), ctypes.byref(e), 1, None, 1, 1, ctypes.byref(o), None)
+    assert rc == _lib.YVMOE_ERR_WORKSPACE
+    assert b"static" in l.yvmoe_last_error()
+
+
 @pytest.mark.parametrize("E,k,code", [(0, 1, _lib.YVMOE_ERR_SHAPE), (257, 2, _lib.YVMOE_ERR_SHAPE),
                                       (8, 9, _lib.YVMOE_ERR_SHAPE), (8, 0, _lib.YVMOE_ERR_SHAPE),
                                       (64, 17, _lib.YVMOE_ERR_SHAPE)])
