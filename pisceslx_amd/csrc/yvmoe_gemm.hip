@@ -660,7 +660,8 @@ __global__ __launch_bounds__(64 * WV) void gemm_stream_kernel(GemmParams p, int 
 // no barrier in the loop). The four partial sums meet in LDS in wavefront order.
 // Measured (FFN, against the weight-streaming form): H 4096, 64 experts of 1408, 6 + 2 per token, 1
 // token int8 48 -> 34 us, int4 56 -> 33, fp8 49 -> 32, bf16 58 -> 48; H 1024, 8 experts of 2816, 16
-// tokens int8 43 -> 28 us.
+// tokens int8 43 -> 28 us. (The one token's experts were read by the calls before; with tokens whose
+// experts were not, the layer gains 29 % as well: 64.4 -> 49.6 us.)
 template <int WF, int EPI>
 __global__ __launch_bounds__(256, 2) void gemm_few_kernel(GemmParams p, int ngroups) {
     typedef BLoad<WF> BL;
@@ -2937,6 +2938,36 @@ int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf) {
     return 128;
 }
 
+// Which GEMMs of a batch on 16-row tiles take the few-token form: bit 0 gate/up, bit 1 down. It pays
+// while the streaming form's work-groups (32 h or 64 output columns of a tile each) leave CUs
+// short of loads in flight, so the lines are drawn by that count, over the experts that a batch of
+// independent choices is expected to touch. It reads a shared expert's weights once per 16 rows,
+// the streaming form once per 64, so past those lines only where that costs little and an expert
+// holds a few rows. Measured (FFN, the GEMM streaming -> on the few-token form, by streaming
+// work-groups):
+// * gate/up, int8 H 4096, 64 experts of 1408, 6 + 2 per token: 352 52 -> 38 us, 808 70 -> 66, 1950 133 ->
+//   132, 2636 170 -> 174 (int4 58 -> 39, 79 -> 65, 134 -> 127, 170 -> 167; fp8 52 -> 38, 70 -> 65, 138 -> 131,
+//   168 -> 174); H 1024, 8 experts of 2816: 264 39 -> 35, 880 49 -> 49.
+// * gate/up, bf16 (its streams stay short of loads longer): the same layer 352 62 -> 53, 1950 249 -> 235,
+//   2871 339 -> 330, 3153 365 -> 369.
+// * down, int8: H 1024, 8 experts of 2816 160 50 -> 32; H 4096, F 1408 512 52 -> 51, 1175 70 -> 71, 2837 133 ->
+//   137; H 2048, F 256 (four k-steps for four wavefronts) 288 26 -> 25, 964 29 -> 30, 2670 38 -> 45. fp8 H
+//   7168, F 1024: 1970 93 -> 89, 3385 124 -> 123. bf16 H 4096, F 4096: 1010 264 -> 255; F 1408 3376 292 -> 287.
+// * shared rows: int8 top-1 of 256 experts and 2 shared, H 2048, F 1024, 102 tokens (14 of 99 tiles are
+//   shared): gate/up 105 -> 117.
+int ffn_few_forms(int N, int k, int E, int S, int H, int F, int wf) {
+    const double routed = E * (1.0 - std::pow(std::max(0.0, 1.0 - (double)k / E), N));
+    const double tiles = routed + (double)S * ceil_div(N, 16);
+    const double up = tiles * F / 32, down = tiles * H / 64;  // streaming work-groups
+    const bool bf16 = wf == YVMOE_W_BF16;
+    const bool rereads = 16.0 * S * (ceil_div(N, 16) - ceil_div(N, 64)) > tiles;
+    const bool more = !rereads && ((long long)N * k < (bf16 ? 4LL : 3LL) * E || (bf16 && S == 0));
+    const bool few_up = up <= std::max(896, bf16 ? H / 4 : 3 * H / 16) || (more && up <= (bf16 ? H : 5 * H / 8));
+    const int most = H < 4096 ? (bf16 ? 0 : F) : bf16 ? 4096 : wf == YVMOE_W_FP8 ? 2560 : F;
+    const bool few_down = down <= 768 || (more && down <= most);
+    return (few_up ? 1 : 0) | (few_down ? 2 : 0);
+}
+
 TileTable ffn_tile_table(int N, int k, int E, int S, int H, int F, int act, int wf, int tile_rows, char* ws) {
     const RouteWs RL = route_ws(N, E, k);
     const FfnWs FL = ffn_ws(N, k, E, S, F, act);
@@ -2977,16 +3008,7 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
     // every tile of the main table holds a row
     const int T = (int)std::min<long long>(max_tiles(N, k, E, S, tile_rows),
                                            (long long)N * k + (long long)S * ceil_div(N, tile_rows));
-    // a few tokens: by the mean rows per expert (from where the streaming form's work-groups fill
-    // the chip; H 4096, 64 experts, 4 / 6 / 8 tokens: int8 69 / 87 / 113 us there, 67 / 89 / 114 on
-    // the few-token form; 8 / 16: fp8 113 / 151 and 111 / 152; 32 / 64: bf16 350 / 367 and 338 / 371;
-    // H 5120, 128 experts, 8 / 16: int4 164 / 238 and 163 / 252), and always where a layer's experts
-    // are too few to fill it
-    const long long slots = (long long)N * k;
-    const bool few = streaming && (E * ceil_div(F, 32) <= 1024 ||
-                                   (w->format == YVMOE_W_BF16  ? slots < 3LL * E
-                                    : w->format == YVMOE_W_FP8 ? slots < E
-                                                               : 2 * slots < E));
+    const int few = streaming ? ffn_few_forms(N, k, E, S, H, F, w->format) : 0;
     if (!tiles_ready) {
         build_tiles_kernel<<<1, 512, 0, st>>>(routing->offsets, E, S, N, k, tile_rows, tt.fold, seg,
                                               tile_seg, tile_row0, ntiles, tt.light, tt.light_min,
@@ -3032,7 +3054,7 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
     p.ldo = F;
     p.kchunk = H;
     const bool f3 = act != YVMOE_ACT_BF16 && tile_rows == 128;
-    int rc = few ? few_dispatch<EPI_SWIGLU>(wf, p, T, st, "expert_gemm1")
+    int rc = (few & 1) ? few_dispatch<EPI_SWIGLU>(wf, p, T, st, "expert_gemm1")
            : f3 ? f32x3_dispatch<EPI_SWIGLU>(p, T, st, "expert_gemm1")
            : mid ? mid_dispatch<EPI_SWIGLU>(wf, p, T, tile_rows, st, "expert_gemm1")
            : tiled ? tile_dispatch<EPI_SWIGLU>(wf, p, T, st, "expert_gemm1", tt.fold > 0)
@@ -3067,7 +3089,7 @@ int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_w
         if (rc != YVMOE_OK || tt.light == 0) return rc;
         return light_launch(p, std::integral_constant<int, EPI_DOWN>{}, "expert_gemm2_light");
     }
-    if (few) return few_dispatch<EPI_DOWN>(wf, p, T, st, "expert_gemm2");
+    if (few & 2) return few_dispatch<EPI_DOWN>(wf, p, T, st, "expert_gemm2");
     if (f3) return f32x3_dispatch<EPI_DOWN>(p, T, st, "expert_gemm2");
     if (mid) return mid_dispatch<EPI_DOWN>(wf, p, T, tile_rows, st, "expert_gemm2");
     return streaming ? (S > 0

@@ -382,6 +382,7 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
 // Rows per tile of the expert GEMMs for this batch and layer, and the tile table's location
 // in the workspace.
 int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf);
+int ffn_few_forms(int N, int k, int E, int S, int H, int F, int wf);
 TileTable ffn_tile_table(int N, int k, int E, int S, int H, int F, int act, int wf, int tile_rows, char* ws);
 int expert_ffn_launch(const void* x, int act, int N, int k, const yvmoe_expert_weights* w,
                       const yvmoe_routing* routing, void* y, char* ws, hipStream_t st,

@@ -92,3 +92,9 @@ def check_ulps(got: torch.Tensor, want: torch.Tensor, label: str, max_ulps: int 
           f"differ={differ}/{d.numel()}", flush=True)
     assert n_ulps <= max_ulps, f"{label}: {n_ulps} ulps"
     assert cs >= 0.99999, f"{label}: cosine {cs}"
+
+
+def few_forms(tokens, top_k, experts, shared, hidden, ffn, fmt):
+    """The expert GEMMs that take the few-token form on 16-row tiles (bit 0 gate/up, bit 1 down)."""
+    from pisceslx_amd import _lib
+    return _lib.lib()["_ZN5yvmoe13ffn_few_formsEiiiiiii"](tokens, top_k, experts, shared, hidden, ffn, fmt)
