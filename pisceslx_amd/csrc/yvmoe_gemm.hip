@@ -2145,9 +2145,10 @@ __global__ __launch_bounds__(256, 3) void gemm_f32_stream_kernel(GemmParams p, i
 // owns 64 x 64 outputs and reads 24 KB for its 96 MFMAs. 48 KB of LDS: the work-groups of a CU
 // overlap one's split with another's MFMAs.
 //
-// A term of a non-finite (or all but overflowing) operand is NaN, so a work-group that ends with
-// a non-finite sum computes its tile again on the fp32 MFMAs (f32_tile_direct): infinities and
-// NaN come out as that form gives them. Operands below 2^-110 lose low bits to bf16's range.
+// A term of a non-finite (or all but overflowing) operand is NaN: outputs whose sum is not finite,
+// and only those, are computed again on the fp32 MFMAs (f32_block_direct), so infinities and NaN come
+// out as that form gives them and a row's bits depend on no other row. Operands below 2^-110 lose
+// low bits to bf16's range.
 // Error against 64 bits (relative 2-norm of the FFN's output): 1.11e-6 at H 1024, F 2816 and 1.63e-6
 // at H 4096, F 1408, where single fp32 MFMA sums over K have 1.29e-6 and 1.86e-6.
 // Measured (H 1024, 8 experts of 2816, 2 + 1 per token; FFN, against 64-row tiles on the fp32 MFMAs
@@ -2171,31 +2172,24 @@ __device__ __forceinline__ void split_bf16x3(const float (&v)[8], uint4 (&o)[3])
     o[2] = make_uint4(l[0], l[1], l[2], l[3]);
 }
 
-// The 64 x 16 NBW outputs of one wavefront on the fp32 MFMAs, straight from memory (the operands'
-// rows as the caller's lanes hold them): the accumulator layout of gemm_f32x3_kernel.
+// One 16-row block's 16 x 16 NBW outputs of a wavefront on the fp32 MFMAs, straight from memory (the
+// operands' rows as the caller's lanes hold them): the accumulator layout of gemm_f32x3_kernel.
 template <int NBW>
-__device__ __forceinline__ void f32_tile_direct(const float* const (&arow)[4], const float* const (&brow)[NBW],
-                                                int K, f32x4 (&acc)[4][NBW]) {
+__device__ __forceinline__ void f32_block_direct(const float* arow, const float* const (&brow)[NBW], int K,
+                                                 f32x4 (&acc)[NBW]) {
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < NBW; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int nb = 0; nb < NBW; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int k0 = 0; k0 < K; k0 += 16) {
-        float4 av[4], bv[NBW];
+        const float4 av = *(const float4*)(arow + k0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) av[i] = *(const float4*)(arow[i] + k0);
-#pragma unroll
-        for (int i = 0; i < NBW; ++i) bv[i] = *(const float4*)(brow[i] + k0);
-#pragma unroll
-        for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-            for (int nb = 0; nb < NBW; ++nb) {
-                f32x4& d = acc[mb][nb];
-                d = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[nb].x, av[mb].x, d, 0, 0, 0);
-                d = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[nb].y, av[mb].y, d, 0, 0, 0);
-                d = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[nb].z, av[mb].z, d, 0, 0, 0);
-                d = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[nb].w, av[mb].w, d, 0, 0, 0);
-            }
+        for (int nb = 0; nb < NBW; ++nb) {
+            const float4 bv = *(const float4*)(brow[nb] + k0);
+            f32x4& d = acc[nb];
+            d = __builtin_amdgcn_mfma_f32_16x16x4f32(bv.x, av.x, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x4f32(bv.y, av.y, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x4f32(bv.z, av.z, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x4f32(bv.w, av.w, d, 0, 0, 0);
+        }
     }
 }
 
@@ -2298,21 +2292,29 @@ __global__ __launch_bounds__(256, NBW == 4 ? 2 : 3) void gemm_f32x3_kernel(GemmP
             }
         }
     }
-    // a non-finite sum: the tile again on the fp32 MFMAs
-    bool bad = false;
+    // the sums that are not finite again on the fp32 MFMAs
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
+    for (int mb = 0; mb < 4; ++mb) {
+        bool bad = false;
 #pragma unroll
         for (int nb = 0; nb < NBW; ++nb)
 #pragma unroll
             for (int i = 0; i < 4; ++i) bad |= !(fabsf(acc[mb][nb][i]) < __builtin_inff());
-    if (__any(bad)) {
-        const float *ar[4], *br[NBW];
+        f32x4 direct[NBW];
+        const bool any = __any(bad);
+        if (any) {
+            const float* br[NBW];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ar[i] = a_row(wr * 4 + i) + g * 4;
+            for (int i = 0; i < NBW; ++i) br[i] = w_row(wc * NBW + i) + g * 4;
+            f32_block_direct<NBW>(a_row(wr * 4 + mb) + g * 4, br, K, direct);
+        }
 #pragma unroll
-        for (int i = 0; i < NBW; ++i) br[i] = w_row(wc * NBW + i) + g * 4;
-        f32_tile_direct<NBW>(ar, br, K, acc);
+        for (int nb = 0; nb < NBW; ++nb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float v = acc[mb][nb][i];
+                acc[mb][nb][i] = any && !(fabsf(v) < __builtin_inff()) ? direct[nb][i] : v;
+            }
     }
     // weights are the first operand: a lane holds row i16 of each row block and 4 consecutive
     // columns (4 g ..) of each weight block

@@ -37,14 +37,18 @@ def test_segment_edges(cuda, oracle, hidden, ffn, counts):
     assert routing.counts.cpu().tolist() == counts
 
 
+def _positive_experts(g, E, F, H, up_scale):
+    return [tuple(torch.rand(o, i, device="cuda", generator=g).clamp(min=0.1) * s
+                  for o, i, s in ((F, H, up_scale), (F, H, up_scale), (H, F, 1.0))) for _ in range(E)]
+
+
 @pytest.mark.parametrize("tokens", [40, 400])  # per expert: both forms
 def test_non_finite_and_largest_values(cuda, tokens):
     """Positive weights, so a row with +inf gives +inf and one with NaN gives NaN in every output;
     a row whose largest element rounds past bf16's range stays finite. Each poisons no other row."""
     H, F, E = 128, 192, 2
     g = torch.Generator(device="cuda").manual_seed(3)
-    ws = [tuple(torch.rand(o, i, device="cuda", generator=g).clamp(min=0.1) for o, i in ((F, H), (F, H), (H, F)))
-          for _ in range(E)]
+    ws = _positive_experts(g, E, F, H, 1.0)
     for w in ws:
         for m in w[:2]:
             m[:, 5] = 1e-38
@@ -67,3 +71,23 @@ def test_non_finite_and_largest_values(cuda, tokens):
     # and the product of two of them
     bound = (2 * H + F + 8) * 2.0 ** -24
     assert float(((out[keep].double() - want[keep]).abs() / want[keep]).max()) < bound
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan"), 3e38])
+def test_a_row_depends_on_no_other_row(cuda, bad):
+    """A row that is computed again because its sums are not finite changes no bit of the others."""
+    H, F, E, N = 128, 192, 2, 800
+    g = torch.Generator(device="cuda").manual_seed(6)
+    experts = pack_experts([tuple(torch.randn(o, i, device="cuda", generator=g) * 0.05
+                                  for o, i in ((F, H), (F, H), (H, F))) for _ in range(E)], E, _lib.W_F32)
+    x = torch.randn(N, H, device="cuda", generator=g)
+    idx = (torch.arange(N, device="cuda") % E).view(N, 1)
+    w = torch.ones(N, 1, device="cuda")
+    clean = yvf.dispatch(x, w, idx, experts)[0]
+    rows = [0, 7, 130, 799]
+    y = x.clone()
+    y[rows, 11] = bad
+    out = yvf.dispatch(y, w, idx, experts)[0]
+    keep = torch.ones(N, dtype=torch.bool, device="cuda")
+    keep[rows] = False
+    assert torch.equal(out[keep], clean[keep])
