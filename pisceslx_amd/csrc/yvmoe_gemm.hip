@@ -2142,18 +2142,22 @@ __global__ __launch_bounds__(256, 3) void gemm_f32_stream_kernel(GemmParams p, i
 // are loaded as fp32 into registers a chunk ahead, split once per work-group (5.5 VALU
 // instructions per element) and written to LDS as three planes of 16-row blocks in fragment
 // order (a lane's 16 bytes at 16 x lane: contiguous, conflict-free both ways); each wavefront
-// owns 64 x 64 outputs and reads 24 KB for its 96 MFMAs. 48 KB of LDS: the work-groups of a CU
-// overlap one's split with another's MFMAs.
+// owns 64 x 64 outputs and reads 24 KB for its 96 MFMAs. 48 KB of LDS and 168 VGPRs put three
+// work-groups on a CU, which overlap one's split with another's MFMAs.
 //
-// A term of a non-finite (or all but overflowing) operand is NaN: outputs whose sum is not finite,
-// and only those, are computed again on the fp32 MFMAs (f32_block_direct), so infinities and NaN come
-// out as that form gives them and a row's bits depend on no other row. Operands below 2^-110 lose
-// low bits to bf16's range.
+// Operands are split times 2^24 and the sums taken times 2^-48: the lowest term of the smallest
+// normal number is then a normal bf16 number, so no operand loses bits to bf16's range (unscaled, the
+// error grew to 5e-4 at 2^-124). A term of a non-finite operand, or of one that overflows in this
+// scale, is NaN: outputs whose sum is not finite, and only those, are computed again on the fp32
+// MFMAs (f32_block_direct), so infinities and NaN come out as that form gives them and a row's bits
+// depend on no other row.
 // Error against 64 bits (relative 2-norm of the FFN's output): 1.11e-6 at H 1024, F 2816 and 1.63e-6
 // at H 4096, F 1408, where single fp32 MFMA sums over K have 1.29e-6 and 1.86e-6.
 // Measured (H 1024, 8 experts of 2816, 2 + 1 per token; FFN, against 64-row tiles on the fp32 MFMAs
 // without LDS): 2,052 tokens 1361 -> 663 us (160 TFLOP/s; a large fp32 matrix product reaches
-// 154), 512 438 -> 300 us. A lone work-group on a CU takes about 3,000 cycles per chunk (load,
+// 154), 512 438 -> 300 us. The scale costs an instruction per element, a third work-group per CU gives
+// it back (layer, unscaled and two per CU / scaled / scaled and three: 719 / 723 / 707 us; H 4096, 64
+// experts of 1408, 1,500 tokens 3332 / 3376 / 3131). A lone work-group on a CU takes about 3,000 cycles per chunk (load,
 // split, write, barrier, read, MFMA in turn), which is what bounds small grids; a double-buffered
 // 8-wavefront form of 256 weight rows (one barrier per chunk) measured 702 us at 2,052 tokens.
 __device__ __forceinline__ void split_bf16x3(const float (&v)[8], uint4 (&o)[3]) {
@@ -2195,7 +2199,7 @@ __device__ __forceinline__ void f32_block_direct(const float* arow, const float*
 
 // NBW: 16-row weight blocks per wavefront, 4 (128 weight rows per work-group) or 2 (64).
 template <int EPI, int NBW>
-__global__ __launch_bounds__(256, NBW == 4 ? 2 : 3) void gemm_f32x3_kernel(GemmParams p, int ngroups) {
+__global__ __launch_bounds__(256, 3) void gemm_f32x3_kernel(GemmParams p, int ngroups) {
     constexpr bool SWIGLU = EPI == EPI_SWIGLU;
     constexpr int NBLK = 8 + 2 * NBW, PER = NBLK / 4;  // 16-row blocks of a chunk; per wavefront to stage
     constexpr int WCOLS = SWIGLU ? 16 * NBW / 2 : 16 * NBW;  // output columns per wavefront
@@ -2262,8 +2266,10 @@ __global__ __launch_bounds__(256, NBW == 4 ? 2 : 3) void gemm_f32x3_kernel(GemmP
         __syncthreads();  // every wavefront has read the chunk before
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
-            const float v[8] = {raw[j][0].x, raw[j][0].y, raw[j][0].z, raw[j][0].w,
-                                raw[j][1].x, raw[j][1].y, raw[j][1].z, raw[j][1].w};
+            float v[8] = {raw[j][0].x, raw[j][0].y, raw[j][0].z, raw[j][0].w,
+                          raw[j][1].x, raw[j][1].y, raw[j][1].z, raw[j][1].w};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] *= 0x1p24f;
             uint4 pl[3];
             split_bf16x3(v, pl);
 #pragma unroll
@@ -2292,7 +2298,7 @@ __global__ __launch_bounds__(256, NBW == 4 ? 2 : 3) void gemm_f32x3_kernel(GemmP
             }
         }
     }
-    // the sums that are not finite again on the fp32 MFMAs
+    // the sums out of the operands' scale; those that are not finite again on the fp32 MFMAs
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {
         bool bad = false;
@@ -2313,7 +2319,7 @@ __global__ __launch_bounds__(256, NBW == 4 ? 2 : 3) void gemm_f32x3_kernel(GemmP
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float v = acc[mb][nb][i];
-                acc[mb][nb][i] = any && !(fabsf(v) < __builtin_inff()) ? direct[nb][i] : v;
+                acc[mb][nb][i] = any && !(fabsf(v) < __builtin_inff()) ? direct[nb][i] : v * 0x1p-48f;
             }
     }
     // weights are the first operand: a lane holds row i16 of each row block and 4 consecutive

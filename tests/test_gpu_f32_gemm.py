@@ -73,6 +73,25 @@ def test_non_finite_and_largest_values(cuda, tokens):
     assert float(((out[keep].double() - want[keep]).abs() / want[keep]).max()) < bound
 
 
+@pytest.mark.parametrize("tokens", [40, 400])
+@pytest.mark.parametrize("x_exp,w_exp", [(-122, 100), (100, -122), (-60, 40)])
+def test_operands_at_the_ends_of_the_range(cuda, tokens, x_exp, w_exp):
+    """Operands next to fp32's smallest normal number keep all of their bits: positive terms only, so
+    the relative error of a sum of K is below K * 2^-24."""
+    H, F, E = 128, 192, 2
+    g = torch.Generator(device="cuda").manual_seed(5)
+    ws = _positive_experts(g, E, F, H, 2.0 ** w_exp)
+    N = tokens * E
+    x = torch.rand(N, H, device="cuda", generator=g).clamp(min=0.1) * 2.0 ** x_exp
+    idx = (torch.arange(N, device="cuda") % E).view(N, 1)
+    out = yvf.dispatch(x, torch.ones(N, 1, device="cuda"), idx, pack_experts(ws, E, _lib.W_F32))[0]
+    for e, w in enumerate(ws):
+        a, b, d = (m.double() for m in w)
+        xs = x[e::E].double()
+        want = (torch.nn.functional.silu(xs @ a.t()) * (xs @ b.t())) @ d.t()
+        assert float(((out[e::E].double() - want).abs() / want).max()) < (2 * H + F + 8) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan"), 3e38])
 def test_a_row_depends_on_no_other_row(cuda, bad):
     """A row that is computed again because its sums are not finite changes no bit of the others."""
