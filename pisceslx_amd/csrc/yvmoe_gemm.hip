@@ -2956,6 +2956,7 @@ int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf) {
 // * gate/up, int8 H 4096, 64 experts of 1408, 6 + 2 per token: 352 52 -> 38 us, 808 70 -> 66, 1950 133 ->
 //   132, 2636 170 -> 174 (int4 58 -> 39, 79 -> 65, 134 -> 127, 170 -> 167; fp8 52 -> 38, 70 -> 65, 138 -> 131,
 //   168 -> 174); H 1024, 8 experts of 2816: 264 39 -> 35, 880 49 -> 49.
+//   H 2048, 128 experts of 256, 8 + 1: 1040 54 -> 50, H 4096, 64 of 512, top-2: 1023 83 -> 85.
 // * gate/up, bf16 (its streams stay short of loads longer): the same layer 352 62 -> 53, 1950 249 -> 235,
 //   2871 339 -> 330, 3153 365 -> 369.
 // * down, int8: H 1024, 8 experts of 2816 160 50 -> 32; H 4096, F 1408 512 52 -> 51, 1175 70 -> 71, 2837 133 ->
@@ -2968,10 +2969,11 @@ int ffn_few_forms(int N, int k, int E, int S, int H, int F, int wf) {
     const double tiles = routed + (double)S * ceil_div(N, 16);
     const double up = tiles * F / 32, down = tiles * H / 64;  // streaming work-groups
     const bool bf16 = wf == YVMOE_W_BF16;
-    const bool rereads = 16.0 * S * (ceil_div(N, 16) - ceil_div(N, 64)) > tiles;
+    const bool rereads = 10.0 * S * (ceil_div(N, 16) - ceil_div(N, 64)) > tiles;
     const bool more = !rereads && ((long long)N * k < (bf16 ? 4LL : 3LL) * E || (bf16 && S == 0));
-    const bool few_up = up <= std::max(896, bf16 ? H / 4 : 3 * H / 16) || (more && up <= (bf16 ? H : 5 * H / 8));
-    const int most = H < 4096 ? (bf16 ? 0 : F) : bf16 ? 4096 : wf == YVMOE_W_FP8 ? 2560 : F;
+    const int base = H >= 2048 && (H < 4096 || (long long)N * k < 3LL * E) ? 1152 : 896;
+    const bool few_up = up <= std::max(base, bf16 ? H / 4 : 3 * H / 16) || (more && up <= (bf16 ? H : 5 * H / 8));
+    const int most = wf == YVMOE_W_INT4 ? 1024 : H < 4096 ? 0 : bf16 ? 4096 : wf == YVMOE_W_FP8 ? 2560 : 0;
     const bool few_down = down <= 768 || (more && down <= most);
     return (few_up ? 1 : 0) | (few_down ? 2 : 0);
 }

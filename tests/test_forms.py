@@ -11,13 +11,14 @@ I8, I4, F8, B16 = _lib.W_INT8, _lib.W_INT4, _lib.W_FP8, _lib.W_BF16
 
 @pytest.mark.parametrize("tokens,k,E,S,H,F,fmt,want", [
     # few work-groups on the streaming form: both GEMMs; then gate/up alone; then neither
-    (1, 6, 64, 2, 4096, 1408, I8, UP | DOWN), (3, 6, 64, 2, 4096, 1408, I8, UP | DOWN),
+    (1, 6, 64, 2, 4096, 1408, I8, UP | DOWN), (3, 6, 64, 2, 4096, 1408, I8, UP), (3, 6, 64, 2, 4096, 1408, F8, UP | DOWN),
     (4, 6, 64, 2, 4096, 1408, I8, UP), (16, 6, 64, 2, 4096, 1408, I8, UP), (32, 6, 64, 2, 4096, 1408, I8, 0),
     (16, 6, 64, 2, 4096, 1408, B16, UP | DOWN), (41, 6, 64, 2, 4096, 1408, B16, UP),
     (43, 6, 64, 2, 4096, 1408, B16, 0), (64, 6, 64, 2, 4096, 1408, I8, 0),
     (31, 2, 8, 1, 1024, 2816, I8, UP | DOWN), (31, 2, 8, 1, 1024, 2816, I4, UP | DOWN),
     # a down projection of four k-steps leaves the form early
-    (10, 8, 128, 1, 2048, 256, I8, UP), (104, 8, 128, 1, 2048, 256, I8, 0),
+    (2, 8, 128, 1, 2048, 256, I8, UP | DOWN), (10, 8, 128, 1, 2048, 256, I8, UP),
+    (20, 1, 64, 2, 4096, 1408, I8, UP),
     # many shared rows, which it would read once per 16: not beyond the first lines
     (15, 1, 256, 2, 2048, 1024, I8, UP | DOWN), (100, 1, 256, 2, 2048, 1024, I8, 0),
     (400, 1, 64, 2, 4096, 512, I8, 0), (64, 1, 64, 2, 4096, 1408, B16, 0), (250, 1, 256, 2, 2048, 1024, F8, 0),
