@@ -2911,9 +2911,21 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
     return reduce_splits_launch(partials, ks, (long long)N * ld, out, st, "router_reduce");
 }
 
-// Rows per tile of the expert GEMMs, which is also their form, by the mean rows per expert (slots
-// / E) and the weight format. fp32 activations: 64-row tiles on the fp32 MFMAs up to 48 rows (32 /
-// 50 / 64 rows: 166 / 226 / 287 us against 223 / 222 / 232), 128-row tiles on the bf16 MFMAs above.
+// Rows per tile of the expert GEMMs, which is also their form. The lines are drawn by the mean rows of
+// a segment (routed slots and shared rows over experts and shared experts), by the mean rows of an
+// expert (slots / E) and by the work-groups of the grid. Measured on FFN calls of 16 layer shapes
+// (hidden 640-7168, ffn 256-4096, 8-256 experts), even and Zipf-skewed loads; "mid" below is
+// gemm_mid_kernel.
+//
+// fp32 activations: 64-row tiles on the fp32 MFMAs, or 128-row tiles on the bf16 MFMAs (x3), whose
+// split costs the same for one row as for 16. x3 from 48 rows of an expert, and earlier where the
+// matrix rate and not the weights' stream bounds the 64-row tiles, that is with a wide K and many
+// work-groups: H 5120, 128 experts 4 / 12 rows 2809 / 3411 us on 64-row tiles, 2722 / 3048 x3; H 4096, 64
+// experts of 1408 12 / 24 rows 1187 / 1626 and 1295 / 1344; H 2048, 256 experts of 768 12 / 24 1303 / 1691
+// and 1427 / 1469; H 896, 256 experts 17 / 32 653 / 866 and 715 / 753; small grids later: H 4096, 64 experts of
+// 512 and 2 shared, 8 / 16 rows 594 / 889 and 619 / 648; H 2688, 64 of 640 24 / 36 532 / 670 and 618 / 642;
+// H 1024, 8 of 2816 36 / 48 186 / 228 and 216 / 229.
+//
 // bf16 activations:
 // * 16: weight streaming, up to 8 rows (int4: 4). It reads a tile's weights once per 16 rows;
 //   int8 6 / 9 / 12 rows: 191 / 205 / 220 us against 197 / 200 / 204 on the mid form (H 4096, 64
@@ -2934,8 +2946,15 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
 //   95 / 130 against 138 / 141).
 // * 256: the LDS-tiled form above that.
 int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf) {
-    const long long slots = (long long)N * k;
-    if (act != YVMOE_ACT_BF16) return slots < 48LL * E ? kTileRows : 128;
+    const long long slots = (long long)N * k, rows = slots + (long long)S * N;
+    const int segs = E + S;
+    // rows of a segment at least n
+    auto seg_rows = [&](int n) { return rows >= (long long)n * segs; };
+    if (act != YVMOE_ACT_BF16) {
+        const bool wide = (long long)segs * ceil_div(F, 64) >= 1024;
+        const int line = wide ? (H >= 5120 ? 8 : H >= 2048 ? 18 : 26) : H >= 4096 ? 24 : H >= 2048 ? 40 : 64;
+        return slots >= 48LL * E || seg_rows(line) ? 128 : kTileRows;
+    }
     if (slots < (wf == YVMOE_W_INT4 ? 4LL : 8LL) * E) return 16;
     const bool tiles = wf == YVMOE_W_INT8 || wf == YVMOE_W_BF16 || (H <= 8192 && F <= 8192);
     const long long most = wf == YVMOE_W_INT8 || wf == YVMOE_W_INT4 ? 150

@@ -98,3 +98,11 @@ def few_forms(tokens, top_k, experts, shared, hidden, ffn, fmt):
     """The expert GEMMs that take the few-token form on 16-row tiles (bit 0 gate/up, bit 1 down)."""
     from pisceslx_amd import _lib
     return _lib.lib()["_ZN5yvmoe13ffn_few_formsEiiiiiii"](tokens, top_k, experts, shared, hidden, ffn, fmt)
+
+
+def tile_rows(tokens, top_k, experts, shared, hidden, ffn, fmt):
+    """Rows per tile of the expert GEMMs, which is their form (16 streaming or few-token, 64 and 128
+    mid-sized, 256 LDS-tiled; fp32: 64 on the fp32 MFMAs, 128 on split operands)."""
+    from pisceslx_amd import _lib
+    act = _lib.ACT_F32 if fmt == _lib.W_F32 else _lib.ACT_BF16
+    return _lib.lib()["_ZN5yvmoe13ffn_tile_rowsEiiiiiiii"](act, tokens, top_k, experts, shared, hidden, ffn, fmt)

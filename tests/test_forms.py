@@ -3,10 +3,10 @@ library; no GPU needed)."""
 import pytest
 
 from pisceslx_amd import _lib
-from helpers import few_forms
+from helpers import few_forms, tile_rows
 
 UP, DOWN = 1, 2
-I8, I4, F8, B16 = _lib.W_INT8, _lib.W_INT4, _lib.W_FP8, _lib.W_BF16
+I8, I4, F8, B16, F32 = _lib.W_INT8, _lib.W_INT4, _lib.W_FP8, _lib.W_BF16, _lib.W_F32
 
 
 @pytest.mark.parametrize("tokens,k,E,S,H,F,fmt,want", [
@@ -27,3 +27,16 @@ I8, I4, F8, B16 = _lib.W_INT8, _lib.W_INT4, _lib.W_FP8, _lib.W_BF16
 ])
 def test_few_token_form(tokens, k, E, S, H, F, fmt, want):
     assert few_forms(tokens, k, E, S, H, F, fmt) == want
+
+
+MID, SMALL = (6, 64, 2, 4096, 1408), (2, 8, 1, 1024, 2816)  # k, E, S, H, F
+
+
+@pytest.mark.parametrize("layer,fmt,tokens,rows", [
+    # fp32
+    (SMALL, F32, 191, 64), (SMALL, F32, 192, 128), ((8, 128, 1, 5120, 1536), F32, 114, 64), ((8, 128, 1, 5120, 1536), F32, 115, 128),
+    ((6, 64, 2, 4096, 1408), F32, 148, 64), ((6, 64, 2, 4096, 1408), F32, 149, 128),
+])
+def test_rows_per_tile(layer, fmt, tokens, rows):
+    k, E, S, H, F = layer
+    assert tile_rows(tokens, k, E, S, H, F, fmt) == rows
