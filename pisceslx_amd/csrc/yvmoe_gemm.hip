@@ -2927,23 +2927,40 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
 // H 1024, 8 of 2816 36 / 48 186 / 228 and 216 / 229.
 //
 // bf16 activations:
-// * 16: weight streaming, up to 8 rows (int4: 4). It reads a tile's weights once per 16 rows;
-//   int8 6 / 9 / 12 rows: 191 / 205 / 220 us against 197 / 200 / 204 on the mid form (H 4096, 64
-//   experts); int4 6 rows: 190 against 171 (its 8-byte weight loads want the mid form's ring).
-// * 64: the mid form with 64-row tiles, which take less LDS and give more work-groups: int4 up to
-//   48 rows (its scale table costs 128-row tiles a third work-group per CU: 32 rows 228 us
-//   against 246), and any format up to 48 rows when 128-row tiles would leave the down
-//   projection under two work-groups per CU (H 1024, 8 experts of 16 / 32 rows: 48.5 / 48.7 us
-//   against 48.2 / 58.3).
-// * 128: the mid form, up to 150 rows for int8 and int4, 125 for fp8 and 112 for bf16 and for fp8
-//   layers of 128 experts and more, from where an expert's rows past 128 cost a second pass over its
-//   weights (H 4096, 64 experts, 96 / 131 / 159 rows: int8 386 / 546 / 690 us against 576 / 601 /
-//   686 on 256-row tiles, bf16 546 / 817 / 1038 against 646 / 653 / 680; fp8 H 2944, 64 experts, 122
-//   rows 305 against 389; H 7168, 256 experts, 109 / 128 rows 3205 / 4203 against 3429 / 3823, with
-//   a skewed load 3935 / 4313 against 3720 / 4004); any number of rows where the 256-row form's scale
-//   tables (fp8, int4: 8192 of K) do not hold the shape; and where 256-row tiles would be under two
-//   work-groups per CU (H 1024, 8 experts, 256 / 375 rows: bf16 100 / 150 us against 127 / 134, int8
-//   95 / 130 against 138 / 141).
+// * 16: weight streaming, up to 8 rows of a segment, 9 with shared experts. It reads a tile's weights once per 16 rows: int8 H
+//   4096, 64 experts of 1408, 6.5 / 10 / 13 rows of an expert 202 / 210 / 245 us, on 64-row mid tiles 203 /
+//   203 / 212. Up to 14 on the few-token form alone (H 1024, 8 experts of 2816, 7 / 10 / 13 rows of an
+//   expert: int8 32 / 34 / 36 us against 36 / 40 / 41). On grids of two to four mid work-groups per CU of
+//   many experts, which mid's three leave part empty, up to 12 (int8 H 1024, 64 of 640, 8 / 13 rows 42 / 44 us, mid 45 / 46; bf16 H 7168, 32 of 1024, 8 rows 253
+//   and 278). int4 streams suffer where a row of weights is a multiple of 1,024 wide (top-4 of 64 experts
+//   of 1024, 4 / 6 / 9 rows: H 4096 154 / 145 / 146 us, mid 136 / 124 / 120; H 2048 89 / 84 / 92 and 78 / 73 /
+//   72): 4 rows there; 7 else (H 4224 135 / 136 / 145 and 143 / 134 / 129; H 2688 94 / 93 / 101 and 96 / 90 /
+//   92); 14 on grids just past its two work-groups per CU (H 4096, 64 of 640, 9 / 13 rows 101 / 116 us and
+//   105 / 107; H 2688, 64 of 640, 4 / 13 rows 66 / 82 and 78 / 88) and for a short K (H 896, 256 of 768, 4 /
+//   10 / 13 rows 87 / 97 / 108 and 100 / 106 / 108; H 1152 alike).
+// * 64: mid with 64-row tiles, which take less LDS and give more work-groups: int4 up to 48 rows (its
+//   scale table costs 128-row tiles a third work-group per CU: 32 rows 228 us against 246), any format up
+//   to 16 rows of a segment on a small grid (int8 H 1024, 64 experts of 640, 13 rows 45 against 46 us; H 4096, 64 of
+//   512 and 2 shared, 8 rows 101 against 113) and up to 48 where 128-row tiles would leave the down
+//   projection under two work-groups per CU (H 1024, 8 experts of 16 / 32 rows: 48.5 / 48.7 us against
+//   48.2 / 58.3).
+// * 128: mid, from there to where an expert's rows past 128 cost a second pass over its weights: int8
+//   and int4 150 rows, fp8 125, bf16, which converts nothing, 112 (H 4096, 64 experts of 1408, 112 / 128 /
+//   150 rows: int8 451 / 562 / 679 us against 672 / 672 / 716 on 256-row tiles, int4 510 / 618 / 711 against
+//   685 / 629 / 699; bf16 96 / 112 / 128 rows 553 / 600 / 794 against 598 / 653 / 661; fp8 H 5120, 128 experts
+//   of 1536, 112 / 128 rows a ratio of 0.83 / 0.99, 64 experts of H 2688 and 1024 0.83 / 1.00). With 128
+//   experts and more a skewed load moves most rows to a few experts of many tiles each and leaves a tail
+//   of short ones, which the 256-row form hands to mid (tile_light): fp8 112, bf16 96 (bf16 96 rows,
+//   even / Zipf loads: H 7168, 256 experts 4300 / 5103 and 4316 / 4404 us, H 5120, 128 experts 1289 / 1510
+//   and 1340 / 1398; fp8 H 7168, 256 experts 112 rows 3207 / 3874 and 3549 / 3743). In bf16 shared experts
+//   alone may fill the 256-row tiles: 256 rows of a segment (H 4096, 64 experts of 512, top-1 and 2
+//   shared, 96 rows of an expert 419 and 386 us). Any number of rows where the 256-row form's scale
+//   tables (fp8, int4: 8192 of K) do not hold the shape, and, up to 400 rows, where the rounds of 256-row
+//   work-groups would leave a fifth of the chip idle over both GEMMs, in bf16 two fifths, near its lines
+//   a quarter (H 1024, 8 experts of 2816, 180 / 210 rows, a third in use: int8 97 / 99 us against 124 / 154,
+//   bf16 101 / 102 against 116 / 147; H 7168, 32 of 1024, 112 / 150 rows, 0.69 / 0.73 in use: bf16 392 / 744
+//   against 514 / 590, int8 150 rows 511 against 567; but H 4096, 64 of 512, whose gate/up has one
+//   work-group per CU and whose down has four, int8 150 / 180 rows 284 / 301 and 228 / 239).
 // * 256: the LDS-tiled form above that.
 int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf) {
     const long long slots = (long long)N * k, rows = slots + (long long)S * N;
@@ -2955,14 +2972,31 @@ int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf) {
         const int line = wide ? (H >= 5120 ? 8 : H >= 2048 ? 18 : 26) : H >= 4096 ? 24 : H >= 2048 ? 40 : 64;
         return slots >= 48LL * E || seg_rows(line) ? 128 : kTileRows;
     }
-    if (slots < (wf == YVMOE_W_INT4 ? 4LL : 8LL) * E) return 16;
-    const bool tiles = wf == YVMOE_W_INT8 || wf == YVMOE_W_BF16 || (H <= 8192 && F <= 8192);
-    const long long most = wf == YVMOE_W_INT8 || wf == YVMOE_W_INT4 ? 150
-                           : wf == YVMOE_W_FP8 && E < 128                   ? 125 : 112;
-    const long long items = (long long)max_tiles(N, k, E, S, TBM) * ceil_div(F, TBN / 2);
-    if (tiles && slots >= most * E && items > 448) return TBM;
-    if (slots <= 48LL * E && (wf == YVMOE_W_INT4 || (long long)E * ceil_div(H, 128) < 512)) return 64;
-    return 128;
+    const bool int4 = wf == YVMOE_W_INT4;
+    // mid's gate/up work-groups, with every expert in use
+    const long long grid = ((long long)E + (long long)S * ceil_div(N, 64)) * ceil_div(F, 64);
+    const bool small = grid <= 1024;
+    const bool past = E >= 32 && (int4 ? grid > 600 && grid < 740 : small && grid > 512);
+    const bool few = grid <= 448 && ffn_few_forms(N, k, E, S, H, F, wf) == 3;
+    const int line = few || (int4 && (past || H <= 1280)) ? 14
+                     : !int4                      ? (past ? 12 : S > 0 ? 9 : 8)
+                     : H >= 2048 && H % 1024 == 0 ? 4
+                                                  : 7;
+    if (!seg_rows(line)) return 16;
+    const bool bf16 = wf == YVMOE_W_BF16, many = E >= 128;
+    if (wf == YVMOE_W_INT8 || bf16 || (H <= 8192 && F <= 8192)) {
+        // k-steps' worth of 256-row work-groups of an even load against the rounds of 256 that they take
+        const double tiles = (double)E * ((slots + 256LL * E - 1) / (256LL * E)) + (double)S * ceil_div(N, TBM);
+        const double up = tiles * ceil_div(F, TBN / 2), down = tiles * ceil_div(H, TBN);
+        const double used = (up * H + down * F) / (256.0 * (std::ceil(up / 256) * H + std::ceil(down / 256) * F));
+        const int most = wf == YVMOE_W_FP8 ? (many ? 112 : 125) : !bf16 ? 150 : many && used >= 0.72 ? 96 : 112;
+        const bool enough = slots >= (long long)most * E || (bf16 && S > 0 && seg_rows(256));
+        const double least = bf16 ? (slots < 128LL * E ? 0.72 : 0.6) : 0.8;
+        const bool large = slots >= 400LL * E && max_tiles(N, k, E, S, TBM) * (long long)ceil_div(F, TBN / 2) > 448;
+        if (enough && (used >= least || large)) return TBM;
+    }
+    if (slots <= 48LL * E && (int4 || (long long)E * ceil_div(H, 128) < 512)) return 64;
+    return small && !seg_rows(16) ? 64 : 128;
 }
 
 // Which GEMMs of a batch on 16-row tiles take the few-token form: bit 0 gate/up, bit 1 down. It pays
