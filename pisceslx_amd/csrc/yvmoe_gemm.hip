@@ -2955,7 +2955,7 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
 //   and 1340 / 1398; fp8 H 7168, 256 experts 112 rows 3207 / 3874 and 3549 / 3743). In bf16 shared experts
 //   alone may fill the 256-row tiles: 256 rows of a segment (H 4096, 64 experts of 512, top-1 and 2
 //   shared, 96 rows of an expert 419 and 386 us). Any number of rows where the 256-row form's scale
-//   tables (fp8, int4: 8192 of K) do not hold the shape, and, up to 400 rows, where the rounds of 256-row
+//   tables (fp8, int4: 8192 of K) do not hold the shape, and, up to 256 rows, where the rounds of 256-row
 //   work-groups would leave a fifth of the chip idle over both GEMMs, in bf16 two fifths, near its lines
 //   a quarter (H 1024, 8 experts of 2816, 180 / 210 rows, a third in use: int8 97 / 99 us against 124 / 154,
 //   bf16 101 / 102 against 116 / 147; H 7168, 32 of 1024, 112 / 150 rows, 0.69 / 0.73 in use: bf16 392 / 744
@@ -2992,7 +2992,7 @@ int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf) {
         const int most = wf == YVMOE_W_FP8 ? (many ? 112 : 125) : !bf16 ? 150 : many && used >= 0.72 ? 96 : 112;
         const bool enough = slots >= (long long)most * E || (bf16 && S > 0 && seg_rows(256));
         const double least = bf16 ? (slots < 128LL * E ? 0.72 : 0.6) : 0.8;
-        const bool large = slots >= 400LL * E && max_tiles(N, k, E, S, TBM) * (long long)ceil_div(F, TBN / 2) > 448;
+        const bool large = slots > 256LL * E && max_tiles(N, k, E, S, TBM) * (long long)ceil_div(F, TBN / 2) > 448;
         if (enough && (used >= least || large)) return TBM;
     }
     if (slots <= 48LL * E && (int4 || (long long)E * ceil_div(H, 128) < 512)) return 64;

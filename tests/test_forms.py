@@ -58,3 +58,13 @@ MID, CFG5, SMALL = (6, 64, 2, 4096, 1408), (8, 256, 0, 7168, 2048), (2, 8, 1, 10
 def test_rows_per_tile(layer, fmt, tokens, rows):
     k, E, S, H, F = layer
     assert tile_rows(tokens, k, E, S, H, F, fmt) == rows
+
+
+@pytest.mark.parametrize("fmt", [I8, I4, F8, B16])
+@pytest.mark.parametrize("layer", [MID, CFG5, SMALL, (8, 128, 1, 5120, 1536), (2, 40, 1, 1024, 1024), (4, 32, 2, 7168, 1024),
+                                   (2, 64, 0, 4096, 512), (6, 64, 2, 2688, 640)])
+def test_rows_per_tile_grow_with_the_batch(layer, fmt):
+    """A larger batch never goes back to smaller tiles."""
+    k, E, S, H, F = layer
+    rows = [tile_rows(n, k, E, S, H, F, fmt) for n in range(1, 20000, 7)]
+    assert rows == sorted(rows)
