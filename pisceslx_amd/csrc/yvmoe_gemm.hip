@@ -1915,7 +1915,9 @@ __device__ __forceinline__ void mid_item(const GemmParams& p, int e, int row0, i
 // tiles of one expert read a column group's weights on one XCD, and an XCD's groups of a tile
 // run together on the tile's rows. Tiles run last to first, so the full ones do not end the
 // launch. (FFN at 64 experts of 47 rows: contiguous ranges of the items per XCD 348 us tile by
-// tile, 309 us group by group; 288 us in this order.)
+// tile, 309 us group by group; 288 us in this order.) A dense GEMM has one "expert"; with fewer groups
+// than XCDs its tiles take turns instead, so that no XCD is left out (gate call without HiCL, H 4096, 512
+// columns, 16,000 tokens 170 -> 150 us; 256 columns 165 -> 135).
 // NT: non-temporal weight loads, where (nearly) every weight is read by one tile only.
 template <int WF, int EPI, int MAXMRB, bool NT = true>
 __global__ __launch_bounds__(256, (MAXMRB == 8 ? 3 : 4) - (WF == YVMOE_W_INT4 ? 1 : 0)) void gemm_mid_kernel(GemmParams p, int ngroups) {
@@ -1928,7 +1930,8 @@ __global__ __launch_bounds__(256, (MAXMRB == 8 ? 3 : 4) - (WF == YVMOE_W_INT4 ? 
     if (tile < 0) return;
     const int e = EPI == EPI_F32 ? 0 : p.tile_seg[tile];
     const int row0 = EPI == EPI_F32 ? tile * MAXMRB * 16 : p.tile_row0[tile];
-    const int cgroup = ((x + e) & 7) + 8 * (local % per_tile);
+    const int turn = EPI != EPI_F32 ? e : ngroups < 8 ? tile : 0;
+    const int cgroup = ((x + turn) & 7) + 8 * (local % per_tile);
     if (cgroup >= ngroups) return;
     const int seg_end = min(EPI == EPI_F32 ? p.nrows : p.seg_start[e + 1], row0 + MAXMRB * 16);
     const int rows = seg_end - row0;
@@ -2849,9 +2852,11 @@ int dense_partials_launch(const void* x, int act, int N, int K, const void* w, i
         // up to 144 256 x 256 tiles, the mid-sized form: more work-groups in flight on the weights
         // (whole gate call, H 4096, 16,896 columns: 100 / 256 / 450 tokens 120 / 143 / 162 us on
         // 256-row tiles, 72 / 97 / 146; 700 tokens, 198 tiles: 179 and 247; H 2048, 700 tokens, 99
-        // tiles: 117 and 99). Non-temporal weight loads for a single row tile (100 tokens 79 -> 72 us;
-        // 300 tokens 122 -> 135).
-        if (ceil_div(N, TBM) * (ncols / TBN) <= 144) {
+        // tiles: 117 and 99), up to 96 tiles of less than 1,024 columns, whose row tiles share less (512
+        // columns: 12,000 / 16,000 tokens, 94 / 126 tiles, 125 / 145 us and 113 / 150; 256 columns: 24,000 /
+        // 30,000 tokens, 94 / 118 tiles, 156 / 166 and 155 / 192). Non-temporal weight loads for a single
+        // row tile (100 tokens 79 -> 72 us; 300 tokens 122 -> 135).
+        if (ceil_div(N, TBM) * (ncols / TBN) <= (ncols < 1024 ? 96 : 144)) {
             const int ngroups = ncols / 128;
             const unsigned items = 8u * ceil_div(N, 128) * ceil_div(ngroups, 8);
             if (N <= 128) gemm_mid_kernel<YVMOE_W_BF16, EPI_F32, 8><<<items, 256, 0, st>>>(p, ngroups);

@@ -88,6 +88,18 @@ def test_projection_of_mid_sized_batches(cuda, oracle, n):
     _check(g, x, oracle)
 
 
+@pytest.mark.parametrize("n", [65, 129, 130, 400, 1000])
+def test_projection_of_few_columns(cuda, oracle, n):
+    """A gate whose HiCL head is pruned projects on a few 256-column blocks: fewer column groups
+    than XCDs, over one to eight row tiles of the mid-sized form."""
+    g = _gate(512, 96, 6, scale_heads=True, seed=n)
+    with torch.no_grad():
+        g.sparse_gate_hicl.fill_(-10.0)
+    g.prune_routing_heads(0.05)
+    x = torch.randn(n, 1, 512, generator=torch.Generator().manual_seed(n)).to(torch.bfloat16).cuda()
+    _check(g, x, oracle, heads=("got", "soft_moe", "expert_orient"))
+
+
 def test_dg_ties_and_few_positives(cuda, oracle):
     H, E = 256, 8
     g = _gate(H, E, 2, scale_heads=True, seed=1)
