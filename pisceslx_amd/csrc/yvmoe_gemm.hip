@@ -1929,11 +1929,14 @@ __global__ __launch_bounds__(256, (MAXMRB == 8 ? 3 : 4) - (WF == YVMOE_W_INT4 ? 
     const int tile = nt - 1 - local / per_tile;  // dense fp32 output: one segment of nrows rows
     if (tile < 0) return;
     const int e = EPI == EPI_F32 ? 0 : p.tile_seg[tile];
-    const int row0 = EPI == EPI_F32 ? tile * MAXMRB * 16 : p.tile_row0[tile];
+    // dense: tiles of one height, which stay in step on the weights they share (gate call, H 4096, 16,896
+    // columns, against full tiles and a remainder: 129 / 257 / 400 tokens 85 -> 71, 112 -> 84, 132 -> 126 us)
+    const int height = EPI == EPI_F32 ? ((p.nrows + nt - 1) / nt + 15) / 16 * 16 : MAXMRB * 16;
+    const int row0 = EPI == EPI_F32 ? tile * height : p.tile_row0[tile];
     const int turn = EPI != EPI_F32 ? e : ngroups < 8 ? tile : 0;
     const int cgroup = ((x + turn) & 7) + 8 * (local % per_tile);
     if (cgroup >= ngroups) return;
-    const int seg_end = min(EPI == EPI_F32 ? p.nrows : p.seg_start[e + 1], row0 + MAXMRB * 16);
+    const int seg_end = min(EPI == EPI_F32 ? p.nrows : p.seg_start[e + 1], row0 + height);
     const int rows = seg_end - row0;
     if constexpr (MAXMRB == 8) {
         if (rows > 96) return mid_item<WF, EPI, 8, MAXMRB, NT>(p, e, row0, seg_end, cgroup, lds_a, lds_s);
@@ -2850,9 +2853,9 @@ int dense_partials_launch(const void* x, int act, int N, int K, const void* w, i
     p.kchunk = K / ks;
     if (dense_tiled(act, N, ncols, K)) {
         // up to 144 256 x 256 tiles, the mid-sized form: more work-groups in flight on the weights
-        // (whole gate call, H 4096, 16,896 columns: 100 / 256 / 450 tokens 120 / 143 / 162 us on
-        // 256-row tiles, 72 / 97 / 146; 700 tokens, 198 tiles: 179 and 247; H 2048, 700 tokens, 99
-        // tiles: 117 and 99), up to 96 tiles of less than 1,024 columns, whose row tiles share less (512
+        // (logits call, H 4096, 16,896 columns: 128 / 256 / 400 / 448 tokens 96 / 117 / 128 / 127 us on
+        // 256-row tiles, 69 / 82 / 126 / 116; H 7168, 300 tokens, 234 tiles: 262 and 316; H 2048, 700
+        // tokens, 102 tiles: 96 and 76), up to 96 tiles of less than 1,024 columns, whose row tiles share less (512
         // columns: 12,000 / 16,000 tokens, 94 / 126 tiles, 125 / 145 us and 113 / 150; 256 columns: 24,000 /
         // 30,000 tokens, 94 / 118 tiles, 156 / 166 and 155 / 192). Non-temporal weight loads for a single
         // row tile (100 tokens 79 -> 72 us; 300 tokens 122 -> 135).
