@@ -43,8 +43,9 @@ class YvRMSNorm(nn.Module):
 
     def norm_params(self):
         # straight from the parameter table where they stand there (not, say, parametrized): the
-        # attribute lookups of nn.Module take longer than the rest of this function
-        p = self._parameters
+        # attribute lookups of nn.Module take longer than the rest of this function; a subclass may
+        # define the attributes otherwise
+        p = self._parameters if type(self) is YvRMSNorm else {}
         weight = p["weight"] if "weight" in p else self.weight
         bias = p["bias"] if "bias" in p else self.bias
         return (weight.detach(), None if bias is None else bias.detach(), self.eps)
