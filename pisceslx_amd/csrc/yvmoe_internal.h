@@ -64,10 +64,13 @@ constexpr int kFoldSplits = 4;
 // that the (tile, column block, split) items spread over the 256 CUs. A batch of a few tiles needs
 // many splits there, whose reduction is a launch of its own (layer, H 4096, 64 experts, 300 / 700 /
 // 3,000 tokens: 299 / 382 / 1125 us tiled, 285 / 368 / 1110 streamed; H 1024, 8 experts, 500 tokens
-// 114 and 96).
+// 114 and 96). The streaming form reads the rows once per 64 columns: with more than six such groups
+// it ends sooner (H 7168, 160 experts of F 128, six groups, 3,072 tokens: 548 us tiled, 550 streamed; 256
+// experts, seven, 2,200 / 3,072 tokens: 466 / 569 and 460 / 580).
 constexpr int kStreamRouteTok = 3072;
 inline bool router_tiled(int act, int N, int ncols, int K) {
-    return act == YVMOE_ACT_BF16 && N > kStreamRouteTok && ncols % 16 == 0 && K % 64 == 0 && K > 0;
+    return act == YVMOE_ACT_BF16 && (N > kStreamRouteTok || (long)N * ceil_div(ncols, 64) > 6 * kStreamRouteTok) &&
+           ncols % 16 == 0 && K % 64 == 0 && K > 0;
 }
 
 // k-steps (of 64) per split of the tiled router GEMM: the choice with the least estimated time,

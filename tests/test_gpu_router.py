@@ -1,6 +1,6 @@
 """The router GEMM (yvmoe_router_logits) on the GPU against float64, across the shapes its
-forms take: the streaming form with 16 K splits up to 256 tokens; above, the LDS-tiled form with
-K splits chosen per shape, including a partial last column block (router operand widths
+forms take: the streaming form with up to 16 K splits up to 256 tokens and up to 4 above; for larger
+batches the LDS-tiled form with K splits chosen per shape, including a partial last column block (router operand widths
 Ep + 192 that are not multiples of 256) and splits whose last one is shorter.
 
 Every logit within 2e-4 * max(1, max |logit|) of x @ gate.weight^T computed in float64 from the
@@ -44,6 +44,8 @@ def _router(E, H, dev, seed):
     (258, 3008, 40),    # above the small-batch bound: splits of 12, the last of 11
     (3072, 320, 8),     # the streaming form's last size: 5 k-steps in splits of 3 and 2
     (3073, 1024, 64),   # and the tiled form's first
+    (2633, 320, 256),   # the same with seven 64-column groups
+    (2634, 320, 256),
 ])
 def test_router_logits_against_float64(cuda, N, H, E):
     gw, st = _router(E, H, cuda, seed=N + H + E)
