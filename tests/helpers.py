@@ -106,3 +106,44 @@ def tile_rows(tokens, top_k, experts, shared, hidden, ffn, fmt):
     from pisceslx_amd import _lib
     act = _lib.ACT_F32 if fmt == _lib.W_F32 else _lib.ACT_BF16
     return _lib.lib()["_ZN5yvmoe13ffn_tile_rowsEiiiiiiii"](act, tokens, top_k, experts, shared, hidden, ffn, fmt)
+
+
+def tile_rows_of(w):
+    """tile_rows of a workload's expert GEMMs."""
+    s = w.spec
+    return tile_rows(w.n_tokens, s.top_k, s.num_experts, s.num_shared, s.hidden, s.ffn, s.fmt)
+
+
+def few_forms_of(w):
+    """few_forms of a workload's expert GEMMs."""
+    s = w.spec
+    return few_forms(w.n_tokens, s.top_k, s.num_experts, s.num_shared, s.hidden, s.ffn, s.fmt)
+
+
+def forced_experts(counts, seed):
+    """The expert of each token, in an order of its own, such that expert e has counts[e] tokens."""
+    g = torch.Generator().manual_seed(seed)
+    N = sum(counts)
+    return torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))[torch.randperm(N, generator=g)]
+
+
+def forced_rows(spec, counts, seed=7):
+    """A workload whose expert e receives exactly counts[e] tokens (one-hot gate rows, top-1)."""
+    from pisceslx_amd.workloads import make_workload
+    N, E, H = sum(counts), len(counts), spec.hidden
+    w = make_workload(spec, device="cuda", lengths=[N])
+    x = torch.randn(N, H, generator=torch.Generator().manual_seed(seed + 1)) * 0.5
+    x[torch.arange(N), forced_experts(counts, seed)] += 8.0
+    gate = torch.zeros(E, H)
+    gate[torch.arange(E), torch.arange(E)] = 1.0
+    w.x, w.gate_weight = x.to(w.x.dtype).cuda(), gate.to(w.gate_weight.dtype).cuda()
+    return w
+
+
+def ends_of_segments(counts, seed=7, last=40):
+    """Tokens (sorted) in the first two and the last rows of every segment of forced_rows(spec,
+    counts, seed): an expert's rows keep the order of its tokens, a shared expert's too."""
+    import numpy as np
+    expert = forced_experts(counts, seed).numpy()
+    rows = [np.flatnonzero(expert == e) for e in range(len(counts))] + [np.arange(len(expert))]
+    return np.unique(np.concatenate([np.concatenate([r[:2], r[-last:]]) for r in rows]))

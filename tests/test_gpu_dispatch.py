@@ -78,7 +78,7 @@ def _check_dispatch(oracle, w, idx, wts, label, tokens=None, weight_dtype=torch.
     ("cfg2", {"n_tokens": 700}, 6),
     ("cfg4", {"n_tokens": 96}, 8),
     ("cfg5", {"n_tokens": 200, "num_experts": 32}, 8),
-    ("cfg5", {"n_tokens": 64, "num_experts": 32}, 8),   # fp8 weights on the streaming form
+    ("cfg5", {"n_tokens": 64, "num_experts": 32}, 8),   # fp8 weights, 16 rows of an expert: mid-sized form
     ("cfg5", {"n_tokens": 200, "num_experts": 32}, 12),  # the combine's second 8-slot chunk
     ("cfg5", {"n_tokens": 64, "num_experts": 32}, 16),   # the operator's largest k
     ("cfg2", {"n_tokens": 100}, 1),

@@ -8,31 +8,23 @@ from pisceslx_amd import _lib
 from pisceslx_amd import functional as yvf
 from pisceslx_amd.quant import pack_experts
 from pisceslx_amd.workloads import LayerSpec, make_workload
+from helpers import forced_rows, tile_rows_of
 from test_gpu_layer import _run_and_check
 
 pytestmark = pytest.mark.gpu
 
 
-def forced_rows(spec, counts):
-    N, E, H = sum(counts), len(counts), spec.hidden
-    w = make_workload(spec, device="cuda", lengths=[N])
-    g = torch.Generator().manual_seed(9)
-    expert = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(N, generator=g)]
-    x = torch.randn(N, H, generator=g) * 0.5
-    x[torch.arange(N), expert] += 8.0
-    gate = torch.zeros(E, H)
-    gate[torch.arange(E), torch.arange(E)] = 1.0
-    w.x, w.gate_weight = x.cuda(), gate.cuda()
-    return w
+FEW, FEWER = [0, 1, 15, 16, 17, 33, 48, 49, 64, 65], [0, 1, 15, 16, 17, 33]
+MANY = [0, 1, 16, 63, 64, 65, 80, 127, 128, 129, 200]
 
 
-@pytest.mark.parametrize("counts", [[0, 1, 15, 16, 17, 33, 48, 49, 64, 65],            # mean 31
-                                    [0, 1, 16, 63, 64, 65, 80, 127, 128, 129, 200]],  # mean 79
-                         ids=["few_rows", "many_rows"])
-@pytest.mark.parametrize("hidden,ffn", [(64, 64), (192, 320), (1024, 1088), (4160, 192)])
-def test_segment_edges(cuda, oracle, hidden, ffn, counts):
+@pytest.mark.parametrize("hidden,ffn,counts,rows", [
+    (64, 64, FEW, 64), (192, 320, FEW, 64), (1024, 1088, FEW, 64), (4160, 192, FEWER, 64), (4160, 192, FEW, 128),
+    (64, 64, MANY, 128), (192, 320, MANY, 128), (1024, 1088, MANY, 128), (4160, 192, MANY, 128)])
+def test_segment_edges(cuda, oracle, hidden, ffn, counts, rows):
     spec = LayerSpec("f32", hidden, ffn, len(counts), 1, 1, _lib.W_F32, torch.float32, fixed_shape_mode=True)
     w = forced_rows(spec, counts)
+    assert tile_rows_of(w) == rows
     _, _, routing = _run_and_check(oracle, w, label=f"f32 H={hidden} F={ffn} N={sum(counts)}")
     assert routing.counts.cpu().tolist() == counts
 

@@ -19,7 +19,7 @@ import torch
 from pisceslx_amd import functional as yvf
 from pisceslx_amd.workloads import make_workload, mix_weights, router_state
 
-from helpers import check_close, oracle_params
+from helpers import check_close, ends_of_segments, few_forms_of, forced_rows, oracle_params, tile_rows_of
 
 pytestmark = pytest.mark.gpu
 
@@ -73,7 +73,7 @@ def _run_and_check(oracle, w, skip=None, tokens=None, label=None):
     ("cfg3", {"n_tokens": 512}),
     ("cfg4", {"n_tokens": 384}),
     ("cfg5", {"n_tokens": 384, "num_experts": 32}),
-    ("cfg5", {"n_tokens": 64, "num_experts": 32}),       # fp8 weights on the streaming form
+    ("cfg5", {"n_tokens": 64, "num_experts": 32}),       # fp8 weights, 16 rows of an expert: mid-sized form
     ("cfg2", {"n_tokens": 1}),                             # one token: six one-row experts
     ("cfg2", {"n_tokens": 200}),                           # the small-batch routing at 200 tokens
 ])
@@ -112,7 +112,7 @@ def test_cfg5_full_size_sampled_tokens(cuda, oracle):
 
 
 def test_cfg4_full_size_tiled_int4_sampled_tokens(cuda, oracle):
-    """cfg4 at its full size (4344 tokens, N*k >= 64*E): the LDS-tiled form with int4 weights
+    """cfg4 at its full size (4344 tokens, 271 rows per expert): the LDS-tiled form with int4 weights
     (group scales staged in LDS, 512-byte weight blocks), checked on sampled tokens."""
     w = make_workload("cfg4", device="cuda")
     rng = np.random.default_rng(1)
@@ -130,70 +130,55 @@ def test_bf16_and_small_shapes(cuda, oracle):
 
 
 def test_bf16_tiled_prefill_shapes(cuda, oracle):
-    # unquantized bf16 experts with many rows per expert (the 128-row LDS-tiled GEMMs), segment
+    # unquantized bf16 experts with many rows per expert (the mid-sized form's 128-row tiles), segment
     # ends inside tiles
     from pisceslx_amd import _lib
     from pisceslx_amd.workloads import LayerSpec
     spec = LayerSpec("tiled_bf16", 256, 384, 4, 2, 1, _lib.W_BF16, torch.bfloat16)
     w = make_workload(spec, device="cuda", lengths=[200, 77, 3])
+    assert tile_rows_of(w) == 128
     _run_and_check(oracle, w)
 
 
 @pytest.mark.parametrize("fmt,hidden", [("int8", 256), ("int4", 256), ("fp8", 256), ("bf16", 256),
                                         ("int4", 6144)])
 def test_tiled_folded_remainders(cuda, oracle, fmt, hidden):
-    """Expert segments of 256, 257, 272, 273, 288, 289, 320, 321, 544 and 16 rows and a shared
-    segment of 2836 rows (11 x 256 + 20), forced through one-hot gate rows: the LDS-tiled form
-    folds a remainder of 1 .. 32 rows into the segment's last full tile (a second launch runs
-    those tiles; 17+ rows reach the second wavefront row's block), sends remainders of 33 .. 64
-    rows and a segment of 16 rows to the weight-streaming form's 64-row light tiles, and keeps
-    65 rows as a tile of its own. int4 at hidden 6144 takes the gate/up form for K > 5120
-    (2-stage ring beside the 64-group scale table)."""
+    """Expert segments of 256, 257, 272, 273, 288, 289, 320, 321, 544 and 16 rows, seven of each,
+    and a shared segment of 19852 rows (77 x 256 + 140), forced through one-hot gate rows: the
+    LDS-tiled form folds a remainder of 1 .. 32 rows into the segment's last full tile (a second
+    launch runs those tiles; 17+ rows reach the second wavefront row's block), sends remainders of
+    33 .. 64 rows and a segment of 16 rows to the mid-sized form's light tiles, and keeps 65 rows as
+    a tile of its own. int4 at hidden 6144 takes the gate/up form for K > 5120 (2-stage ring beside
+    the 64-group scale table); its ffn of 256 leaves no light tiles."""
     from pisceslx_amd import _lib
     from pisceslx_amd.workloads import LayerSpec
-    counts = [256, 257, 272, 273, 288, 289, 320, 321, 544, 16]
-    E, H, F, N = len(counts), hidden, 256, sum(counts)
-    assert N == 11 * 256 + 20
-    spec = LayerSpec("folds", H, F, E, 1, 1, getattr(_lib, "W_" + fmt.upper()), torch.bfloat16,
-                     fixed_shape_mode=True)
-    w = make_workload(spec, device="cuda", lengths=[N])
-    g = torch.Generator().manual_seed(5)
-    expert = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(N, generator=g)]
-    x = torch.randn(N, H, generator=g) * 0.5
-    x[torch.arange(N), expert] += 8.0
-    gate = torch.zeros(E, H)
-    gate[torch.arange(E), torch.arange(E)] = 1.0
-    w.x = x.to(torch.bfloat16).cuda()
-    w.gate_weight = gate.to(torch.bfloat16).cuda()
-    _, _, routing = _run_and_check(oracle, w, label=f"layer folded tiles {fmt} H={hidden} N={N}")
+    counts = [256, 257, 272, 273, 288, 289, 320, 321, 544, 16] * 7
+    spec = LayerSpec("folds", hidden, 512 if hidden == 256 else 256, len(counts), 1, 1, getattr(_lib, "W_" + fmt.upper()),
+                     torch.bfloat16, fixed_shape_mode=True)
+    w = forced_rows(spec, counts)
+    assert tile_rows_of(w) == 256
+    _, _, routing = _run_and_check(oracle, w, tokens=ends_of_segments(counts, last=66),
+                                   label=f"layer folded tiles {fmt} H={hidden} N={sum(counts)}")
     assert routing.counts.cpu().tolist() == counts
 
 
-@pytest.mark.parametrize("fmt,hidden", [("int8", 256), ("int4", 256), ("fp8", 256), ("bf16", 256),
-                                        ("fp8", 1024)])
+@pytest.mark.parametrize("fmt,hidden", [("int8", 1024), ("int4", 1024), ("fp8", 1024), ("bf16", 1024),
+                                        ("fp8", 896)])
 def test_tiled_light_remainders(cuda, oracle, fmt, hidden):
-    """Skewed prefill-sized batches (mean under two 256-row tiles per expert, no folding): an
-    expert's remainder of at most 32 rows runs on the weight-streaming form with 32-row tiles
-    after the LDS-tiled launch (segments of 10 and 32 rows, and 256 + 24, 256 + 32 and the
-    shared segment's 6 x 256 + 20), a longer remainder keeps its 256-row tile (33, 57, 512 + 88),
-    and a segment of exactly 256 rows has no remainder; forced through one-hot gate rows."""
+    """Skewed prefill-sized batches (mean under two 256-row tiles per expert, no folding) with too few
+    light remainders for all of them to leave the tiles: one of at most 32 rows runs on the
+    mid-sized form after the LDS-tiled launch (segments of 10, 32, 256 + 24 and 256 + 32 rows), a
+    longer remainder keeps its 256-row tile (33, 57, 512 + 88, and the shared segment's 48 x 256 +
+    60), and a segment of exactly 256 rows has no remainder; forced through one-hot gate rows."""
     from pisceslx_amd import _lib
     from pisceslx_amd.workloads import LayerSpec
-    counts = [10, 32, 33, 256, 280, 288, 600, 57]
-    E, H, F, N = len(counts), hidden, 256, sum(counts)
-    assert N == 6 * 256 + 20
-    spec = LayerSpec("light", H, F, E, 1, 1, getattr(_lib, "W_" + fmt.upper()), torch.bfloat16,
+    counts = [10, 32, 33, 256, 280, 288, 600, 57] * 3 + [256] * 30
+    spec = LayerSpec("light", hidden, 768, len(counts), 1, 1, getattr(_lib, "W_" + fmt.upper()), torch.bfloat16,
                      fixed_shape_mode=True)
-    w = make_workload(spec, device="cuda", lengths=[N])
-    g = torch.Generator().manual_seed(6)
-    expert = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(N, generator=g)]
-    x = torch.randn(N, H, generator=g) * 0.5
-    x[torch.arange(N), expert] += 8.0
-    gate = torch.zeros(E, H)
-    gate[torch.arange(E), torch.arange(E)] = 1.0
-    w.x = x.to(torch.bfloat16).cuda()
-    w.gate_weight = gate.to(torch.bfloat16).cuda()
-    _, _, routing = _run_and_check(oracle, w, label=f"layer light remainders {fmt} H={hidden} N={N}")
+    w = forced_rows(spec, counts)
+    assert w.n_tokens == 48 * 256 + 60 and tile_rows_of(w) == 256
+    _, _, routing = _run_and_check(oracle, w, tokens=ends_of_segments(counts),
+                                   label=f"layer light remainders {fmt} H={hidden} N={w.n_tokens}")
     assert routing.counts.cpu().tolist() == counts
 
 
@@ -207,11 +192,26 @@ def _shared_spec(fmt_name, S):
 @pytest.mark.parametrize("fmt,S,n", [("int8", 2, 23), ("fp8", 3, 5), ("int4", 1, 64),
                                      ("bf16", 2, 17)])
 def test_decode_shared_expert_segments(cuda, oracle, fmt, S, n):
-    """Decode sizes (the streaming form, 16-row tiles): the shared experts' segments of the
-    tile table (rows N*k + s*N, tiles cut at each segment end) for every weight format, 1-3
-    shared experts and batches that end inside a 16-row tile."""
+    """Decode sizes of a small layer (the few-token form; int4's 64 tokens the mid-sized one): the
+    shared experts' segments of the tile table (rows N*k + s*N, tiles cut at each segment end) for
+    every weight format, 1-3 shared experts and batches that end inside a 16-row tile."""
     w = make_workload(_shared_spec(fmt, S), device="cuda", lengths=[n])
+    assert (tile_rows_of(w), few_forms_of(w)) == (64 if n == 64 else 16, 3)
     _run_and_check(oracle, w, label=f"shared segments {fmt} S={S} N={n}")
+
+
+@pytest.mark.parametrize("fmt,S,n,few", [("int8", 2, 33, 0), ("int4", 1, 33, 0), ("fp8", 3, 24, 0), ("fp8", 1, 49, 0),
+                                         ("bf16", 2, 40, 0), ("int8", 0, 33, 2), ("bf16", 0, 40, 2)])
+def test_decode_on_the_streaming_form(cuda, oracle, fmt, S, n, few):
+    """Decode sizes of a layer large enough for the streaming form, in both GEMMs or in gate/up alone
+    (few: the GEMMs on the few-token form): 16-row tiles of 3 to 6 rows, the shared experts' 64-row
+    items, batches that end inside either, none to three shared experts."""
+    from pisceslx_amd import _lib
+    from pisceslx_amd.workloads import LayerSpec
+    spec = LayerSpec("streaming", 1536, 2048, 32, 4, S, getattr(_lib, "W_" + fmt.upper()), torch.bfloat16)
+    w = make_workload(spec, device="cuda", lengths=[n])
+    assert (tile_rows_of(w), few_forms_of(w)) == (16, few)
+    _run_and_check(oracle, w, label=f"streaming {fmt} S={S} N={n}")
 
 
 def test_forward_is_deterministic(cuda, oracle):

@@ -2,34 +2,21 @@
 expert) where it can go wrong: segment lengths at the edges of its row-block variants and
 tiles, K of fewer k-steps than its weight ring, partial last column groups, and scale tables
 refilled every 8192 of K."""
+import numpy as np
 import pytest
 import torch
 
+from helpers import ends_of_segments, few_forms_of, forced_rows, tile_rows_of
 from test_gpu_layer import _run_and_check
 from pisceslx_amd.workloads import LayerSpec, make_workload
 
 pytestmark = pytest.mark.gpu
 
 # rows per expert: the edges of the 32-, 64-, 96- and 128-row variants, an empty expert and an
-# expert of two tiles; the first list is mean 56 (128-row tiles), the second 30 (64-row tiles on
-# these small layers)
+# expert of two tiles; the first list has 56 rows on average (128-row tiles), the second 30 (64-row
+# tiles on these small layers, but for fp8 at hidden 8320)
 WIDE = [0, 1, 15, 17, 32, 33, 63, 65, 96, 97, 128, 129]
 NARROW = [1, 16, 31, 33, 64, 65, 0, 30]
-
-
-def forced_rows(spec, counts, seed=7):
-    """A workload whose expert e receives exactly counts[e] tokens (one-hot gate rows, top-1)."""
-    N, E, H = sum(counts), len(counts), spec.hidden
-    w = make_workload(spec, device="cuda", lengths=[N])
-    g = torch.Generator().manual_seed(seed)
-    expert = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(N, generator=g)]
-    x = torch.randn(N, H, generator=g) * 0.5
-    x[torch.arange(N), expert] += 8.0
-    gate = torch.zeros(E, H)
-    gate[torch.arange(E), torch.arange(E)] = 1.0
-    w.x = x.to(torch.bfloat16).cuda()
-    w.gate_weight = gate.to(torch.bfloat16).cuda()
-    return w
 
 
 @pytest.mark.parametrize("counts", [WIDE, NARROW], ids=["rows128", "rows64"])
@@ -47,16 +34,31 @@ def test_segment_edges(cuda, oracle, fmt, hidden, ffn, counts):
     spec = LayerSpec("mid", hidden, ffn, len(counts), 1, 1, getattr(_lib, "W_" + fmt.upper()),
                      torch.bfloat16, fixed_shape_mode=True)
     w = forced_rows(spec, counts)
+    assert tile_rows_of(w) == (128 if counts is WIDE or (fmt, hidden) == ("fp8", 8320) else 64)
     _, _, routing = _run_and_check(oracle, w, label=f"mid {fmt} H={hidden} F={ffn} N={sum(counts)}")
     assert routing.counts.cpu().tolist() == counts
 
 
-@pytest.mark.parametrize("n", [10, 11, 85, 86, 193, 512])
-def test_form_boundaries(cuda, oracle, n):
-    """Token counts on both sides of the rules' lines (8 experts' rows at top-6 of 8)."""
+@pytest.mark.parametrize("layer,fmt,n", [
+    ((6, 8, 256), "int8", 18), ((6, 8, 256), "int4", 18),    # few-token form to 64-row tiles
+    ((6, 8, 256), "int8", 65), ((6, 8, 256), "bf16", 65),    # 64- to 128-row tiles
+    ((2, 40, 1024), "int8", 21), ((2, 40, 1024), "bf16", 21),  # gate/up leaves the few-token form
+    ((2, 40, 1024), "fp8", 164), ((2, 40, 1024), "int4", 192),
+    ((2, 40, 1024), "int8", 961), ((2, 40, 1024), "int4", 961),
+    ((2, 40, 1024), "bf16", 2817), ((2, 40, 1024), "int8", 5121), ((2, 40, 1024), "fp8", 5121),  # to 256 rows
+])
+def test_form_boundaries(cuda, oracle, layer, fmt, n):
+    """The last token count of one form and the first of the next (hidden 512, one shared expert)."""
     from pisceslx_amd import _lib
-    spec = LayerSpec("midline", 512, 256, 8, 6, 1, _lib.W_INT8, torch.bfloat16)
-    _run_and_check(oracle, make_workload(spec, device="cuda", lengths=[n]), label=f"mid line N={n}")
+    k, E, F = layer
+    spec = LayerSpec("line", 512, F, E, k, 1, getattr(_lib, "W_" + fmt.upper()), torch.bfloat16)
+    forms = []
+    for m in (n - 1, n):
+        w = make_workload(spec, device="cuda", lengths=[m])
+        forms.append((tile_rows_of(w), few_forms_of(w) if tile_rows_of(w) == 16 else 0))
+        tokens = None if m <= 1000 else np.linspace(0, m - 1, 256).astype(np.int64)
+        _run_and_check(oracle, w, tokens=tokens, label=f"form line {fmt} F={F} N={m}")
+    assert forms[0] != forms[1]
 
 
 @pytest.mark.parametrize("fmt,light", [("int8", 64), ("int8", 63), ("int4", 64), ("fp8", 64), ("bf16", 64)])
@@ -67,15 +69,16 @@ def test_light_remainders_of_many_experts(cuda, oracle, fmt, light):
     takes up to 64 rows, so here too few and only those of up to 32.)"""
     from pisceslx_amd import _lib
     counts = [1 + (e * 37) % 96 for e in range(light - 8)] + [256 + 96, 512 + 1] * 4
-    counts += [97, 0, 256, 700, 3 * 256 + 200] * 5
+    counts += [97, 0, 256, 700, 3 * 256 + 200] * 7
     counts.append((128 - sum(counts)) % 256 + 512)  # the shared segment ends in 128 rows: not light
     counts[-1] += 97 if 0 < counts[-1] % 256 <= 96 else 0
     assert sum(0 < c % 256 <= 96 for c in counts) == light and not 0 < sum(counts) % 256 <= 96
-    assert sum(counts) >= 150 * len(counts)         # the rule's line for the 256-row form
     spec = LayerSpec("manylight", 256, 512, len(counts), 1, 1, getattr(_lib, "W_" + fmt.upper()),
                      torch.bfloat16, fixed_shape_mode=True)
     w = forced_rows(spec, counts)
-    _, _, routing = _run_and_check(oracle, w, label=f"many light {fmt} N={sum(counts)} E={len(counts)}")
+    assert tile_rows_of(w) == 256
+    _, _, routing = _run_and_check(oracle, w, tokens=ends_of_segments(counts, last=100),
+                                   label=f"many light {fmt} N={sum(counts)} E={len(counts)}")
     assert routing.counts.cpu().tolist() == counts
 
 
@@ -95,6 +98,7 @@ def test_tiled_forms(cuda, oracle, fmt, hidden, ffn):
     spec = LayerSpec("tiled", hidden, ffn, len(MANY), 1, 1, getattr(_lib, "W_" + fmt.upper()),
                      torch.bfloat16, fixed_shape_mode=True)
     w = forced_rows(spec, MANY)
+    assert tile_rows_of(w) == 256
     _, _, routing = _run_and_check(oracle, w, label=f"tiled {fmt} H={hidden} F={ffn} N={sum(MANY)}")
     assert routing.counts.cpu().tolist() == MANY
 
@@ -114,6 +118,7 @@ def test_a_few_rows(cuda, oracle, fmt, hidden, ffn):
     spec = LayerSpec("few", hidden, ffn, len(counts), 1, 1, getattr(_lib, "W_" + fmt.upper()),
                      torch.bfloat16, fixed_shape_mode=True)
     w = forced_rows(spec, counts)
+    assert tile_rows_of(w) == 16 and few_forms_of(w) == 3
     _, _, routing = _run_and_check(oracle, w, label=f"few {fmt} H={hidden} F={ffn} N={sum(counts)}")
     assert routing.counts.cpu().tolist() == counts
     _run_and_check(oracle, make_workload(spec, device="cuda", lengths=[1]), label=f"few {fmt} N=1")
