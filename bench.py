@@ -5,9 +5,9 @@ A step is one forward of the whole layer (router GEMM + complexity predictor, ro
 permutation, grouped SwiGLU FFN of routed and shared experts, combine with the skip residual)
 over one packed batch whose inputs and weights are already resident in HBM.
 
-Default workload: BASELINE configs[1] (cfg2) — W8A16 layer, hidden 4096, 64 experts (FFN
+Default workload: cfg2 — W8A16 layer, hidden 4096, 64 experts (FFN
 1408), top-6, 2 shared experts, decode batch of 64 sequences x 1 token. The same run also
-times configs[2] (cfg3, the same layer on a ~16K-token ragged prefill) as the "prefill"
+times cfg3 (the same layer on a ~16K-token ragged prefill) as the "prefill"
 object, and the CPU oracle (the reference algorithm restated in torch on the host) on cfg2
 as "cpu_baseline", with bounded samples of cfg3, cfg1, cfg4 and cfg5 beside it.
 
@@ -28,8 +28,7 @@ profiles/expert_ffn_cfg2_decode_traffic.json and reported when present.
 "rmsnorm": the MoE input norms of the hybrid block (two RMSNorms in one pass) at the decode
 and prefill token counts, HBM roofline of the kernel.
 
-"other_configs": configs[0], [3], [4] (cfg1 fp32, cfg4 W4A16 mixed batch, cfg5 fp8 with skewed
-routing): layer step and grouped FFN, the FFN against both rooflines; cfg5 also reports its
+"other_configs": cfg1 (fp32), cfg4 (W4A16 mixed batch) and cfg5 (fp8 with skewed routing): layer step and grouped FFN, the FFN against both rooflines; cfg5 also reports its
 realised expert load against the Zipf(1.2) target (KL).
 
 Usage: python bench.py [--steps K] [--warmup W] [--gpus 1]
@@ -51,7 +50,7 @@ METRIC = "MoE layer tokens/s at 1 GPU; HBM GB/s (decode) & MFMA util % (prefill)
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "expert_ffn_cfg2_decode_traffic.json")
 HBM_PEAK_GBS = 8000.0
 BF16_PEAK_TFLOPS = 2500.0
-F32_PEAK_TFLOPS = 157.3
+F32_PEAK_TFLOPS = BF16_PEAK_TFLOPS / 6  # an fp32 product is six bf16 ones (the fp32 MFMAs: 157.3)
 
 
 def parse():
@@ -320,10 +319,10 @@ def norm_bench(w, steps, lengths):
 
 
 def other_configs(names, steps):
-    """The BASELINE configs that are not bench lines (cfg1 fp32 parity layer, cfg4 W4A16 mixed
+    """The configurations that are not bench lines (cfg1 fp32 parity layer, cfg4 W4A16 mixed
     batch, cfg5 fp8 skewed routing): the layer step and the grouped FFN, each FFN priced against
     both rooflines (algorithmic bytes over 8 TB/s, algorithmic FLOPs over the MFMA peak of the
-    compute dtype: fp32 157.3 TFLOP/s for cfg1, bf16 2.5 PFLOP/s otherwise)."""
+    compute dtype: bf16 2.5 PFLOP/s; cfg1's fp32 products are six bf16 ones each, a sixth of it)."""
     import torch
     from pisceslx_amd import functional as yvf
     from pisceslx_amd.quant import FORMAT_NAMES
@@ -484,7 +483,7 @@ def main():
         "vs_baseline": None,
         "dtype": "bf16",
         "data": "synthetic",
-        "config": {"workload": "cfg2: W8A16 Yv MoE layer decode (BASELINE configs[1])",
+        "config": {"workload": "cfg2: W8A16 Yv MoE layer decode",
                    "tokens": N, "hidden": H, "experts": spec.num_experts, "ffn": spec.ffn,
                    "top_k": spec.top_k, "shared_experts": spec.num_shared,
                    "weights": "int8 per-output-channel, bf16 scales", "seed": 0},
@@ -512,7 +511,7 @@ def main():
         tf = wp["flops"] / tpf / 1e12
         layer_flops = wp["flops"] + 2 * Np * H * (spec.num_experts + 192)
         result["prefill"] = {
-            "workload": "cfg3: same layer, ragged prefill of 32 sequences (BASELINE configs[2])",
+            "workload": "cfg3: same layer, ragged prefill of 32 sequences",
             "tokens": Np, "tokens_per_s": round(Np / tp, 1), "ms_per_step": round(tp * 1e3, 3),
             "layer_tflops": round(layer_flops / tp / 1e12, 1),
             "roofline": {"bound": "mfma", "achieved": round(tf, 1), "peak": BF16_PEAK_TFLOPS,

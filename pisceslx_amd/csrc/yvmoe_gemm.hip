@@ -1692,9 +1692,14 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(GemmParams p, int ncb) {
 // What bounds it: HBM while the rows are few, then the conversion (2.3-2.5 VALU instructions per
 // weight) and the LDS reads of the activations beside the MFMAs. Every weight is read and
 // converted once per tile and needed by one wavefront only, so the weights go straight to
-// registers in their stored order (1 KB per load), kMidRing - 1 k-steps ahead of their use; the
-// activation rows, which all four wavefronts need, travel by direct-to-LDS loads through a
-// 3-stage ring two k-steps ahead (the swizzle of the 256-row tile). 48 KB of LDS and under 170
+// registers in their stored order (1 KB per load), issued MidCfg<WF>::RING - 1 k-steps ahead of
+// their use (two for bf16, three else); the activation rows, which all four wavefronts need, travel
+// by direct-to-LDS loads through a 3-stage ring, issued two k-steps ahead (the swizzle of the
+// 256-row tile). How much of that is in flight: the compiler waits for a step's weights by the
+// number of its own, later weight loads (6; bf16 8), but the activation loads, which it does not
+// count, share the counter. In the 128-row copy, whose steps issue that many loads each, everything
+// older than the current step's loads has landed then, that is one step is in flight; in the 96-,
+// 64- and 32-row copies up to 1 1/5, 1 1/2 and 2. 48 KB of LDS and under 170
 // VGPRs put three work-groups on a CU, so one's conversion and LDS reads run beside another's
 // MFMAs and loads. A tile runs the copy of the loop for its row blocks rounded up to an even
 // count, so rows past its end are neither loaded nor multiplied. The scheduling barriers keep
@@ -1706,13 +1711,14 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(GemmParams p, int ncb) {
 // Measured (H 4096, 64 experts of 1408, 6 + 2 per token; FFN, against the form it replaced):
 // int8 200 tokens 345 -> 213 us, 500 516 -> 271 us, 700 486 -> 321 us (16-, 64- and 256-row
 // forms); bf16 341 tokens 859 -> 420 us; int4 341 tokens 462 -> 228 us.
-// Accumulation per output is in the order of the other forms (k-step by k-step, k = 16 g + 0..7
-// before 16 g + 8..15), so the results are bit-identical to them.
+// Accumulation per output is in the order of the streaming and the 256-row forms (k-step by k-step,
+// k = 16 g + 0..7 before 16 g + 8..15), so the results are bit-identical to theirs (not to the
+// few-token form's, which sums four parts of K).
 constexpr int kMidGroups = 64;  // scale groups (128 of K) per LDS table
 
 template <int WF>
 struct MidCfg {
-    static constexpr int RING = WF == YVMOE_W_BF16 ? 3 : 4;  // weight ring, k-steps (deeper: no gain)
+    static constexpr int RING = WF == YVMOE_W_BF16 ? 3 : 4;  // weight ring, k-steps (deeper: no gain, see above)
     static constexpr int WD = WF == YVMOE_W_BF16 ? 4 : 2;    // weight loads per k-step
     static constexpr bool GROUPED = WF == YVMOE_W_INT4 || WF == YVMOE_W_FP8;
     // group scales of a range of K in LDS: int4 bf16, kMidGroups (+ 2 against bank conflicts) per
@@ -2963,7 +2969,9 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
 //   and 1340 / 1398; fp8 H 7168, 256 experts 112 rows 3207 / 3874 and 3549 / 3743). In bf16 shared experts
 //   alone may fill the 256-row tiles: 256 rows of a segment (H 4096, 64 experts of 512, top-1 and 2
 //   shared, 96 rows of an expert 419 and 386 us). Any number of rows where the 256-row form's scale
-//   tables (fp8, int4: 8192 of K) do not hold the shape, and, up to 256 rows, where the rounds of 256-row
+//   tables (fp8, int4: 8192 of K) do not hold the shape, and, up to 256 rows (above while there are at
+//   most 448 work-groups: H 512, 8 experts of 256, int8 1,500 / 2,500 / 4,000 rows, 0.44 / 0.73 / 0.58 of the
+//   chip in use: mid 53 / 67 / 87 us, 256-row tiles 51 / 55 / 87), where the rounds of 256-row
 //   work-groups would leave a fifth of the chip idle over both GEMMs, in bf16 two fifths, near its lines
 //   a quarter (H 1024, 8 experts of 2816, 180 / 210 rows, a third in use: int8 97 / 99 us against 124 / 154,
 //   bf16 101 / 102 against 116 / 147; H 7168, 32 of 1024, 112 / 150 rows, 0.69 / 0.73 in use: bf16 392 / 744

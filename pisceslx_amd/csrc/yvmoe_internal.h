@@ -119,7 +119,8 @@ inline RouterSplit router_split(int N, int E, int act, int H, size_t room = ~(si
 }
 
 // Dense fp32-output GEMMs of more than 64 rows with bf16 operands, 256-multiple columns and
-// 64-multiple K run on the LDS-tiled MFMA form (256 x 256 output tiles, no K split).
+// 64-multiple K run without a K split: on the mid-sized form while their 256 x 256 tiles would leave
+// much of the chip idle, on the LDS-tiled MFMA forms above (dense_partials_launch).
 inline bool dense_tiled(int act, int N, int ncols, int K) {
     return act == YVMOE_ACT_BF16 && N > 64 && ncols % 256 == 0 && K % 64 == 0;
 }

@@ -6,7 +6,8 @@
 // Kernels:
 //   moegate_proj (dense_partials_launch): fp32 [N][P] = x · W_projᵀ, W_proj = [dg_proj
 //     (hicl_router.py:77); gate; got_cluster_proj; gate_k; gate_v; input_encoder.0; zero
-//     rows] — the LDS-tiled MFMA form for batches above 64 rows, the streaming form below.
+//     rows] — the streaming form up to 64 rows, then the mid-sized form up to 144 tiles of 256 x 256
+//     (narrow projections 96), the LDS-tiled forms above.
 //   moegate_token_kernel: per token — relu(dg + dg_bias), the sel_k largest kept (radix select
 //     on the float bit patterns, ties to the lower index), L2-normalised, dotted with the
 //     prototypes (HiCL, gate.py:335-340); the lower median of gate_k, sigmoid, softmax of

@@ -13,7 +13,7 @@ measures it against the correctly rounded oracle:
   correctly rounded statement, so it cannot bind a third correct implementation either;
 * every one of them lies at |out| >= 2, within two bf16 steps of the oracle (0.03125), and
   the whole output lies inside ``bf16_allowance``;
-* at most 1e-5 of the elements exceed 2e-2 and the cosine is >= 0.9999 (the north star's
+* at most 1e-5 of the elements exceed 2e-2 and the cosine is >= 0.9999 (the target's
   other two figures).
 """
 import numpy as np
