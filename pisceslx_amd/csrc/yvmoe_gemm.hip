@@ -2966,14 +2966,20 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
 //   experts and more a skewed load moves most rows to a few experts of many tiles each and leaves a tail
 //   of short ones, which the 256-row form hands to mid (tile_light): fp8 112, bf16 96 (bf16 96 rows,
 //   even / Zipf loads: H 7168, 256 experts 4300 / 5103 and 4316 / 4404 us, H 5120, 128 experts 1289 / 1510
-//   and 1340 / 1398; fp8 H 7168, 256 experts 112 rows 3207 / 3874 and 3549 / 3743). In bf16 shared experts
-//   alone may fill the 256-row tiles: 256 rows of a segment (H 4096, 64 experts of 512, top-1 and 2
-//   shared, 96 rows of an expert 419 and 386 us). Any number of rows where the 256-row form's scale
+//   and 1340 / 1398; fp8 H 7168, 256 experts 112 rows 3207 / 3874 and 3549 / 3743). Earlier where
+//   shared experts fill 256-row tiles beside few rows of the others, and where an F of up to 768 gives mid
+//   few column groups, which eight XCDs share unevenly (two of them do twice the work of ten groups): int8
+//   128 rows of an expert, int4 120, bf16 80; with most rows in shared experts int8 and fp8 96, bf16 80 for
+//   any F, times that evenness (top-1 of 64 experts and 2 shared: H 3840, F 640, int8 101 / 112 / 140 rows 477 /
+//   518 / 686 us and 463 / 480 / 501, bf16 56 / 72 / 80 rows 417 / 484 / 515 and 366 / 396 / 408; H 4096, F 1408,
+//   bf16 64 / 80 rows 805 / 912 and 802 / 792; top-2 and 1 shared, H 3840, F 640, int8 101 / 128 / 140 rows 262 /
+//   349 / 407 and 305 / 317 / 323). Without shared experts a skewed load has more to lose there (H 4096, F 512,
+//   top-2, int8 140 rows even / skewed 260 / 238 and 212 / 325). Any number of rows where the 256-row form's scale
 //   tables (fp8, int4: 8192 of K) do not hold the shape, and, up to 256 rows (above while there are at
 //   most 448 work-groups: H 512, 8 experts of 256, int8 1,500 / 2,500 / 4,000 rows, 0.44 / 0.73 / 0.58 of the
 //   chip in use: mid 53 / 67 / 87 us, 256-row tiles 51 / 55 / 87), where the rounds of 256-row
-//   work-groups would leave a fifth of the chip idle over both GEMMs, in bf16 two fifths, near its lines
-//   a quarter (H 1024, 8 experts of 2816, 180 / 210 rows, a third in use: int8 97 / 99 us against 124 / 154,
+//   work-groups would leave a fifth of the chip idle over both GEMMs (a quarter for a narrow F with
+//   most rows in shared experts), in bf16 two fifths, near its lines a quarter (H 1024, 8 experts of 2816, 180 / 210 rows, a third in use: int8 97 / 99 us against 124 / 154,
 //   bf16 101 / 102 against 116 / 147; H 7168, 32 of 1024, 112 / 150 rows, 0.69 / 0.73 in use: bf16 392 / 744
 //   against 514 / 590, int8 150 rows 511 against 567; but H 4096, 64 of 512, whose gate/up has one
 //   work-group per CU and whose down has four, int8 150 / 180 rows 284 / 301 and 228 / 239).
@@ -3005,9 +3011,17 @@ int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf) {
         const double tiles = (double)E * ((slots + 256LL * E - 1) / (256LL * E)) + (double)S * ceil_div(N, TBM);
         const double up = tiles * ceil_div(F, TBN / 2), down = tiles * ceil_div(H, TBN);
         const double used = (up * H + down * F) / (256.0 * (std::ceil(up / 256) * H + std::ceil(down / 256) * F));
-        const int most = wf == YVMOE_W_FP8 ? (many ? 112 : 125) : !bf16 ? 150 : many && used >= 0.72 ? 96 : 112;
-        const bool enough = slots >= (long long)most * E || (bf16 && S > 0 && seg_rows(256));
-        const double least = bf16 ? (slots < 128LL * E ? 0.72 : 0.6) : 0.8;
+        // a narrow F with shared experts, the same with most rows theirs
+        const bool narrow = F <= 768 && S > 0, shared = (long long)S * N >= slots;
+        const int groups = ceil_div(F, 64);
+        const int most = bf16 ? (shared                        ? 80 * groups / (8 * ceil_div(groups, 8))
+                                 : narrow && !many             ? 80
+                                 : many && used >= 0.72 ? 96 : 112)
+                         : wf == YVMOE_W_FP8 ? (narrow && shared ? 96 : many ? 112 : 125)
+                         : narrow            ? (int4 ? 120 : shared ? 96 : 128)
+                                             : 150;
+        const bool enough = slots >= (long long)most * E;
+        const double least = bf16 ? (slots < 128LL * E ? 0.72 : 0.6) : narrow && shared ? 0.77 : 0.8;
         const bool large = slots > 256LL * E && max_tiles(N, k, E, S, TBM) * (long long)ceil_div(F, TBN / 2) > 448;
         if (enough && (used >= least || large)) return TBM;
     }

@@ -304,7 +304,9 @@ __host__ __device__ inline int seg_tiles(int rows, int tile_rows, int fold, int 
 // 256 experts, skewed, mean 256 / 125 rows 6995 -> 6661 / 4338 -> 4044 us; int8 H 4096, 64 experts,
 // mean 768 / 1567 2316 -> 2194 / 4467 -> 4414. bf16 tiles, which convert nothing, gain less: up to 32
 // rows above the folding range (H 7168, 256 experts, mean 330 / 375: up to 32 rows 9191 / 9459 us, 96
-// 9714 / 9979), none from 512 (mean 562: 1823 -> 1896 us); layers of 128 experts and more, whose tiles
+// 9714 / 9979), none from 512 (mean 562: 1823 -> 1896 us), nor
+// where F is up to 768 (H 3840, 64 experts of 640, top-1 and 2 shared, skewed, mean 80 / 101 / 150: up to 96
+// rows 470 / 503 / 635 us, 32 412 / 437 / 561); layers of 128 experts and more, whose tiles
 // start below 128 rows, up to 128 there (Zipf load, H 5120, mean 96: up to 96 rows 1456 us, 128 1398; with
 // 16 experts, mean 119, 384 and 497). int4, whose mid-sized form has two
 // work-groups per CU instead of three, takes 64 (H 5120, 128 experts, mean 375: 2936 us on 32 rows,
@@ -320,7 +322,7 @@ inline int tile_light(int N, int k, int E, int S, int F, int wf) {
     if (wf == YVMOE_W_BF16 && mean >= 512) return 0;
     if ((E + S) * ceil_div(F, 64) < kLightGroups) return 0;
     if (wf == YVMOE_W_BF16 && mean < 128 && E >= 128) return 128;
-    if (wf == YVMOE_W_BF16 && mean > 256 + 2 * kTileFold) return 32;
+    if (wf == YVMOE_W_BF16 && (mean > 256 + 2 * kTileFold || F <= 768)) return 32;
     return wf == YVMOE_W_INT4 ? 64 : kLightRows;
 }
 

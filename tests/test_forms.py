@@ -45,7 +45,14 @@ MID, CFG5, SMALL = (6, 64, 2, 4096, 1408), (8, 256, 0, 7168, 2048), (2, 8, 1, 10
     # mid-sized to the 256-row tiles: int8 and int4 150 rows, fp8 125, bf16 112; many experts fp8 112, bf16 96
     (MID, I8, 1599, 128), (MID, I8, 1600, 256), (MID, I4, 1600, 256), (MID, F8, 1333, 128), (MID, F8, 1334, 256),
     (MID, B16, 1194, 128), (MID, B16, 1195, 256), (CFG5, F8, 3583, 128), (CFG5, F8, 3584, 256),
-    (CFG5, B16, 3071, 128), (CFG5, B16, 3072, 256), ((1, 64, 2, 4096, 512), B16, 5631, 128), ((1, 64, 2, 4096, 512), B16, 5632, 256),
+    (CFG5, B16, 3071, 128), (CFG5, B16, 3072, 256), ((1, 64, 2, 4096, 512), B16, 5119, 128), ((1, 64, 2, 4096, 512), B16, 5120, 256),
+    # ... earlier for shared experts and a narrow F
+    ((1, 64, 2, 4096, 1408), B16, 4671, 128), ((1, 64, 2, 4096, 1408), B16, 4672, 256),
+    ((1, 64, 2, 3840, 640), I8, 6143, 128), ((1, 64, 2, 3840, 640), I8, 6144, 256), ((1, 64, 2, 3840, 640), I8, 11520, 256),
+    ((1, 64, 2, 3840, 640), B16, 3199, 128), ((1, 64, 2, 3840, 640), B16, 3200, 256),
+    ((2, 64, 1, 3840, 640), I8, 4095, 128), ((2, 64, 1, 3840, 640), I8, 4096, 256), ((2, 64, 1, 3840, 640), I4, 3839, 128),
+    ((2, 64, 1, 3840, 640), I4, 3840, 256), ((2, 64, 1, 3840, 640), B16, 2559, 128), ((2, 64, 1, 3840, 640), B16, 2560, 256),
+    ((1, 64, 2, 3840, 640), F8, 6143, 128), ((1, 64, 2, 3840, 640), F8, 6144, 256),
     # ... not where those would leave much of the chip idle
     (SMALL, I8, 1000, 128), (SMALL, B16, 1000, 128), (SMALL, B16, 1600, 256), ((4, 32, 2, 7168, 1024), B16, 1000, 128),
     ((4, 32, 2, 7168, 1024), B16, 1200, 256), ((2, 64, 0, 4096, 512), I8, 4800, 256), (SMALL, I8, 2000, 256),

@@ -66,7 +66,7 @@ def test_light_remainders_of_many_experts(cuda, oracle, fmt, light):
     """Prefill-sized skewed batches of many experts: remainders of 1 .. 96 rows leave the 256-row
     tiles for the mid-sized form when there are enough of them (64 at ffn 512; the tile table's
     kernel decides), whole experts and tails after full tiles alike; 97 rows keep a tile. (int4
-    takes up to 64 rows, so here too few and only those of up to 32.)"""
+    takes up to 64 rows, so here too few and only those of up to 32, as with bf16 at this ffn.)"""
     from pisceslx_amd import _lib
     counts = [1 + (e * 37) % 96 for e in range(light - 8)] + [256 + 96, 512 + 1] * 4
     counts += [97, 0, 256, 700, 3 * 256 + 200] * 7
