@@ -28,8 +28,9 @@ profiles/expert_ffn_cfg2_decode_traffic.json and reported when present.
 "rmsnorm": the MoE input norms of the hybrid block (two RMSNorms in one pass) at the decode
 and prefill token counts, HBM roofline of the kernel.
 
-"other_configs": cfg1 (fp32), cfg4 (W4A16 mixed batch) and cfg5 (fp8 with skewed routing): layer step and grouped FFN, the FFN against both rooflines; cfg5 also reports its
-realised expert load against the Zipf(1.2) target (KL).
+"other_configs": cfg1 (fp32), cfg4 (W4A16 mixed batch) and cfg5 (fp8 with skewed routing): layer
+step and grouped FFN, the FFN against both rooflines; cfg5 also reports its realised expert load
+against the Zipf(1.2) target (KL).
 
 Usage: python bench.py [--steps K] [--warmup W] [--gpus 1]
        python bench.py --pmc-probe {cfg2,cfg3,cfg5,moegate,moegate_decode}   (launches only, for counter runs)

@@ -258,8 +258,9 @@ int32_t yvmoe_forward(const void* x, int32_t act_dtype, int32_t n_tokens,
  * returns YVMOE_ERR_WORKSPACE (at cfg2's shape, hidden 4096 / 64 experts / top-6 / 2 shared,
  * up to 635 tokens fit); of the router's K splits only as many count there as divide hidden
  * into equal parts, and a call takes fewer splits than yvmoe_forward's where the scratch holds
- * no more (its logits may then differ in the last bits). Every call on one GPU shares that GPU's scratch, which keeps the last
- * call's contents: calls that overlap on one GPU (other streams, other host threads) race.
+ * no more (its logits may then differ in the last bits). Every call on one GPU shares that GPU's
+ * scratch, which keeps the last call's contents: calls that overlap on one GPU (other streams,
+ * other host threads) race.
  */
 #define YVMOE_STATIC_SCRATCH_BYTES (64u << 20)
 int32_t yvmoe_forward_static(const void* x, int32_t act_dtype, int32_t n_tokens,

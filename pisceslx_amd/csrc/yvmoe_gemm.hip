@@ -2941,48 +2941,53 @@ int router_gemm_launch(const void* x, int act, int N, const yvmoe_router* r, flo
 // H 1024, 8 of 2816 36 / 48 186 / 228 and 216 / 229.
 //
 // bf16 activations:
-// * 16: weight streaming, up to 8 rows of a segment, 9 with shared experts. It reads a tile's weights once per 16 rows: int8 H
-//   4096, 64 experts of 1408, 6.5 / 10 / 13 rows of an expert 202 / 210 / 245 us, on 64-row mid tiles 203 /
-//   203 / 212. Up to 14 on the few-token form alone (H 1024, 8 experts of 2816, 7 / 10 / 13 rows of an
-//   expert: int8 32 / 34 / 36 us against 36 / 40 / 41). On grids of two to four mid work-groups per CU of
-//   many experts, which mid's three leave part empty, up to 12 (int8 H 1024, 64 of 640, 8 / 13 rows 42 / 44 us, mid 45 / 46; bf16 H 7168, 32 of 1024, 8 rows 253
-//   and 278). int4 streams suffer where a row of weights is a multiple of 1,024 wide (top-4 of 64 experts
-//   of 1024, 4 / 6 / 9 rows: H 4096 154 / 145 / 146 us, mid 136 / 124 / 120; H 2048 89 / 84 / 92 and 78 / 73 /
-//   72): 4 rows there; 7 else (H 4224 135 / 136 / 145 and 143 / 134 / 129; H 2688 94 / 93 / 101 and 96 / 90 /
-//   92); 14 on grids just past its two work-groups per CU (H 4096, 64 of 640, 9 / 13 rows 101 / 116 us and
-//   105 / 107; H 2688, 64 of 640, 4 / 13 rows 66 / 82 and 78 / 88) and for a short K (H 896, 256 of 768, 4 /
-//   10 / 13 rows 87 / 97 / 108 and 100 / 106 / 108; H 1152 alike).
-// * 64: mid with 64-row tiles, which take less LDS and give more work-groups: int4 up to 48 rows (its
-//   scale table costs 128-row tiles a third work-group per CU: 32 rows 228 us against 246), any format up
-//   to 16 rows of a segment on a small grid (int8 H 1024, 64 experts of 640, 13 rows 45 against 46 us; H 4096, 64 of
-//   512 and 2 shared, 8 rows 101 against 113) and up to 48 where 128-row tiles would leave the down
-//   projection under two work-groups per CU (H 1024, 8 experts of 16 / 32 rows: 48.5 / 48.7 us against
-//   48.2 / 58.3).
-// * 128: mid, from there to where an expert's rows past 128 cost a second pass over its weights: int8
-//   and int4 150 rows, fp8 125, bf16, which converts nothing, 112 (H 4096, 64 experts of 1408, 112 / 128 /
-//   150 rows: int8 451 / 562 / 679 us against 672 / 672 / 716 on 256-row tiles, int4 510 / 618 / 711 against
-//   685 / 629 / 699; bf16 96 / 112 / 128 rows 553 / 600 / 794 against 598 / 653 / 661; fp8 H 5120, 128 experts
-//   of 1536, 112 / 128 rows a ratio of 0.83 / 0.99, 64 experts of H 2688 and 1024 0.83 / 1.00). With 128
-//   experts and more a skewed load moves most rows to a few experts of many tiles each and leaves a tail
-//   of short ones, which the 256-row form hands to mid (tile_light): fp8 112, bf16 96 (bf16 96 rows,
-//   even / Zipf loads: H 7168, 256 experts 4300 / 5103 and 4316 / 4404 us, H 5120, 128 experts 1289 / 1510
-//   and 1340 / 1398; fp8 H 7168, 256 experts 112 rows 3207 / 3874 and 3549 / 3743). Earlier where
-//   shared experts fill 256-row tiles beside few rows of the others, and where an F of up to 768 gives mid
-//   few column groups, which eight XCDs share unevenly (two of them do twice the work of ten groups): int8
-//   128 rows of an expert, int4 120, bf16 80; with most rows in shared experts int8 and fp8 96, bf16 80 for
-//   any F, times that evenness (top-1 of 64 experts and 2 shared: H 3840, F 640, int8 101 / 112 / 140 rows 477 /
-//   518 / 686 us and 463 / 480 / 501, bf16 56 / 72 / 80 rows 417 / 484 / 515 and 366 / 396 / 408; H 4096, F 1408,
-//   bf16 64 / 80 rows 805 / 912 and 802 / 792; top-2 and 1 shared, H 3840, F 640, int8 101 / 128 / 140 rows 262 /
-//   349 / 407 and 305 / 317 / 323). Without shared experts a skewed load has more to lose there (H 4096, F 512,
-//   top-2, int8 140 rows even / skewed 260 / 238 and 212 / 325). Any number of rows where the 256-row form's scale
-//   tables (fp8, int4: 8192 of K) do not hold the shape, and, up to 256 rows (above while there are at
-//   most 448 work-groups: H 512, 8 experts of 256, int8 1,500 / 2,500 / 4,000 rows, 0.44 / 0.73 / 0.58 of the
-//   chip in use: mid 53 / 67 / 87 us, 256-row tiles 51 / 55 / 87), where the rounds of 256-row
-//   work-groups would leave a fifth of the chip idle over both GEMMs (a quarter for a narrow F with
-//   most rows in shared experts), in bf16 two fifths, near its lines a quarter (H 1024, 8 experts of 2816, 180 / 210 rows, a third in use: int8 97 / 99 us against 124 / 154,
-//   bf16 101 / 102 against 116 / 147; H 7168, 32 of 1024, 112 / 150 rows, 0.69 / 0.73 in use: bf16 392 / 744
-//   against 514 / 590, int8 150 rows 511 against 567; but H 4096, 64 of 512, whose gate/up has one
-//   work-group per CU and whose down has four, int8 150 / 180 rows 284 / 301 and 228 / 239).
+// * 16: weight streaming, up to 8 rows of a segment, 9 with shared experts. It reads a tile's
+//   weights once per 16 rows: int8 H 4096, 64 experts of 1408, 6.5 / 10 / 13 rows of an expert 202
+//   / 210 / 245 us, on 64-row mid tiles 203 / 203 / 212. Up to 14 on the few-token form alone (H
+//   1024, 8 experts of 2816, 7 / 10 / 13 rows of an expert: int8 32 / 34 / 36 us against 36 / 40 /
+//   41). On grids of two to four mid work-groups per CU of many experts, which mid's three leave
+//   part empty, up to 12 (int8 H 1024, 64 of 640, 8 / 13 rows 42 / 44 us, mid 45 / 46; bf16 H 7168,
+//   32 of 1024, 8 rows 253 and 278). int4 streams suffer where a row of weights is a multiple of
+//   1,024 wide (top-4 of 64 experts of 1024, 4 / 6 / 9 rows: H 4096 154 / 145 / 146 us, mid 136 /
+//   124 / 120; H 2048 89 / 84 / 92 and 78 / 73 / 72): 4 rows there; 7 else (H 4224 135 / 136 / 145
+//   and 143 / 134 / 129; H 2688 94 / 93 / 101 and 96 / 90 / 92); 14 on grids just past its two
+//   work-groups per CU (H 4096, 64 of 640, 9 / 13 rows 101 / 116 us and 105 / 107; H 2688, 64 of
+//   640, 4 / 13 rows 66 / 82 and 78 / 88) and for a short K (H 896, 256 of 768, 4 / 10 / 13 rows 87
+//   / 97 / 108 and 100 / 106 / 108; H 1152 alike).
+// * 64: mid with 64-row tiles, which take less LDS and give more work-groups: int4 up to 48 rows
+//   (its scale table costs 128-row tiles a third work-group per CU: 32 rows 228 us against 246),
+//   any format up to 16 rows of a segment on a small grid (int8 H 1024, 64 experts of 640, 13 rows
+//   45 against 46 us; H 4096, 64 of 512 and 2 shared, 8 rows 101 against 113) and up to 48 where
+//   128-row tiles would leave the down projection under two work-groups per CU (H 1024, 8 experts
+//   of 16 / 32 rows: 48.5 / 48.7 us against 48.2 / 58.3).
+// * 128: mid, from there to where an expert's rows past 128 cost a second pass over its weights:
+//   int8 and int4 150 rows, fp8 125, bf16, which converts nothing, 112 (H 4096, 64 experts of 1408,
+//   112 / 128 / 150 rows: int8 451 / 562 / 679 us against 672 / 672 / 716 on 256-row tiles, int4
+//   510 / 618 / 711 against 685 / 629 / 699; bf16 96 / 112 / 128 rows 553 / 600 / 794 against 598 /
+//   653 / 661; fp8 H 5120, 128 experts of 1536, 112 / 128 rows a ratio of 0.83 / 0.99, 64 experts
+//   of H 2688 and 1024 0.83 / 1.00). With 128 experts and more a skewed load moves most rows to a
+//   few experts of many tiles each and leaves a tail of short ones, which the 256-row form hands to
+//   mid (tile_light): fp8 112, bf16 96 (bf16 96 rows, even / Zipf loads: H 7168, 256 experts 4300 /
+//   5103 and 4316 / 4404 us, H 5120, 128 experts 1289 / 1510 and 1340 / 1398; fp8 H 7168, 256
+//   experts 112 rows 3207 / 3874 and 3549 / 3743). Earlier where shared experts fill 256-row tiles
+//   beside few rows of the others, and where an F of up to 768 gives mid few column groups, which
+//   eight XCDs share unevenly (two of them do twice the work of ten groups): int8 128 rows of an
+//   expert, int4 120, bf16 80; with most rows in shared experts int8 and fp8 96, bf16 80 for any F,
+//   times that evenness (top-1 of 64 experts and 2 shared: H 3840, F 640, int8 101 / 112 / 140 rows
+//   477 / 518 / 686 us and 463 / 480 / 501, bf16 56 / 72 / 80 rows 417 / 484 / 515 and 366 / 396 /
+//   408; H 4096, F 1408, bf16 64 / 80 rows 805 / 912 and 802 / 792; top-2 and 1 shared, H 3840, F
+//   640, int8 101 / 128 / 140 rows 262 / 349 / 407 and 305 / 317 / 323). Without shared experts a
+//   skewed load has more to lose there (H 4096, F 512, top-2, int8 140 rows even / skewed 260 / 238
+//   and 212 / 325). Any number of rows where the 256-row form's scale tables (fp8, int4: 8192 of K)
+//   do not hold the shape, and, up to 256 rows (above while there are at most 448 work-groups: H
+//   512, 8 experts of 256, int8 1,500 / 2,500 / 4,000 rows, 0.44 / 0.73 / 0.58 of the chip in use:
+//   mid 53 / 67 / 87 us, 256-row tiles 51 / 55 / 87), where the rounds of 256-row work-groups would
+//   leave a fifth of the chip idle over both GEMMs (a quarter for a narrow F with most rows in
+//   shared experts), in bf16 two fifths, near its lines a quarter (H 1024, 8 experts of 2816, 180 /
+//   210 rows, a third in use: int8 97 / 99 us against 124 / 154, bf16 101 / 102 against 116 / 147;
+//   H 7168, 32 of 1024, 112 / 150 rows, 0.69 / 0.73 in use: bf16 392 / 744 against 514 / 590, int8
+//   150 rows 511 against 567; but H 4096, 64 of 512, whose gate/up has one work-group per CU and
+//   whose down has four, int8 150 / 180 rows 284 / 301 and 228 / 239).
 // * 256: the LDS-tiled form above that.
 int ffn_tile_rows(int act, int N, int k, int E, int S, int H, int F, int wf) {
     const long long slots = (long long)N * k, rows = slots + (long long)S * N;

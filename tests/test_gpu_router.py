@@ -1,7 +1,7 @@
 """The router GEMM (yvmoe_router_logits) on the GPU against float64, across the shapes its
 forms take: the streaming form with up to 16 K splits up to 256 tokens and up to 4 above; for larger
-batches the LDS-tiled form with K splits chosen per shape, including a partial last column block (router operand widths
-Ep + 192 that are not multiples of 256) and splits whose last one is shorter.
+batches the LDS-tiled form with K splits chosen per shape, including a partial last column block
+(router operand widths Ep + 192 that are not multiples of 256) and splits whose last one is shorter.
 
 Every logit within 2e-4 * max(1, max |logit|) of x @ gate.weight^T computed in float64 from the
 same bf16 operands; the call is deterministic (two calls give the same bits).
